@@ -81,6 +81,13 @@ struct State {
   size_t field32 = 0;          // floats per field
   size_t f32_bytes = 0;        // the whole FP32 allocation
 
+  // exchange buffers of the on-chip solver loops (tl_resident.hip), null where
+  // the mesh does not fit, and the tag of their next exchange
+  unsigned long long *res_mem = nullptr;
+  long res_words = 0;
+  unsigned res_epoch = 1;
+  bool res_refused = false;    // a cooperative launch was refused
+
   // device staging buffer of host copies (allocated on first use)
   double *stage = nullptr;
   size_t stage_len = 0;       // doubles
@@ -91,6 +98,7 @@ struct State {
 
   // profiling
   bool prof = false;
+  bool passes = false;      // run the pass kernels though prof is off (tl_cg_loop_noalloc)
   int prof_period = 1;      // time every prof_period-th launch of each class
   long prof_seq[8] = {0};   // launches seen per class while enabled
   struct Ev { hipEvent_t a, b; int cls; };
@@ -174,6 +182,9 @@ int copy_host(double *p11, double *host, int host_halo, bool up);
 // synchronous copy of the interior cells between it and p11 (tl_runtime.hip)
 int check_device_array(const double *p, long ld, const char *who);
 int copy_interior_device(double *p11, double *dev, long ld, bool up, const char *who);
+
+// 64-bit words of the exchange buffers an nx x ny mesh needs (tl_resident.hip)
+long resident_words(int nx, int ny);
 
 // Chebyshev iterations on the vector walk (tl_loops.hip): 1 = done,
 // 0 = not applicable here, < 0 = -(error code)

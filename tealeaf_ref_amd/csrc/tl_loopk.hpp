@@ -51,6 +51,27 @@ struct LoopParams {
   int presteps;
 };
 
+// CG iterations with the whole mesh on the chip (tl_resident.hip), for meshes
+// that fit.  pin: direction of the first iteration; the other pointers as in
+// run_cg_loop, p read and written in place.
+template <typename T>
+struct ResCg {
+  T *u, *r, *p, *w, *z;
+  const T *pin;
+  const T *Mi, *Di, *cp, *bfp, *Kx, *Ky;
+  T rx, ry;
+  int n_first, n_last, n_pause;
+  LoopParams lp;
+  double rro;
+  Ctl *ctl;
+  double *hrro, *halpha, *hbeta, *herr;
+};
+// 1: the loop has run and *out holds its result; 0: the mesh does not fit;
+// < 0: -(error code)
+template <typename T>
+int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out);
+constexpr int RES_PAUSED = 0;  // reason of a launch that stopped for the host only
+
 bool use_nontemporal();
 int batch_size();
 // allocates the library's loop history for iterations up to n_last
@@ -1105,16 +1126,25 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
     return TL_OK;
   };
   Ctl res;
-  if ((rc = drive(st->n_first, st->n_last, launch, tail, &res, m.ctl))) return rc;
+  ResCg<T> a = {b.u,  b.r,  b.p[c0], b.w,         b.z,        pin_first ? pin_first : b.p[c0],
+                b.Mi, b.Di, b.cp,    b.bfp,       b.Kx,       b.Ky,
+                b.rx, b.ry, st->n_first, st->n_last, 0,       lp,
+                st->rro, m.ctl, m.hrro, m.halpha, m.hbeta, m.herr};
+  const int ran = resident_cg<T>(
+      a, b.block ? TL_PREC_JAC_BLOCK : (b.diag ? TL_PREC_JAC_DIAG : TL_PREC_NONE), G.pitch, &res);
+  if (ran < 0) return -ran;
+  if (!ran && (rc = drive(st->n_first, st->n_last, launch, tail, &res, m.ctl))) return rc;
   st->n_end = res.n_end;
   st->reason = res.reason;
   st->error = res.error;
   st->rro = res.rro;
   st->old_error = res.old_error;
   if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("CG", res.n_end);
-  // the launch that stopped the loop applied the last p update
-  const int n_det = res.reason == TL_LOOP_SWITCH ? res.n_end : res.n_end + 1;
-  *b.pcur = c0 ^ ((n_det - st->n_first + 1) & 1);
+  if (!ran) {
+    // the launch that stopped the loop applied the last p update
+    const int n_det = res.reason == TL_LOOP_SWITCH ? res.n_end : res.n_end + 1;
+    *b.pcur = c0 ^ ((n_det - st->n_first + 1) & 1);
+  }
   const int last_done = res.reason == TL_LOOP_SWITCH ? res.n_end - 1 : res.n_end;
   if ((rc = copy_hist(cg_alphas, m.halpha, st->n_first, last_done))) return rc;
   if ((rc = copy_hist(cg_betas, m.hbeta, st->n_first, last_done))) return rc;

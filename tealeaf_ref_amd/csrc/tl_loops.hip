@@ -957,12 +957,15 @@ extern "C" int tl_cg_loop_noalloc(tl_loop_state *st, double *cg_alphas, double *
   hipLaunchKernelGGL(k_zero_bytes, dim3(1), dim3(64), 0, s.stream, (unsigned char *)m.ctl,
                      (int)NOALLOC_CTL_BYTES);
   TL_HIP(hipGetLastError());
-  // kernel timing creates events on demand: off for this call
+  // kernel timing creates events on demand: off for this call, which still
+  // takes the kernels that tl_cg_loop would
   const bool prof = s.prof;
   s.prof = false;
+  s.passes = prof;
   LoopBufs<double> bb = fp64_bufs();
   rc = run_cg_loop<double, TL_V64>(bb, st, cg_alphas, cg_betas, nullptr, &m);
   s.prof = prof;
+  s.passes = false;
   return rc;
 }
 

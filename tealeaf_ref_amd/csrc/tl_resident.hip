@@ -1,0 +1,469 @@
+// Kernels and launches of the on-chip solver loops (tl_resident.hpp).
+#include <cstring>
+
+#include "tl_resident.hpp"
+
+using namespace tl;
+
+namespace {
+
+using dev::ResFaces;
+using dev::ResGhost;
+using dev::ResShared;
+using dev::ResTile;
+
+// A field a lane keeps for the whole loop: in registers, or in the block's
+// dynamic LDS where the registers are needed for others.
+template <typename T, int R, bool LDS>
+struct Kept {
+  typedef typename dev::Vec<T, 2>::type VT;
+  VT v[R];
+  __device__ Kept(char *, int) {}
+  __device__ VT get(int j) const { return v[j]; }
+  __device__ void set(int j, VT x) { v[j] = x; }
+};
+template <typename T, int R>
+struct Kept<T, R, true> {
+  typedef typename dev::Vec<T, 2>::type VT;
+  VT *v;
+  __device__ Kept(char *lds, int slot) : v((VT *)lds + (long)slot * R * RES_THREADS + threadIdx.x) {}
+  __device__ VT get(int j) const { return v[j * RES_THREADS]; }
+  __device__ void set(int j, VT x) { v[j * RES_THREADS] = x; }
+};
+
+// The ghosts of a field in memory, for the first iteration.
+template <typename T, int R>
+__device__ inline ResGhost<T> load_ghosts(const ResTile<T, R> &t, const ResGeo &g, const T *f) {
+  ResGhost<T> o;
+  o.dn = t.load(f, g, t.y0 - 1);
+  o.up = t.load(f, g, t.y0 + R);
+  o.side = T(0);
+  if (t.lane < 2 * R) {
+    const bool lft = t.lane < R;
+    const int y = t.y0 + (lft ? t.lane : t.lane - R);
+    if (y < g.ny && (lft ? t.left : t.right))
+      o.side = *t.at(f, g, lft ? t.bx * RES_COLS - 1 : (t.bx + 1) * RES_COLS, y);
+  }
+  return o;
+}
+
+// ---------------------------------------------------------------------------
+// CG: iterations n_first.. of run_cg_loop in one launch
+// ---------------------------------------------------------------------------
+// Where a lane's fields live at R rows: it has 256 registers, of which r, p,
+// w (or z) and kx take four fields.  Larger tiles move u and ky to LDS (160 KB
+// per CU); the preconditioner's fields are then read again in every
+// iteration, from the L2.  The splits are those at which the kernel spills no
+// vector register, and it must not: the compiler may place a spill inside a
+// region that only some lanes run, where it misses the others.
+//
+// What bounds it: the two exchanges of an iteration, about 1.4 us each of 4.6
+// (512^2), and with 16 cells per lane the arithmetic (3 of 6 us).  Against
+// the pass kernels: 512^2 step 5.7 -> 2.5 ms, 777x1031 with jac_diag 23.0 ->
+// 4.8 ms, the 1024^2 adjoint's CG solves 155 -> 43 ms.
+enum Where { REGS, MEMORY };
+template <typename T, int R, int PREC>
+struct CgPlan {
+  static constexpr int SIZE = (int)sizeof(T) / 4 * 2 * R;  // registers of one field
+  static constexpr bool U_LDS = SIZE >= 24;
+  static constexpr bool KY_LDS = SIZE >= (PREC == TL_PREC_NONE ? 32 : 24);
+  static constexpr Where M = PREC == TL_PREC_NONE  ? REGS
+                             : PREC == TL_PREC_JAC_BLOCK ? MEMORY
+                             : SIZE >= 24  ? MEMORY
+                                           : REGS;
+  static constexpr int SLOTS = (U_LDS ? 1 : 0) + (KY_LDS ? 1 : 0);
+  static constexpr size_t BYTES = (size_t)SLOTS * R * RES_THREADS * 2 * sizeof(T);
+};
+
+template <typename T, int R, int PREC>
+__global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
+  typedef typename dev::Vec<T, 2>::type VT;
+  typedef CgPlan<T, R, PREC> Plan;
+  extern __shared__ char dyn[];
+  __shared__ ResShared<T, R, 1> sh;
+  if (threadIdx.x < 2) sh.dead[threadIdx.x] = 0;
+  const ResTile<T, R> t(g);
+  ResFaces<T, R, Plan::KY_LDS> k;
+  k.load(t, g, a.Kx, a.Ky, sh.kxr[t.wave],
+         (VT *)dyn + (long)(Plan::U_LDS ? 1 : 0) * R * RES_THREADS + threadIdx.x);
+  VT r[R], p[R];
+  constexpr bool HAS_Z = PREC != TL_PREC_NONE;
+  VT z[HAS_Z ? R : 1];
+  Kept<T, R, Plan::U_LDS> u(dyn, 0);
+  // Mi of the diagonal preconditioner, where it is kept
+  Kept<T, Plan::M == MEMORY || !HAS_Z ? 1 : R, false> m(dyn, 0);
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int y = t.y0 + j;
+    r[j] = t.load(a.r, g, y);
+    p[j] = t.load(a.pin, g, y);
+    u.set(j, t.load(a.u, g, y));
+    if constexpr (HAS_Z && Plan::M != MEMORY) m.set(j, t.load(a.Mi, g, y));
+  }
+  ResGhost<T> pg = load_ghosts<T, R>(t, g, a.pin);
+  const bool lead = t.blk == 0 && threadIdx.x == 0;
+  double rro = a.rro, err = 0.0, rrn = 0.0;
+  int reason = 0, n_end = 0;
+  bool dead = false, update = false;
+  T be = T(0);
+  ResGhost<T> gh;
+  unsigned s = 0;
+  if (lead) a.hrro[a.n_first] = rro;
+  __syncthreads();
+  // body(j, w) of row j of w = A p
+  auto apply_p = [&](auto body) {
+    if (t.lane < 2 * R) sh.side[t.wave][t.lane] = pg.side;
+    __builtin_amdgcn_wave_barrier();
+    dev::res_apply<diff_form<T>()>(t, k, p, pg.dn, pg.up, sh.side[t.wave], sh.kxr[t.wave], a.rx,
+                                   a.ry, body);
+  };
+  for (int n = a.n_first;; ++n) {
+    VT w[R];
+    // ---- w = A p, p.w
+    double acc = 0.0;
+    apply_p([&](int j, VT wv) {
+      w[j] = wv;
+      acc += (double)wv.x * (double)p[j].x;
+      acc += (double)wv.y * (double)p[j].y;
+    });
+    double pw;
+    if (!dev::res_exchange<false, true>(t, g, sh, s++, acc, &pw, (const VT(*)[R]) nullptr,
+                                        (ResGhost<T> *)nullptr)) {
+      dead = true;
+      break;
+    }
+    if (!isfinite(pw)) {
+      reason = TL_LOOP_NONFINITE;
+      n_end = n;
+      err = pw;
+      break;
+    }
+    const double alpha = rro / pw;
+    if (lead) a.halpha[n] = alpha;
+    // ---- u += alpha p, r -= alpha w, z = M^-1 r, r.r or r.z
+    const T al = (T)alpha;
+    acc = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      u.set(j, u.get(j) + al * p[j]);
+      r[j] = r[j] - al * w[j];
+    }
+    bool ok;
+    if constexpr (PREC == TL_PREC_NONE) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        acc += (double)r[j].x * (double)r[j].x;
+        acc += (double)r[j].y * (double)r[j].y;
+      }
+      ok = dev::res_exchange<true, true>(t, g, sh, s++, acc, &rrn, &r, &gh);
+    } else {
+      if constexpr (PREC == TL_PREC_JAC_DIAG) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          if constexpr (Plan::M == MEMORY) z[j] = t.load(a.Mi, g, t.y0 + j) * r[j];
+          else z[j] = m.get(j) * r[j];
+        }
+      } else {
+        // 4-row Thomas solve (tea_block_solve, kernels/tea_leaf_common_kernel.f90:
+        // 378-468); cells outside the mesh have r = 0, bfp = cp = 0 and Di = 1
+#pragma unroll
+        for (int b = 0; b < R; b += 4) {
+          __builtin_amdgcn_sched_barrier(0);  // one group's loads at a time
+          VT di = t.load(a.Di, g, t.y0 + b);
+          if (!t.okx || b >= t.rows) di.x = T(1);
+          if (!t.oky || b >= t.rows) di.y = T(1);
+          z[b] = r[b] / di;
+#pragma unroll
+          for (int q = 1; q < 4; ++q)
+            z[b + q] = (r[b + q] - (-k.ky(b + q) * a.ry) * z[b + q - 1]) *
+                       t.load(a.bfp, g, t.y0 + b + q);
+          // back substitution; the last row of a short block has no row above
+#pragma unroll
+          for (int q = 2; q >= 0; --q) {
+            const VT c = t.load(a.cp, g, t.y0 + b + q);
+            z[b + q] = b + q + 1 < t.rows ? z[b + q] - c * z[b + q + 1] : z[b + q];
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        acc += (double)r[j].x * (double)z[j].x;
+        acc += (double)r[j].y * (double)z[j].y;
+      }
+      ok = dev::res_exchange<true, true>(t, g, sh, s++, acc, &rrn, &z, &gh);
+    }
+    if (!ok) {
+      dead = true;
+      break;
+    }
+    // ---- head of iteration n + 1 (loop_head)
+    const double beta = rrn / rro;
+    err = sqrt(fabs(rrn));
+    const bool bad = !isfinite(rrn), conv = !bad && fabs(err) < a.lp.eps_abs;
+    const bool tail = n == a.n_last, pause = n == a.n_pause;
+    const bool sw = !bad && !conv && !tail && a.lp.check_switch && fabs(err) <= a.lp.epslim &&
+                    n + 1 >= a.lp.presteps;
+    if (lead) {
+      a.hbeta[n] = beta;
+      a.herr[n] = err;
+    }
+    be = (T)beta;
+    if (bad || conv || sw || tail || pause) {
+      reason = bad    ? TL_LOOP_NONFINITE
+               : conv ? TL_LOOP_CONVERGED
+               : sw   ? TL_LOOP_SWITCH
+               : tail ? TL_LOOP_MAXITERS
+                      : RES_PAUSED;
+      n_end = sw ? n + 1 : n;
+      update = true;
+      break;
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      if constexpr (HAS_Z) p[j] = z[j] + be * p[j];
+      else p[j] = r[j] + be * p[j];
+    }
+    pg.dn = gh.dn + be * pg.dn;
+    pg.up = gh.up + be * pg.up;
+    pg.side = gh.side + be * pg.side;
+    if (lead) a.hrro[n + 1] = rrn;
+    rro = rrn;
+  }
+  if (dead) {
+    if (threadIdx.x == 0) *g.abort_flag = 1;
+    return;
+  }
+  // the fields as the loop leaves them; w = A p of the last iteration is
+  // formed again rather than held through it
+  const int col = t.col_anew();
+  apply_p([&](int j, VT wv) { t.store(a.w, g, col, t.y0 + j, wv); });
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int y = t.y0 + j;
+    t.store(a.u, g, col, y, u.get(j));
+    t.store(a.r, g, col, y, r[j]);
+    VT pj = p[j];
+    if (update) {
+      if constexpr (HAS_Z) pj = z[j] + be * pj;
+      else pj = r[j] + be * pj;
+      if constexpr (HAS_Z) t.store(a.z, g, col, y, z[j]);
+    }
+    t.store(a.p, g, col, y, pj);
+  }
+  if (lead) {
+    a.ctl->stop = 1;
+    a.ctl->reason = reason;
+    a.ctl->n_end = n_end;
+    a.ctl->error = err;
+    a.ctl->old_error = err;
+    a.ctl->rro = rrn;
+  }
+}
+
+}  // namespace
+
+namespace tl {
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+namespace {
+
+int env_int(const char *name, int dflt) {
+  const char *e = getenv(name);
+  return e ? atoi(e) : dflt;
+}
+
+__global__ void k_res_clear(u64 *__restrict__ p, long n) {
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n;
+       i += (long)gridDim.x * blockDim.x)
+    p[i] = 0;
+}
+
+constexpr long RES_WORDS = (long)(RES_PARTS + RES_HALOS) + 16;
+
+// Rows per lane for an nx x ny mesh, of the counts in `rows` (ascending): 0
+// when no tiling has at most one block per CU.
+int res_rows(int nx, int ny, const int *rows, int nrows) {
+  const State &s = S();
+  const int forced = env_int("TL_RES_ROWS", 0);
+  const int cap = s.cus < RES_MAX_BLOCKS ? s.cus : RES_MAX_BLOCKS;
+  const long tx = (nx + RES_COLS - 1) / RES_COLS;
+  int best = 0;
+  double best_cost = 0.0;
+  for (int i = 0; i < nrows; ++i) {
+    const int R = rows[i];
+    const long ty = (ny + (long)RES_WAVES * R - 1) / ((long)RES_WAVES * R), nb = tx * ty;
+    if (nb > cap) continue;
+    if (forced == R) return R;
+    // time of an iteration in us: two exchanges, dearer with more blocks, and
+    // the arithmetic of R rows.  Measured per step: 512^2 3.04 ms with R = 1
+    // (256 blocks), 2.50 with 2, 2.43 with 4, 2.92 with 8; 250^2 (ten steps)
+    // 12.5 ms with 1, 12.2 with 2, 13.0 with 4, 16.2 with 8
+    const double sync = nb == 1 ? 0.4 : (nb <= 8 ? 1.2 : (nb <= 128 ? 1.4 : 2.1));
+    const double cost = 2.0 * sync + 0.2 * R;
+    if (!best || cost < best_cost) {
+      best = R;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+constexpr int ROWS64[] = {1, 2, 3, 4, 6, 8}, ROWS64_BLK[] = {4};
+constexpr int ROWS32[] = {1, 2, 3, 4, 6, 8, 12, 16};
+
+template <typename T>
+int rows_for(int nx, int ny, int prec) {
+  if (sizeof(T) == 4) return res_rows(nx, ny, ROWS32, 8);
+  return prec == TL_PREC_JAC_BLOCK ? res_rows(nx, ny, ROWS64_BLK, 1)
+                                   : res_rows(nx, ny, ROWS64, prec == TL_PREC_NONE ? 6 : 5);
+}
+
+constexpr int RES_REFUSED = -1;
+
+// One launch of a kernel over a's mesh: cooperatively, so that every block is
+// resident when the first one waits (a single block waits for none).  The
+// runtime refuses cooperative launches while another process holds the
+// device's; the chunk's loops then run the pass kernels from there on.
+template <typename A>
+int res_launch(void (*k)(ResGeo, A), ResGeo g, A a, size_t lds) {
+  State &s = S();
+  const int nb = g.tx * g.ty;
+  if (nb == 1) {
+    hipLaunchKernelGGL(k, dim3(1), dim3(RES_THREADS), lds, s.stream, g, a);
+    TL_HIP(hipGetLastError());
+    return TL_OK;
+  }
+  void *args[] = {&g, &a};
+  if (hipLaunchCooperativeKernel((const void *)k, dim3(nb), dim3(RES_THREADS), args,
+                                 (unsigned)lds, s.stream) == hipSuccess)
+    return TL_OK;
+  (void)hipGetLastError();
+  s.res_refused = true;
+  return RES_REFUSED;
+}
+
+ResGeo res_geo(int R, long pitch) {
+  State &s = S();
+  ResGeo g;
+  g.nx = s.nx;
+  g.ny = s.ny;
+  g.pitch = (unsigned)pitch;
+  g.tx = (s.nx + RES_COLS - 1) / RES_COLS;
+  g.ty = (s.ny + RES_WAVES * R - 1) / (RES_WAVES * R);
+  g.part = s.res_mem;
+  g.halo = s.res_mem + RES_PARTS;
+  g.abort_flag = (int *)(s.res_mem + RES_PARTS + RES_HALOS);
+  g.limit = 2000000000LL;  // 20 s
+  if (const char *e = getenv("TL_RES_LIMIT")) g.limit = atoll(e);
+  return g;
+}
+
+// Tags for `exchanges` exchanges; before they run out the buffers start over.
+int res_tags(long exchanges, unsigned *epoch) {
+  State &s = S();
+  if ((u64)s.res_epoch + (u64)exchanges > 0xfffffff0ull) {
+    hipLaunchKernelGGL(k_res_clear, dim3(1024), dim3(BLOCK), 0, s.stream, s.res_mem, RES_WORDS);
+    TL_HIP(hipGetLastError());
+    s.res_epoch = 1;
+  }
+  *epoch = s.res_epoch;
+  s.res_epoch += (unsigned)exchanges;
+  return TL_OK;
+}
+
+// The control block of a finished launch, and whether a wait ran out.
+int res_result(const ResGeo &g, Ctl *dctl, Ctl *out) {
+  State &s = S();
+  Ctl *hc = (Ctl *)s.hctl;
+  int *ha = (int *)(hc + 3);
+  TL_HIP(hipMemcpyAsync(&hc[2], dctl, sizeof(Ctl), hipMemcpyDeviceToHost, s.stream));
+  TL_HIP(hipMemcpyAsync(ha, g.abort_flag, sizeof(int), hipMemcpyDeviceToHost, s.stream));
+  TL_HIP(hipStreamSynchronize(s.stream));
+  if (*ha) {
+    hipLaunchKernelGGL(k_res_clear, dim3(1), dim3(1), 0, s.stream, (u64 *)g.abort_flag, 1L);
+    return fail(TL_ERR_HIP, "solver loop: a block waited too long for the others");
+  }
+  *out = hc[2];
+  return TL_OK;
+}
+
+// iterations of one launch: long loops come back to the host in between
+int res_chunk() {
+  const int c = env_int("TL_RES_CHUNK", 1 << 16);
+  return c < 1 ? 1 : (c > 1 << 20 ? 1 << 20 : c);
+}
+
+template <typename T, int R, int PREC>
+int cg_launch(const ResGeo &g, const ResCg<T> &a) {
+  return res_launch(&k_res_cg<T, R, PREC>, g, a, CgPlan<T, R, PREC>::BYTES);
+}
+
+template <typename T>
+int cg_dispatch(int R, int prec, const ResGeo &g, const ResCg<T> &a) {
+#define CASE(RR, PP)   if (R == RR && prec == PP) return cg_launch<T, RR, PP>(g, a)
+  CASE(1, TL_PREC_NONE);
+  CASE(2, TL_PREC_NONE);
+  CASE(3, TL_PREC_NONE);
+  CASE(4, TL_PREC_NONE);
+  CASE(6, TL_PREC_NONE);
+  CASE(8, TL_PREC_NONE);
+  if constexpr (sizeof(T) == 4) {
+    CASE(12, TL_PREC_NONE);
+    CASE(16, TL_PREC_NONE);
+  } else {
+    CASE(1, TL_PREC_JAC_DIAG);
+    CASE(2, TL_PREC_JAC_DIAG);
+    CASE(3, TL_PREC_JAC_DIAG);
+    CASE(4, TL_PREC_JAC_DIAG);
+    CASE(6, TL_PREC_JAC_DIAG);
+    CASE(4, TL_PREC_JAC_BLOCK);
+  }
+#undef CASE
+  return fail(TL_ERR_STATE, "solver loop: no kernel for this tiling");
+}
+
+}  // namespace
+
+// Kernel timing counts the launches of the pass kernels: while it is on, the
+// loops run them.  TL_RESIDENT=0 (read on every call) switches to them too.
+static bool resident_on() {
+  const State &s = S();
+  return s.res_mem && !s.res_refused && !s.prof && !s.passes && env_int("TL_RESIDENT", 1);
+}
+
+long resident_words(int nx, int ny) {
+  return (rows_for<double>(nx, ny, TL_PREC_NONE) || rows_for<float>(nx, ny, TL_PREC_NONE))
+             ? RES_WORDS
+             : 0;
+}
+
+template <typename T>
+int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out) {
+  State &s = S();
+  if (!resident_on()) return 0;
+  const int R = rows_for<T>(s.nx, s.ny, prec);
+  if (!R) return 0;
+  ResGeo g = res_geo(R, pitch);
+  const int n_first = a.n_first, chunk = res_chunk();
+  for (;;) {
+    const long left = (long)a.n_last - a.n_first + 1;
+    const long run = left < chunk ? left : chunk;
+    a.n_pause = (int)(a.n_first + run - 1);
+    int rc;
+    if ((rc = res_tags(2 * run, &g.epoch))) return -rc;
+    rc = cg_dispatch<T>(R, prec, g, a);
+    if (rc == RES_REFUSED) return a.n_first == n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
+    if (rc || (rc = res_result(g, a.ctl, out))) return -rc;
+    if (out->reason != RES_PAUSED) return 1;
+    // p has been updated: the next launch starts as a first iteration does
+    a.n_first = out->n_end + 1;
+    a.rro = out->rro;
+    a.pin = a.p;
+  }
+}
+template int resident_cg<double>(ResCg<double>, int, long, Ctl *);
+template int resident_cg<float>(ResCg<float>, int, long, Ctl *);
+
+}  // namespace tl

@@ -225,6 +225,7 @@ extern "C" int tl_finalize(void) {
   if (s.ctl) (void)hipFree(s.ctl);
   if (s.hctl) (void)hipHostFree(s.hctl);
   if (s.hist) (void)hipFree(s.hist);
+  if (s.res_mem) (void)hipFree(s.res_mem);
   for (hipEvent_t e : s.loop_ev)
     if (e) (void)hipEventDestroy(e);
   if (s.f32) (void)hipFree(s.f32);
@@ -276,6 +277,11 @@ extern "C" int tl_init(int nx, int ny, int halo, int device) {
   TL_HIP(hipMalloc(&s.ctl, 64));
   TL_HIP(hipMemsetAsync(s.ctl, 0, 64, s.stream));
   TL_HIP(hipHostMalloc(&s.hctl, 256, hipHostMallocDefault));
+  // the exchange buffers of the on-chip loops: zeros, since their tags start at 1
+  if ((s.res_words = resident_words(nx, ny))) {
+    TL_HIP(hipMalloc((void **)&s.res_mem, sizeof(*s.res_mem) * (size_t)s.res_words));
+    TL_HIP(hipMemsetAsync(s.res_mem, 0, sizeof(*s.res_mem) * (size_t)s.res_words, s.stream));
+  }
   TL_HIP(hipEventCreateWithFlags(&s.loop_ev[0], hipEventDisableTiming));
   TL_HIP(hipEventCreateWithFlags(&s.loop_ev[1], hipEventDisableTiming));
   TL_HIP(hipStreamSynchronize(s.stream));
@@ -485,6 +491,7 @@ extern "C" int tl_device_bytes(double *bytes) {
   b += (double)s.snaps.size() * (double)s.field_bytes;
   b += (double)s.f32_bytes;
   b += sizeof(double) * (double)MAX_GRID * NPART;
+  b += sizeof(*s.res_mem) * (double)s.res_words;
   if (s.hist) b += sizeof(double) * 4.0 * (double)s.hist_len;
   b += sizeof(double) * (double)s.stage_len;
   *bytes = b;
