@@ -156,14 +156,18 @@ void prof_end(int cls, hipEvent_t a);
 // Launch on the library's stream; inside a prof_arm region the launch takes
 // the region's events.
 template <typename... F, typename... A>
-inline void klaunch(void (*k)(F...), dim3 grid, dim3 block, A... args) {
+inline void klaunch_lds(void (*k)(F...), dim3 grid, dim3 block, size_t lds, A... args) {
   State &s = S();
   if (s.prof && s.arm_a && !s.arm_fired) {
     s.arm_fired = true;
-    hipExtLaunchKernelGGL(k, grid, block, 0, s.stream, s.arm_a, s.arm_b, 0, args...);
+    hipExtLaunchKernelGGL(k, grid, block, (unsigned)lds, s.stream, s.arm_a, s.arm_b, 0, args...);
   } else {
-    hipLaunchKernelGGL(k, grid, block, 0, s.stream, args...);
+    hipLaunchKernelGGL(k, grid, block, lds, s.stream, args...);
   }
+}
+template <typename... F, typename... A>
+inline void klaunch(void (*k)(F...), dim3 grid, dim3 block, A... args) {
+  klaunch_lds(k, grid, block, 0, args...);
 }
 
 // finish a reduction: sum `n` partials of `slot` (deterministically) into

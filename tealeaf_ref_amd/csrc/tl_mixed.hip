@@ -433,7 +433,7 @@ extern "C" int tl_mixed_solve(tl_mixed_state *st) {
         return rc;
       const int slot = P2;
       double zr;
-      if ((rc = finish_sums(&slot, 1, b.G.blocks, &zr))) return rc;
+      if ((rc = finish_sums(&slot, 1, sweep_parts<float, 4>(b, st->inner_steps), &zr))) return rc;
       st->sweeps += st->inner_steps;
       if (!(zr > 0.0)) return fail(TL_ERR_NONFINITE, "tl_mixed_solve: z.r is not positive");
       tl_loop_state ls;

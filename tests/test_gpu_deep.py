@@ -1,0 +1,88 @@
+"""Passes of many sweeps (tl_deep*.hpp) against the one- and two-sweep passes
+(TL_DEEP=0) on the same chunk.  A wave's strip is 108 to 120 columns wide in
+FP64 and 232 to 248 in FP32, with ghosts of as many rows and columns as the
+pass has sweeps: the meshes are narrower and wider than one and two strips,
+ragged, and of fewer rows than the ghosts."""
+import ctypes as C
+import math
+
+import numpy as np
+import pytest
+
+from helpers import interior
+from tealeaf_ref_amd import _lib as L
+from tealeaf_ref_amd.adjoint import chebyshev_coefs
+from test_gpu_resident import _chunk, _norm_a, _start, env
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(3, 2), (7, 31), (107, 9), (109, 64), (217, 45), (250, 37), (501, 133), (130, 400)]
+
+
+@pytest.mark.parametrize("inner", [4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 16, 21, 30])
+@pytest.mark.parametrize("reflective", [False, True])
+def test_ppcg_sweeps(inner, reflective):
+    """z after one outer iteration, i.e. the Chebyshev polynomial of r.
+
+    Tolerance: with bounds that hold the spectrum the recurrence is stable, so
+    a sweep's rounding (row sums of about 10 operations on terms of up to
+    |A| |sd|, which is about 2 |r|) reaches z divided by theta = |A|/2 and is
+    not amplified by more than the condition of the bounds used here, at most
+    100.  That is 10 * 100 roundings per sweep relative to the largest z."""
+    pd = C.POINTER(C.c_double)
+    for nx, ny in SIZES:
+        print(f"deep ppcg {nx}x{ny} inner {inner} reflective {reflective}", flush=True)
+        d, rx, ry = _chunk(nx, ny, 1, reflective)
+        try:
+            out = []
+            for deep in (0, 1):
+                with env(TL_DEEP=deep):
+                    r0 = _start(d, rx, ry)
+                    hi = 1.05 * _norm_a(d, rx, ry)
+                    ca, cb, theta = chebyshev_coefs(hi / 100.0, hi, inner)
+                    d.scalar("tl_cg_init")
+                    L.call("tl_set_ppcg_active", 1)
+                    d.scalar("tl_ppcg_init", 2)
+                    # the switch to PPCG (tea_solve.f90:229-250)
+                    L.call("tl_ppcg_init_sd", theta)
+                    d.update_halo([0, 0, 0, 0, 0, 1, 1] + [0] * 4, 1)
+                    L.call("tl_ppcg_inner", ca.ctypes.data_as(pd), cb.ctypes.data_as(pd), 1, inner)
+                    L.call("tl_ppcg_update_z")
+                    rro = d.scalar("tl_ppcg_init", 3)
+                    st = L.LoopState(n_first=2, n_last=2, eps_abs=0.0, rro=rro, old_error=r0)
+                    n = C.c_int(0)
+                    rc = L.lib().tl_ppcg_loop(C.byref(st), ca.ctypes.data_as(pd),
+                                              cb.ctypes.data_as(pd), inner, theta, C.byref(n))
+                    L.call("tl_set_ppcg_active", 0)
+                    out.append((rc, st.n_end, n.value, st.error, interior(d.download("z"), 1),
+                                interior(d.download("p"), 1)))
+        finally:
+            d.close()
+        ref, got = out
+        assert got[:3] == ref[:3] == (L.TL_OK, 2, inner)
+        tol = 1000.0 * inner * 2.0 ** -53
+        for i in (4, 5):
+            scale = float(np.max(np.abs(ref[i])))
+            assert np.max(np.abs(got[i] - ref[i])) <= tol * scale, (nx, ny, i)
+
+
+@pytest.mark.parametrize("inner", [4, 7, 10, 13, 20])
+def test_mixed_sweeps(inner):
+    """The FP32 passes inside the refined solver: both ways reach the true
+    residual asked for, and |u - x| <= |u0 - A u| (the smallest eigenvalue of A
+    is 1) bounds how far apart the two solutions may be."""
+    for nx, ny in ((7, 31), (231, 40), (233, 64), (500, 133)):
+        print(f"deep mixed {nx}x{ny} inner {inner}", flush=True)
+        d, rx, ry = _chunk(nx, ny, 1, False)
+        try:
+            us = []
+            for deep in (0, 1):
+                with env(TL_DEEP=deep):
+                    r0 = math.sqrt(_start(d, rx, ry))
+                    st = d.mixed_solve(solver=L.MIXED_PPCG, rel_tol=1e-10, inner_steps=inner,
+                                       presteps=20)
+                    assert st.reason == L.LOOP_CONVERGED
+                    us.append(interior(d.download("u"), 1))
+        finally:
+            d.close()
+        assert np.linalg.norm(us[1] - us[0]) <= 2e-10 * r0 * 1.01
