@@ -41,6 +41,43 @@ struct DeepGeo {
 
 namespace dev {
 
+// The coefficients of the sweeps, sweep s's in lane s of vector registers: as
+// scalars over the whole unrolled loop they would be spilled.
+template <typename T>
+struct LaneCoef {
+  T a, b;
+  __device__ explicit LaneCoef(const DeepCoef<T> &co) : a(0), b(0) {
+    const int lane = threadIdx.x & (WAVE - 1);
+#pragma unroll
+    for (int s = 0; s < DEEP_MAX; ++s)
+      if (lane == s) {
+        a = co.a[s];
+        b = co.b[s];
+      }
+    // from here on only readlane knows what the lanes hold
+    asm volatile("" : "+v"(a), "+v"(b));
+  }
+  static __device__ T pick(T v, int s) {
+    if constexpr (sizeof(T) == 8) {
+      const unsigned long long q = __builtin_bit_cast(unsigned long long, v);
+      const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)q, s);
+      const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(q >> 32), s);
+      return __builtin_bit_cast(T, (unsigned long long)lo | ((unsigned long long)hi << 32));
+    } else {
+      return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), s));
+    }
+  }
+  __device__ T alpha(int s) const { return pick(a, s); }
+  __device__ T beta(int s) const { return pick(b, s); }
+};
+
+// Rows in flight: loads run this far ahead of the stages.  A divisor of the
+// ring's length, so that the unrolled rows use fixed registers.
+constexpr int deep_ahead(int stages) {
+  (void)stages;
+  return 2;
+}
+
 constexpr int deep_ghost(int stages, int V) { return (stages + V - 1) / V * V; }
 constexpr int deep_strip(int stages, int V) { return WAVE * V - 2 * deep_ghost(stages, V); }
 
@@ -91,10 +128,12 @@ __device__ inline T keep(T v, unsigned m) {
 template <typename T, int V, int STAGES>
 struct DeepStrip {
   typedef typename Vec<T, V>::type VT;
-  int lane, c, cl;           // first column of the lane; clamped into the row
+  int lane, c;               // first column of the lane
+  unsigned off;              // bytes from the row to it, clamped into the row
   int y0, y1;                // rows this wave stores
   int first, last;           // rows it loads
   bool live;                 // a tile exists
+  bool left_edge, right_edge;  // it has the mesh's first / last column
   bool out, part;            // the lane's columns are stored; only some of them
   bool any_part;             // ... in some lane of the wave
   unsigned in[V], face[V];   // the lane's cells in the mesh; with a face on the left
@@ -112,13 +151,15 @@ struct DeepStrip {
     ny = g.ny;
     pitch = g.pitch;
     const int top = (nx / V) * V;
-    cl = c < 0 ? 0 : (c > top ? top : c);
+    off = (unsigned)(c < 0 ? 0 : (c > top ? top : c)) * (unsigned)sizeof(T);
     y0 = tile * g.rows;
     y1 = y0 + g.rows < ny ? y0 + g.rows : ny;
     first = y0 - STAGES > 0 ? y0 - STAGES : 0;
     last = y1 - 1 + STAGES;
     out = c >= strip * S && c < (strip + 1) * S && c < nx;
     part = out && c + V > nx;
+    left_edge = strip == 0;
+    right_edge = strip == g.strips - 1;
     any_part = __any(part);
     out = out && !part;
 #pragma unroll
@@ -129,7 +170,7 @@ struct DeepStrip {
   }
   // the lane's cells of a row that starts at element `row` of a field
   __device__ VT load(const T *__restrict__ f, long row) const {
-    return *(const VT *)(f + row + cl);
+    return *(const VT *)((const char *)(f + row) + off);
   }
   // zero where the mesh is not: by bits and not by compares, whose masks
   // would fill the scalar registers over the unrolled rows
@@ -140,12 +181,16 @@ struct DeepStrip {
     return v;
   }
   __device__ VT cells(VT v, int y) const { return masked(v, in, y < ny); }
+  __device__ VT cells_if(VT v, bool row) const { return masked(v, in, row); }
   __device__ VT faces_x(VT v, int y) const { return masked(v, face, y < ny); }
   __device__ VT faces_y(VT v, int y) const { return masked(v, in, y > 0 && y < ny); }
-  __device__ void store(T *f, long row, VT v) const {
-    if (out) *(VT *)(f + row + c) = v;
+  // Rows that are not stored (ok false) pass through the same instructions with
+  // no lane on: a branch around the store would leave the compiler unsure how
+  // many are in flight, and it would then wait for them with the loads.
+  __device__ void store(T *f, long row, VT v, bool ok) const {
+    if (out & ok) *(VT *)((char *)(f + row) + off) = v;
     if (any_part) {
-      if (part) stv<false, T, V>(f + row, c, nx, v);
+      if (part & ok) stv<false, T, V>(f + row, c, nx, v);
     }
   }
 };

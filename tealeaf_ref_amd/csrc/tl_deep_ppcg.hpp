@@ -12,7 +12,6 @@ struct DeepPpcg {
   T *sd_out, *rt_out, *ut_out;      // not in a last pass
   T *z;
   T rx, ry, theta_r;
-  int want_rrn;
   double *part_rrn, *part_zr;
   const Ctl *ctl;
 };
@@ -28,7 +27,8 @@ namespace {
 // that no register moves and no ring address is computed (309); the faces of
 // the next stage read from the LDS while the current one is computed, the
 // output row's loads issued before the prefetched row's, and the coefficients
-// in LDS instead of spilled scalar registers (216).
+// in lanes instead of spilled scalar registers (211).  More rows in flight
+// (four or five instead of two) spill, and gain nothing where they do not.
 template <typename T, int V, int STAGES, int FIRST, int LAST>
 __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
                                                      DeepPpcg<T> a) {
@@ -42,17 +42,6 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
   const int b = blockIdx.x;
   const int lb = nb % NUM_XCD == 0 ? (b % NUM_XCD) * (nb / NUM_XCD) + b / NUM_XCD : b;
   const dev::DeepStrip<T, V, STAGES> t(g, lb * (BLOCK / WAVE) + wave);
-  // the sweeps' coefficients behind the rings: in scalar registers they would
-  // not fit, and come back from a vector register a half at a time
-  typedef typename dev::Vec<T, 2>::type AB;
-  AB *coef = (AB *)((VT *)dyn + (BLOCK / WAVE) * STAGES * NF * WAVE);
-  if (threadIdx.x < STAGES) {
-    AB v;
-    v.x = co.a[threadIdx.x];
-    v.y = co.b[threadIdx.x];
-    coef[threadIdx.x] = v;
-  }
-  __syncthreads();
   VT *ring = (VT *)dyn + (long)wave * STAGES * NF * WAVE + t.lane;
   auto at = [&](int slot, int f) -> VT & { return ring[(slot * NF + f) * WAVE]; };
   double arrn = 0.0, azr = 0.0;
@@ -78,7 +67,7 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
     row_l += yl < t.ny ? t.pitch : 0;
     return i;
   };
-  static_assert(STAGES % 2 == 0, "the rows in flight alternate between two sets");
+  dev::LaneCoef<T> cs(co);
   if (t.live) {
     // rows of sd before stage s + 1: behind[s], centre[s]; rtemp and utemp of
     // sweep s on the row stage s + 1 takes next
@@ -88,9 +77,10 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
     VT kx1 = VT(0), ky1 = VT(0);
     // rows below the first one loaded are rows of zeros without faces
     for (int i = 0; i < STAGES * NF; ++i) ring[i * WAVE] = VT(0);
-    In q[2];
-    q[0] = load();
-    q[1] = load();
+    constexpr int AHEAD = dev::deep_ahead(STAGES);
+    In q[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) q[i] = load();
     // what an output row needs besides the stages' results, loaded a step
     // ahead: r and r_store, and utemp of the passes before, which is added
     // there, where only its own cell reads it
@@ -99,28 +89,27 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
     };
     Out o1 = {VT(0), VT(0), VT(0)};
     long row_o = (long)t.y0 * t.pitch;  // row of the next output
-    auto load_out = [&](int yo, long row) {
+    auto load_out = [&](long row) {
       Out o = {VT(0), VT(0), VT(0)};
-      if (yo >= t.y0 && yo < t.y1) {
-        if (LAST) o.rv = t.load(a.r, row);
-        if (LAST && a.want_rrn) o.rs = t.load(a.r_store, row);
-        if (!FIRST && (t.out || t.part)) o.u0 = t.load(a.ut_in, row);
-      }
+      if (LAST) o.rv = t.load(a.r, row);
+      if (LAST) o.rs = t.load(a.r_store, row);
+      if (!FIRST && (t.out || t.part)) o.u0 = t.load(a.ut_in, row);
       return o;
     };
     struct Faces {
       VT kx, ky, di;
-      AB ab;
     };
     // one row; `slot` is the ring slot of row y - 1, a constant in the unrolled
     // loop, as every ring address and register of the stages then is
     auto step = [&](int y, In &qi, const int slot) {
       In in = qi;
+      asm volatile("" : "+v"(cs.a), "+v"(cs.b));  // no readlane leaves the row
       const int yo = y - STAGES;
       // the next output row's loads before the row's after next, so that
       // waiting for the first does not wait for the second
       const Out out = o1;
-      o1 = load_out(yo + 1, yo >= t.y0 ? row_o + t.pitch : row_o);
+      const bool ok = yo >= t.y0 && yo < t.y1;
+      o1 = load_out(row_o + (ok && yo + 1 < t.y1 ? t.pitch : 0));
       qi = load();
       in.kx = t.faces_x(in.kx, y);
       in.ky = t.faces_y(in.ky, y);
@@ -130,7 +119,7 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
       if (FIRST) in.sd = in_ut = in.rt * a.theta_r;
       // faces and diagonal of row y - 1 into the ring
       VT kyu = in.ky;
-      Faces f = {kx1, ky1, VT(0), coef[0]};
+      Faces f = {kx1, ky1, VT(0)};
       T kxr = dev::from_above(f.kx[0]);
       if (!DIFF) {
 #pragma unroll
@@ -153,7 +142,6 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
           nf.kx = at(o, 0);
           nf.ky = at(o, 1);
           if (!DIFF) nf.di = at(o, 2);
-          nf.ab = coef[s + 1];
         }
         __builtin_amdgcn_sched_barrier(0);
         const VT c = centre[s];
@@ -172,7 +160,7 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
                    a.rx * (kr * r + f.kx[e] * l);
         }
         const VT rn = rt - w;
-        const VT sn = f.ab.x * c + f.ab.y * rn;
+        const VT sn = cs.alpha(s) * c + cs.beta(s) * rn;
         const VT un = ut + sn;
         behind[s] = c;
         centre[s] = ahead;
@@ -191,28 +179,27 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
       }
       kx1 = in.kx;
       ky1 = in.ky;
-      if (yo >= t.y0 && yo < t.y1) {
-        if (!FIRST) ut = out.u0 + ut;
-        if (LAST) {
-          t.store(a.z, row_o, ut);
-          const VT rv = t.cells(out.rv, yo), rs = t.cells(out.rs, yo);
+      if (!FIRST) ut = out.u0 + ut;
+      if (LAST) {
+        t.store(a.z, row_o, ut, ok);
+        const VT rv = t.cells_if(out.rv, ok), rs = t.cells_if(out.rs, ok);
+        ut = t.cells_if(ut, ok);
 #pragma unroll
-          for (int e = 0; e < V; ++e) {
-            arrn += ((double)rv[e] - (double)rs[e]) * (double)ut[e];
-            azr += (double)ut[e] * (double)rv[e];
-          }
-        } else {
-          t.store(a.sd_out, row_o, ahead);
-          t.store(a.rt_out, row_o, rt);
-          t.store(a.ut_out, row_o, ut);
+        for (int e = 0; e < V; ++e) {
+          arrn += ((double)rv[e] - (double)rs[e]) * (double)ut[e];
+          azr += (double)ut[e] * (double)rv[e];
         }
-        row_o += t.pitch;
+      } else {
+        t.store(a.sd_out, row_o, ahead, ok);
+        t.store(a.rt_out, row_o, rt, ok);
+        t.store(a.ut_out, row_o, ut, ok);
       }
+      row_o += ok ? t.pitch : 0;
     };
     // steps past the last row store nothing
     for (int y = t.first; y <= t.last; y += STAGES) {
 #pragma unroll
-      for (int j = 0; j < STAGES; ++j) step(y + j, q[j & 1], j);
+      for (int j = 0; j < STAGES; ++j) step(y + j, q[j % AHEAD], j);
     }
   }
   if (LAST) {
@@ -230,11 +217,10 @@ __global__ __launch_bounds__(BLOCK) void k_deep_ppcg(DeepGeo g, DeepCoef<T> co,
   }
 }
 
-// LDS of a block: four waves' rings and the coefficients
+// LDS of a block: four waves' rings
 template <typename T>
 constexpr size_t deep_lds(int stages) {
-  return (size_t)(BLOCK / WAVE) * stages * (diff_form<T>() ? 2 : 3) * WAVE * 16 +
-         2 * sizeof(T) * stages;
+  return (size_t)(BLOCK / WAVE) * stages * (diff_form<T>() ? 2 : 3) * WAVE * 16;
 }
 
 template <typename T, int V, int STAGES, int FIRST, int LAST>
@@ -267,16 +253,20 @@ inline bool deep_on() {
   const char *e = getenv("TL_DEEP");
   return !e || atoi(e) != 0;
 }
+// Not on meshes so wide that their strips alone would leave more partial sums
+// than the slots hold (MAX_GRID blocks of four strips of at least 84 columns).
+inline bool deep_fits() {
+  return S().nx <= MAX_GRID * 4 * 84 && sweep_pairs() && deep_on();
+}
 // Whether the deep passes take these sweeps: not with a preconditioner (one
-// or two sweeps per pass there), not fewer than 4, and not on meshes so wide
-// that their strips alone would leave more partial sums than the slots hold
-// (MAX_GRID blocks of four strips of at least 84 columns).
+// or two sweeps per pass there), and not fewer than 4.
 inline bool deep_takes(int inner, int diag, int block) {
-  return !diag && !block && inner >= 4 && S().nx <= MAX_GRID * 4 * 84 && sweep_pairs() && deep_on();
+  return !diag && !block && inner >= 4 && deep_fits();
 }
 
+// Strips and tiles of a pass whose blocks a CU holds `per_cu` of.
 template <typename T, int V>
-DeepGeo deep_geo(int stages, long pitch) {
+DeepGeo deep_geo(int stages, long pitch, int per_cu) {
   const State &s = S();
   DeepGeo g;
   g.nx = s.nx;
@@ -285,8 +275,6 @@ DeepGeo deep_geo(int stages, long pitch) {
   const int strip = dev::deep_strip(stages, V);
   g.strips = (s.nx + strip - 1) / strip;
   // one round of waves: what the CUs hold at once
-  int per_cu = (int)((160 * 1024) / deep_lds<T>(stages));
-  if (per_cu > 2) per_cu = 2;
   const int waves = (s.cus > 0 ? s.cus : 256) * per_cu * (BLOCK / WAVE);
   int tiles = waves / g.strips;
   if (tiles < 1) tiles = 1;
@@ -300,16 +288,23 @@ DeepGeo deep_geo(int stages, long pitch) {
   return g;
 }
 
+// PPCG's passes: four stages take under 256 registers, so a CU holds two
+// blocks; with more the registers or the rings allow one.
+template <typename T, int V>
+DeepGeo deep_ppcg_geo(int stages, long pitch) {
+  return deep_geo<T, V>(stages, pitch, stages <= 4 ? 2 : 1);
+}
+
 // Partial sums the last pass leaves.
 template <typename T, int V>
 int deep_parts(int inner, long pitch) {
-  return deep_geo<T, V>(deep_last(inner), pitch).blocks;
+  return deep_ppcg_geo<T, V>(deep_last(inner), pitch).blocks;
 }
 
 template <typename T, int V, int FIRST, int LAST>
 int deep_dispatch(int stages, long pitch, const double *alphas, const double *betas,
                   const DeepPpcg<T> &a) {
-  const DeepGeo g = deep_geo<T, V>(stages, pitch);
+  const DeepGeo g = deep_ppcg_geo<T, V>(stages, pitch);
   // 4 sweeps: alone, or after the single sweep of an odd count
   if constexpr (LAST)
     if (stages == 4) return deep_launch<T, V, 4, FIRST, LAST>(g, alphas, betas, a);

@@ -1065,7 +1065,6 @@ int queue_sweeps(const LoopBufs<T> &b, const double *alphas, const double *betas
     a.rx = b.rx;
     a.ry = b.ry;
     a.theta_r = theta_r;
-    a.want_rrn = want_rrn;
     a.part_rrn = m.part(P3);
     a.part_zr = m.part(P2);
     a.ctl = ctl;

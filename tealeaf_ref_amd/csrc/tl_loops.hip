@@ -7,6 +7,7 @@
 
 #include "tl_loopk.hpp"
 #include "tl_cheby2.hpp"
+#include "tl_deep_cheby.hpp"
 #include "tl_jacobi2.hpp"
 
 namespace tl {
@@ -588,6 +589,57 @@ int cheby_run_block(const double *ch_alphas, const double *ch_betas, int step_fi
   return 1;
 }
 
+// Chebyshev iterations without a preconditioner, an even count of at most
+// DEEP_MAX per pass after a single one where `count` is odd
+// (cheby_run_fused's contract).
+int cheby_run_deep(const double *ch_alphas, const double *ch_betas, int step_first, int count,
+                   int want_norm, double *norm) {
+  State &s = S();
+  int done = 0, nparts = 0;
+  if (count & 1) {
+    const Geo G = geo(2 * BLOCK);
+    const int nb = G.blocks < 0 ? -G.blocks : G.blocks, st = step_first - 1;
+    hipEvent_t ev;
+    prof_arm(3, &ev);
+    klaunch(use_nontemporal() ? k_cheby_v<true, 0> : k_cheby_v<false, 0>, dim3(nb), dim3(BLOCK), G,
+            s.u[s.ucur].p11, s.u[1 - s.ucur].p11, s.u0.p11, s.Kx.p11, s.Ky.p11, s.p[s.pcur].p11,
+            s.w.p11, s.r.p11, s.z.p11, s.Mi.p11, s.rx, s.ry, ch_alphas[st], ch_betas[st], 0, 0,
+            part(P0), 1);
+    prof_end(3, ev);
+    if (hipGetLastError() != hipSuccess) return -fail(TL_ERR_HIP, "Chebyshev pass launch");
+    s.ucur = 1 - s.ucur;
+    done = 1;
+  }
+  for (int left = count - done, p = deep_passes(count); p > 0; --p) {
+    const int n = deep_next(left, p), st = step_first + done - 1;
+    DeepCheby a;
+    a.u = s.u[s.ucur].p11;
+    a.p = s.p[s.pcur].p11;
+    a.u0 = s.u0.p11;
+    a.Kx = s.Kx.p11;
+    a.Ky = s.Ky.p11;
+    a.u_out = s.u[1 - s.ucur].p11;
+    a.p_out = s.p[1 - s.pcur].p11;
+    a.w = s.w.p11;
+    a.r = s.r.p11;
+    a.rx = s.rx;
+    a.ry = s.ry;
+    a.part_rr = part(P0);
+    const int rc = deep_cheby(n, ch_alphas + st, ch_betas + st, a, p == 1, &nparts);
+    if (rc) return -rc;
+    s.ucur = 1 - s.ucur;
+    s.pcur = 1 - s.pcur;
+    done += n;
+    left -= n;
+  }
+  if (want_norm) {
+    const int slot = P0;
+    const int rc = finish_sums(&slot, 1, nparts, norm);
+    if (rc) return -rc;
+  }
+  return 1;
+}
+
 // Chebyshev iterations through the vector walk; returns 1 if it ran them,
 // 0 if the configuration needs the per-routine kernel (internal faces, or
 // reflective faces with the block preconditioner), or a negative error.
@@ -598,6 +650,8 @@ int cheby_run_fused(const double *ch_alphas, const double *ch_betas, int step_fi
   if (s.precond == TL_PREC_JAC_BLOCK)
     return s.reflective ? 0 : cheby_run_block(ch_alphas, ch_betas, step_first, count, want_norm,
                                               norm);
+  if (!s.reflective && s.precond == TL_PREC_NONE && count >= 2 && deep_fits())
+    return cheby_run_deep(ch_alphas, ch_betas, step_first, count, want_norm, norm);
   const Geo G = geo_resident(2 * BLOCK, TL_CHEBY_PAIR_WAVES);
   const int nb = G.blocks < 0 ? -G.blocks : G.blocks;
   const int diag = s.precond == TL_PREC_JAC_DIAG;

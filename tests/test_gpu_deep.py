@@ -86,3 +86,45 @@ def test_mixed_sweeps(inner):
         finally:
             d.close()
         assert np.linalg.norm(us[1] - us[0]) <= 2e-10 * r0 * 1.01
+
+
+@pytest.mark.parametrize("count", [2, 3, 4, 5, 6, 8, 9, 10, 12, 17, 24, 31])
+def test_cheby_iterations(count):
+    """u, p, w and r after `count` iterations, and u's halo ring, which the
+    passes carry along unread.
+
+    Tolerance as in test_ppcg_sweeps, relative to the largest u and p; w and r
+    hold u's rounding times |A|."""
+    pd = C.POINTER(C.c_double)
+    for nx, ny in SIZES:
+        print(f"deep chebyshev {nx}x{ny} count {count}", flush=True)
+        d, rx, ry = _chunk(nx, ny, 1, False)
+        try:
+            out = []
+            for deep in (0, 1):
+                with env(TL_DEEP=deep):
+                    _start(d, rx, ry)
+                    hi = 1.05 * _norm_a(d, rx, ry)
+                    ca, cb, theta = chebyshev_coefs(hi / 100.0, hi, count + 1)
+                    u = d.download("u")
+                    u[0], u[-1], u[:, 0], u[:, -1] = 3.0, 4.0, 5.0, 6.0
+                    d.upload("u", u)
+                    L.call("tl_cheby_init", theta)
+                    norm = C.c_double()
+                    L.call("tl_cheby_run", ca.ctypes.data_as(pd), cb.ctypes.data_as(pd), 1, count,
+                           1, C.byref(norm))
+                    out.append([interior(d.download(f), 1) for f in ("u", "p", "w", "r")] +
+                               [math.sqrt(norm.value), d.download("u")])
+            norm_a = hi / 1.05
+        finally:
+            d.close()
+        ref, got = out
+        tol = 1000.0 * count * 2.0 ** -53
+        big = float(np.max(np.abs(ref[0])))
+        for i, scale in ((0, big), (1, big), (2, big * norm_a), (3, big * norm_a)):
+            assert np.max(np.abs(got[i] - ref[i])) <= tol * scale, (nx, ny, i)
+        assert abs(got[4] - ref[4]) <= tol * big * norm_a * math.sqrt(nx * ny)
+        ring = np.ones(ref[5].shape, bool)
+        ring[1:-1, 1:-1] = False
+        ring[0, [0, -1]] = ring[-1, [0, -1]] = False  # corners are not carried
+        assert np.array_equal(got[5][ring], ref[5][ring])
