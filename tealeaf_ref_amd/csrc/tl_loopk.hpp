@@ -354,11 +354,22 @@ __global__ __launch_bounds__(BLOCK, TL_W_WAVES) void k_loop_w(Geo G, int n, int 
 #endif
 constexpr int UR_ROWS = TL_UR_ROWS;
 
-// CG iteration n, second pass: alpha = rro/pw; u += alpha p; r -= alpha w;
-// (z = Mi r); partials of r.r or r.z (kernels/tea_leaf_cg_kernel.f90:237-300)
-template <bool NT, typename T, int V>
+// Directions whose u updates one update pass applies together: u += alpha p
+// of CG_DEFER iterations reads and writes u once (24 bytes a cell and
+// iteration become 12), in the order of the iterations, so that u gets the
+// same bits.  The directions wait in as many buffers.
+constexpr int CG_DEFER = 4;
+template <typename T>
+struct CgDefer {
+  const T *p[CG_DEFER];  // directions of iterations n - NP + 1 .. n
+};
+
+// CG iteration n, second pass: alpha = rro/pw; r -= alpha w; (z = Mi r);
+// partials of r.r or r.z (kernels/tea_leaf_cg_kernel.f90:237-300); and u +=
+// alpha p of the last NP iterations (NP = 0: none).
+template <bool NT, typename T, int V, int NP>
 __global__ __launch_bounds__(BLOCK) void k_cg_ur(Geo G, int n, T *__restrict__ u,
-                                                  const T *__restrict__ p, T *__restrict__ r,
+                                                  CgDefer<T> d, T *__restrict__ r,
                                                   const T *__restrict__ w, T *__restrict__ z,
                                                   const T *__restrict__ Mi, int diag,
                                                   const double *__restrict__ prev_part, int nprev,
@@ -366,6 +377,9 @@ __global__ __launch_bounds__(BLOCK) void k_cg_ur(Geo G, int n, T *__restrict__ u
                                                   const double *__restrict__ hrro,
                                                   double *__restrict__ halpha, int rev) {
   typedef typename dev::Vec<T, V>::type VT;
+  // rows of loads in flight: fewer with more fields
+  constexpr int ROWS = NP ? UR_ROWS / 2 : UR_ROWS;
+  constexpr int NA = NP ? NP : 1;
   __shared__ double lds[BLOCK / WAVE];
   if (ctl->stop) return;
   const double pw = dev::sum_partials(prev_part, nprev, lds);
@@ -373,35 +387,42 @@ __global__ __launch_bounds__(BLOCK) void k_cg_ur(Geo G, int n, T *__restrict__ u
   const double alpha = hrro[n] / pw;
   if (blockIdx.x == 0 && threadIdx.x == 0) halpha[n] = alpha;
   const T a = (T)alpha;
+  T al[NA];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) al[i] = i + 1 < NP ? (T)halpha[n - NP + 1 + i] : a;
   const long P = G.pitch;
   double acc = 0.0;
+  auto update_u = [&](VT uv, const VT (&pv)[NA]) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) uv = uv + al[i] * pv[i];
+    return uv;
+  };
+  constexpr bool NT_U = NT && (TL_ST_NT_LOOP || (TL_ST_NT_U && sizeof(T) == 8));
   dev::TileIter it(G.tiles, G.blocks);
   for (long t = it.t; t < it.t_end; ++t) {
     const dev::TileV<V> tt = dev::tilev_of<V>(G, t);
     if (tt.c >= G.nx) continue;
     int k = tt.y0;
     if (!diag) {
-      // groups of UR_ROWS rows with every load issued before the first
-      // store, so that each lane has 4 x UR_ROWS loads in flight; the r.r
+      // groups of rows with every load issued before the first store; the r.r
       // partial still adds the rows in walking order
-      for (; k + UR_ROWS <= tt.y1; k += UR_ROWS) {
-        VT uu[UR_ROWS], pp[UR_ROWS], rr[UR_ROWS], ww[UR_ROWS];
+      for (; k + ROWS <= tt.y1; k += ROWS) {
+        VT uu[ROWS], pp[ROWS][NA], rr[ROWS], ww[ROWS];
 #pragma unroll
-        for (int q = 0; q < UR_ROWS; ++q) {
+        for (int q = 0; q < ROWS; ++q) {
           const int y = rev ? tt.y1 - 1 - (k + q - tt.y0) : k + q;
           const long i = (long)y * P + tt.c;
-          uu[q] = dev::ldv<NT, T, V>(u + i);
-          pp[q] = dev::ldv<(NT && TL_LD_NT_UR), T, V>(p + i);
+          if (NP) uu[q] = dev::ldv<NT, T, V>(u + i);
+#pragma unroll
+          for (int m = 0; m < NP; ++m) pp[q][m] = dev::ldv<(NT && TL_LD_NT_UR), T, V>(d.p[m] + i);
           rr[q] = dev::ldv<NT, T, V>(r + i);
           ww[q] = dev::ldv<(NT && TL_LD_NT_UR), T, V>(w + i);
         }
 #pragma unroll
-        for (int q = 0; q < UR_ROWS; ++q) {
+        for (int q = 0; q < ROWS; ++q) {
           const int y = rev ? tt.y1 - 1 - (k + q - tt.y0) : k + q;
-          const VT uv = uu[q] + a * pp[q];
           const VT rv = rr[q] - a * ww[q];
-          dev::stv<(NT && (TL_ST_NT_LOOP || (TL_ST_NT_U && sizeof(T) == 8))), T, V>(
-              u + (long)y * P, tt.c, G.nx, uv);
+          if (NP) dev::stv<NT_U, T, V>(u + (long)y * P, tt.c, G.nx, update_u(uu[q], pp[q]));
           dev::stv<(NT && TL_ST_NT_LOOP), T, V>(r + (long)y * P, tt.c, G.nx, rv);
 #pragma unroll
           for (int e = 0; e < V; ++e)
@@ -412,10 +433,14 @@ __global__ __launch_bounds__(BLOCK) void k_cg_ur(Geo G, int n, T *__restrict__ u
     for (; k < tt.y1; ++k) {
       const int y = rev ? tt.y1 - 1 - (k - tt.y0) : k;
       const long i = (long)y * P + tt.c;
-      const VT uv = dev::ldv<NT, T, V>(u + i) + a * dev::ldv<(NT && TL_LD_NT_UR), T, V>(p + i);
       const VT rv = dev::ldv<NT, T, V>(r + i) - a * dev::ldv<(NT && TL_LD_NT_UR), T, V>(w + i);
-      dev::stv<(NT && (TL_ST_NT_LOOP || (TL_ST_NT_U && sizeof(T) == 8))), T, V>(
-          u + (long)y * P, tt.c, G.nx, uv);
+      if (NP) {
+        VT pv[NA];
+#pragma unroll
+        for (int m = 0; m < NP; ++m) pv[m] = dev::ldv<(NT && TL_LD_NT_UR), T, V>(d.p[m] + i);
+        dev::stv<NT_U, T, V>(u + (long)y * P, tt.c, G.nx,
+                             update_u(dev::ldv<NT, T, V>(u + i), pv));
+      }
       dev::stv<(NT && TL_ST_NT_LOOP), T, V>(r + (long)y * P, tt.c, G.nx, rv);
       if (diag) {
         const VT zv = dev::ldv<NT, T, V>(Mi + i) * rv;
@@ -432,6 +457,28 @@ __global__ __launch_bounds__(BLOCK) void k_cg_ur(Geo G, int n, T *__restrict__ u
   }
   acc = dev::block_sum(acc, lds);
   if (threadIdx.x == 0) out_part[blockIdx.x] = acc;
+}
+
+// The u updates of the `count` iterations up to n that a loop's end left over.
+template <typename T, int V>
+__global__ __launch_bounds__(BLOCK) void k_cg_u(Geo G, int n, int count, T *__restrict__ u,
+                                                 CgDefer<T> d,
+                                                 const double *__restrict__ halpha) {
+  typedef typename dev::Vec<T, V>::type VT;
+  const long P = G.pitch;
+  dev::TileIter it(G.tiles, G.blocks);
+  for (long t = it.t; t < it.t_end; ++t) {
+    const dev::TileV<V> tt = dev::tilev_of<V>(G, t);
+    if (tt.c >= G.nx) continue;
+    for (int y = tt.y0; y < tt.y1; ++y) {
+      const long i = (long)y * P + tt.c;
+      VT uv = dev::ldv<true, T, V>(u + i);
+#pragma unroll
+      for (int m = 0; m < CG_DEFER - 1; ++m)
+        if (m < count) uv = uv + (T)halpha[n - count + 1 + m] * dev::ldv<true, T, V>(d.p[m] + i);
+      dev::stv<true, T, V>(u + (long)y * P, tt.c, G.nx, uv);
+    }
+  }
 }
 
 // CG iteration n, second pass with the block-Jacobi preconditioner:
@@ -985,7 +1032,16 @@ struct LoopBufs {
   // G's tiles then start on multiples of 4 rows
   int block = 0;
   const T *Di = nullptr, *cp = nullptr, *bfp = nullptr;
+  // two more buffers for directions, which nothing else uses during CG
+  T *spare[2] = {nullptr, nullptr};
 };
+
+// The u updates of CG_DEFER iterations in one pass unless TL_CG_DEFER=0 (read
+// on every call).
+inline bool cg_defer() {
+  const char *e = getenv("TL_CG_DEFER");
+  return !e || atoi(e) != 0;
+}
 
 inline int abs_blocks(const Geo &G) { return G.blocks < 0 ? -G.blocks : G.blocks; }
 
@@ -1154,40 +1210,57 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   const int nb = abs_blocks(G);
   const bool nt = use_nontemporal();
   auto kw = nt ? k_loop_w<true, T, V> : k_loop_w<false, T, V>;
-  auto kur = nt ? k_cg_ur<true, T, V> : k_cg_ur<false, T, V>;
+  // u is updated once for CG_DEFER iterations, whose directions go round as
+  // many buffers; with the block preconditioner in every iteration
+  const bool defer = !b.block && cg_defer();
+  auto kur0 = nt ? k_cg_ur<true, T, V, 0> : k_cg_ur<false, T, V, 0>;
+  auto kur1 = nt ? k_cg_ur<true, T, V, 1> : k_cg_ur<false, T, V, 1>;
+  auto kurN = nt ? k_cg_ur<true, T, V, CG_DEFER> : k_cg_ur<false, T, V, CG_DEFER>;
   auto kub = nt ? k_cg_ur_blk<true, T, V> : k_cg_ur_blk<false, T, V>;
   const int c0 = *b.pcur;
+  T *ring[CG_DEFER] = {b.p[c0], b.p[1 - c0], b.spare[0], b.spare[1]};
+  const int turn = defer ? CG_DEFER : 2;
+  // the direction entering iteration i of this call (from 0), and the one it makes
+  auto p_in = [&](int i) { return ring[i % turn]; };
+  auto p_out = [&](int i) { return ring[(i + 1) % turn]; };
   LoopParams lp;
   lp.eps_abs = st->eps_abs;
   lp.epslim = st->epslim;
   lp.check_switch = st->check_switch;
   lp.presteps = st->presteps;
   auto launch = [&](int n, bool first) -> int {
-    const int cin = c0 ^ ((n - st->n_first) & 1);
-    const T *pin = (first && pin_first) ? pin_first : b.p[cin];
+    const int i = n - st->n_first;
+    const T *pin = (first && pin_first) ? pin_first : p_in(i);
     hipEvent_t ev;
     prof_arm(0, &ev);
     klaunch(kw, dim3(nb), dim3(BLOCK), G, n, first ? 1 : 0, 0, lp,
-            st->rro, b.cg_src, pin, b.p[1 - cin], b.Kx, b.Ky, b.w, b.rx, b.ry,
+            st->rro, b.cg_src, pin, p_out(i), b.Kx, b.Ky, b.w, b.rx, b.ry,
             m.part(P2), nb, m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1);
     prof_end(0, ev);
     prof_arm(1, &ev);
     if (b.block)
-      klaunch(kub, dim3(nb), dim3(BLOCK), G, n, b.u, b.p[1 - cin], b.r,
+      klaunch(kub, dim3(nb), dim3(BLOCK), G, n, b.u, p_out(i), b.r,
               b.w, b.z, b.Di, b.Ky, b.cp, b.bfp, b.ry, m.part(P1), nb, m.part(P2),
               m.ctl, m.hrro, m.halpha, 1);
-    else
-      klaunch(kur, dim3(nb), dim3(BLOCK), G, n, b.u, b.p[1 - cin], b.r,
-              b.w, b.z, b.Mi, b.diag, m.part(P1), nb, m.part(P2), m.ctl, m.hrro,
-              m.halpha, 1);
+    else {
+      CgDefer<T> d = {};
+      auto kur = kur1;
+      d.p[0] = p_out(i);
+      if (defer) {
+        kur = i % CG_DEFER == CG_DEFER - 1 ? kurN : kur0;
+        for (int m = 0; m < CG_DEFER; ++m) d.p[m] = p_out(i + 1 + m);  // i + 1 - CG_DEFER + m
+      }
+      klaunch(kur, dim3(nb), dim3(BLOCK), G, n, b.u, d, b.r, b.w, b.z, b.Mi, b.diag, m.part(P1),
+              nb, m.part(P2), m.ctl, m.hrro, m.halpha, 1);
+    }
     prof_end(1, ev);
     TL_HIP(hipGetLastError());
     return TL_OK;
   };
   auto tail = [&](int n) -> int {
-    const int cin = c0 ^ ((n - st->n_first) & 1);
+    const int i = n - st->n_first;
     hipLaunchKernelGGL(kw, dim3(nb), dim3(BLOCK), 0, s.stream, G, n, 0, 1, lp, st->rro, b.cg_src,
-                       b.p[cin], b.p[1 - cin], b.Kx, b.Ky, b.w, b.rx, b.ry, m.part(P2), nb,
+                       (const T *)p_in(i), p_out(i), b.Kx, b.Ky, b.w, b.rx, b.ry, m.part(P2), nb,
                        m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1);
     TL_HIP(hipGetLastError());
     return TL_OK;
@@ -1206,12 +1279,30 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   st->error = res.error;
   st->rro = res.rro;
   st->old_error = res.old_error;
-  if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("CG", res.n_end);
   if (!ran) {
+    // iterations whose update pass has run: not the one in which a switch or a
+    // non-finite p.w was found
+    const bool at_end = res.reason == TL_LOOP_SWITCH ||
+                        (res.reason == TL_LOOP_NONFINITE && res.stop == STOP_UPDATE);
+    const int done = res.n_end - st->n_first + (at_end ? 0 : 1);
+    const int left = defer ? done % CG_DEFER : 0;
+    if (left > 0) {
+      CgDefer<T> d = {};
+      for (int q = 0; q < left; ++q) d.p[q] = p_out(done - left + q);
+      hipLaunchKernelGGL((k_cg_u<T, V>), dim3(nb), dim3(BLOCK), 0, s.stream, G,
+                         st->n_first + done - 1, left, b.u, d, m.halpha);
+      TL_HIP(hipGetLastError());
+    }
     // the launch that stopped the loop applied the last p update
-    const int n_det = res.reason == TL_LOOP_SWITCH ? res.n_end : res.n_end + 1;
-    *b.pcur = c0 ^ ((n_det - st->n_first + 1) & 1);
+    T *p_last = p_out(done);
+    if (p_last == b.p[0] || p_last == b.p[1]) {
+      *b.pcur = p_last == b.p[0] ? 0 : 1;
+    } else {
+      TL_HIP(hipMemcpy2DAsync(b.p[c0], G.pitch * sizeof(T), p_last, G.pitch * sizeof(T),
+                              G.nx * sizeof(T), G.ny, hipMemcpyDeviceToDevice, s.stream));
+    }
   }
+  if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("CG", res.n_end);
   const int last_done = res.reason == TL_LOOP_SWITCH ? res.n_end - 1 : res.n_end;
   if ((rc = copy_hist(cg_alphas, m.halpha, st->n_first, last_done))) return rc;
   if ((rc = copy_hist(cg_betas, m.hbeta, st->n_first, last_done))) return rc;

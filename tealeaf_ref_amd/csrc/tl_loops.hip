@@ -735,6 +735,9 @@ LoopBufs<double> fp64_bufs() {
   b.cp = s.cp.p11;
   b.bfp = s.bfp.p11;
   b.cg_src = (b.diag || b.block || s.ppcg_active) ? s.z.p11 : s.r.p11;
+  // the buffers that u's and sd's current ones alternate with
+  b.spare[0] = s.u[1 - s.ucur].p11;
+  b.spare[1] = s.sd[1 - s.sdcur].p11;
   if (b.block) {
     // tiles start on the 4-row blocks of the preconditioner
     Geo &G = b.G;

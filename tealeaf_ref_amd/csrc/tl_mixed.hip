@@ -272,6 +272,8 @@ LoopBufs<float> f32_bufs(int &pcur, int &sdcur) {
   b.ry = (float)s.ry;
   b.diag = 0;
   b.cg_src = f32(R);
+  b.spare[0] = f32(SD_0);  // CG has no sd
+  b.spare[1] = f32(SD_1);
   return b;
 }
 
