@@ -1,30 +1,28 @@
-// Many sweeps of a stencil recurrence in one pass over the mesh (temporal
-// blocking), for PPCG's inner steps (k_deep_ppcg): `steps` sweeps
-//   rtemp -= A sd;  sd' = alpha sd + beta rtemp;  utemp += sd'
-// read r and the faces once and write z once, 40 bytes per cell in FP64
-// instead of 64 for every two sweeps.
+// Many steps of a stencil recurrence in one pass over the mesh (temporal
+// blocking): PPCG's inner sweeps (k_deep_ppcg) and Chebyshev iterations
+// (k_deep_cheby).  The fields are read and written once for all the steps.
 //
 // A wave walks a strip of 64 V columns upwards on its own, with no barrier.
-// Sweep s ("stage s") runs s rows behind the row being loaded: at the step that
-// loads row y, stage s turns sd of sweep s - 1 on rows y-s-1, y-s, y-s+1 into
-// sd of sweep s on row y-s, the last of the three coming from stage s - 1 in
-// the same step.  Every stage keeps two rows of sd and one of rtemp and utemp
-// in registers; the faces and the diagonal of the last STAGES rows, which all
-// stages need in turn, lie in a ring in the wave's own LDS.  The outermost
-// columns and the first and last STAGES rows of a strip are ghosts: each
-// stage's results are wrong one column and row further in, so STAGES on every
-// side (rounded up to whole vectors) are walked and thrown away.  Faces on
-// the mesh's edge are taken as zero (a mirrored neighbour's two terms
-// cancel), and cells outside the mesh as zero with zero faces, so that the
-// mesh's edge needs no code in the stages.
+// Step s ("stage s") runs s rows behind the row being loaded: when row y is
+// loaded, stage s turns the field after s steps on rows y-s-2, y-s-1, y-s into
+// the field after s + 1 steps on row y-s-1, the last of the three coming from
+// stage s - 1 in the same turn.  A stage keeps two rows of the field in
+// registers; what the rows hold for all stages in turn (faces, diagonal, right
+// hand side) lies for the last STAGES rows in a ring in the wave's own LDS.
+// The outermost columns and the first and last STAGES rows of a strip are
+// ghosts: each stage's results are wrong one column and row further in, so
+// STAGES on every side (rounded up to whole vectors) are walked and thrown
+// away.  Faces on the mesh's edge are taken as zero (a mirrored neighbour's two
+// terms cancel), and cells outside the mesh as zero with zero faces, so that
+// the mesh's edge needs no code in the stages.
 #pragma once
 
 #include "tl_stencilv.hpp"
 
 namespace tl {
 
-// Most stages of one kernel: 10 rows x 3 fields x 1 KB of ring per wave are
-// 120 KB of the CU's 160 KB for four waves.
+// Most stages of one kernel: 10 rows x 4 fields x 1 KB of ring per wave are
+// the CU's 160 KB for four waves.
 constexpr int DEEP_MAX = 10;
 
 template <typename T>
@@ -41,8 +39,9 @@ struct DeepGeo {
 
 namespace dev {
 
-// The coefficients of the sweeps, sweep s's in lane s of vector registers: as
-// scalars over the whole unrolled loop they would be spilled.
+// The coefficients of the steps, step s's in lane s of vector registers: as
+// scalars over the whole unrolled loop they are spilled where the kernel has
+// many other scalars (Chebyshev's pass).
 template <typename T>
 struct LaneCoef {
   T a, b;
@@ -72,11 +71,10 @@ struct LaneCoef {
 };
 
 // Rows in flight: loads run this far ahead of the stages.  A divisor of the
-// ring's length, so that the unrolled rows use fixed registers.
-constexpr int deep_ahead(int stages) {
-  (void)stages;
-  return 2;
-}
+// ring's length, so that the unrolled rows use fixed registers.  Five rows
+// instead of two gained nothing at 4096^2 (PPCG FP64 204 us for 206, FP32 136 for
+// 130, Chebyshev 211 for 208).
+constexpr int DEEP_AHEAD = 2;
 
 constexpr int deep_ghost(int stages, int V) { return (stages + V - 1) / V * V; }
 constexpr int deep_strip(int stages, int V) { return WAVE * V - 2 * deep_ghost(stages, V); }
@@ -124,19 +122,26 @@ __device__ inline T keep(T v, unsigned m) {
   }
 }
 
-// What a wave holds of its strip.
+// What a wave holds of its strip.  Rows are read and written through buffer
+// descriptors of their own, whose length is the mesh's width, or 0 for a row
+// that is none: what is read outside is zero and what is written there is
+// dropped, in the hardware, so that no lane is masked and no branch splits the
+// unrolled rows.  (Masks by bits, a row address per lane and stores behind a
+// branch took 60 of the 540 instructions of a row of ten sweeps, and registers
+// that the stages' rows then lacked.)
 template <typename T, int V, int STAGES>
 struct DeepStrip {
   typedef typename Vec<T, V>::type VT;
+  typedef unsigned U4 __attribute__((ext_vector_type(4)));
+  static_assert(sizeof(VT) == 16, "a lane's columns are one 16-byte access");
   int lane, c;               // first column of the lane
-  unsigned off;              // bytes from the row to it, clamped into the row
   int y0, y1;                // rows this wave stores
   int first, last;           // rows it loads
   bool live;                 // a tile exists
   bool left_edge, right_edge;  // it has the mesh's first / last column
-  bool out, part;            // the lane's columns are stored; only some of them
-  bool any_part;             // ... in some lane of the wave
-  unsigned in[V], face[V];   // the lane's cells in the mesh; with a face on the left
+  bool mine;                 // the lane's columns are the strip's own, and in the mesh
+  unsigned off_in, off_out;  // bytes from the row to them; where they are not mine, beyond it
+  unsigned face0;            // bits of the lane's first left face: none on the mesh's edge
   int nx, ny;
   long pitch;
 
@@ -145,53 +150,45 @@ struct DeepStrip {
     const int strip = wave_id % g.strips, tile = wave_id / g.strips;
     live = tile < g.tiles;
     constexpr int G = deep_ghost(STAGES, V), S = deep_strip(STAGES, V);
-    const int x0 = strip * S - G;
-    c = x0 + V * lane;
+    c = strip * S - G + V * lane;
     nx = g.nx;
     ny = g.ny;
     pitch = g.pitch;
-    const int top = (nx / V) * V;
-    off = (unsigned)(c < 0 ? 0 : (c > top ? top : c)) * (unsigned)sizeof(T);
     y0 = tile * g.rows;
     y1 = y0 + g.rows < ny ? y0 + g.rows : ny;
     first = y0 - STAGES > 0 ? y0 - STAGES : 0;
     last = y1 - 1 + STAGES;
-    out = c >= strip * S && c < (strip + 1) * S && c < nx;
-    part = out && c + V > nx;
+    mine = c >= strip * S && c < (strip + 1) * S && c < nx;
     left_edge = strip == 0;
     right_edge = strip == g.strips - 1;
-    any_part = __any(part);
-    out = out && !part;
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      in[e] = c + e >= 0 && c + e < nx ? ~0u : 0u;
-      face[e] = c + e > 0 && c + e < nx ? ~0u : 0u;
-    }
+    constexpr unsigned NOWHERE = ~0u - 15u;
+    off_in = c < 0 ? NOWHERE : (unsigned)c * (unsigned)sizeof(T);
+    off_out = mine ? off_in : NOWHERE;
+    face0 = c == 0 ? 0u : ~0u;
   }
-  // the lane's cells of a row that starts at element `row` of a field
-  __device__ VT load(const T *__restrict__ f, long row) const {
-    return *(const VT *)((const char *)(f + row) + off);
+  // the row that starts at element `row` of a field; none if !is
+  __device__ __amdgpu_buffer_rsrc_t desc(const T *f, long row, bool is) const {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(f + row), 0,
+                                             is ? nx * (int)sizeof(T) : 0, 0x00027000);
   }
-  // zero where the mesh is not: by bits and not by compares, whose masks
-  // would fill the scalar registers over the unrolled rows
-  __device__ static VT masked(VT v, const unsigned (&m)[V], bool row) {
-    const unsigned r = row ? ~0u : 0u;
-#pragma unroll
-    for (int e = 0; e < V; ++e) v[e] = keep(v[e], m[e] & r);
+  __device__ VT load(const T *f, long row, bool is) const {
+    return __builtin_bit_cast(
+        VT, __builtin_amdgcn_raw_buffer_load_b128(desc(f, row, is), (int)off_in, 0, 0));
+  }
+  __device__ void store(T *f, long row, VT v, bool is) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, v), desc(f, row, is),
+                                           (int)off_out, 0, 0);
+  }
+  // faces on the left: none on the mesh's edge
+  __device__ VT faces_x(VT v) const {
+    v[0] = keep(v[0], face0);
     return v;
   }
-  __device__ VT cells(VT v, int y) const { return masked(v, in, y < ny); }
-  __device__ VT cells_if(VT v, bool row) const { return masked(v, in, row); }
-  __device__ VT faces_x(VT v, int y) const { return masked(v, face, y < ny); }
-  __device__ VT faces_y(VT v, int y) const { return masked(v, in, y > 0 && y < ny); }
-  // Rows that are not stored (ok false) pass through the same instructions with
-  // no lane on: a branch around the store would leave the compiler unsure how
-  // many are in flight, and it would then wait for them with the loads.
-  __device__ void store(T *f, long row, VT v, bool ok) const {
-    if (out & ok) *(VT *)((char *)(f + row) + off) = v;
-    if (any_part) {
-      if (part & ok) stv<false, T, V>(f + row, c, nx, v);
-    }
+  // zero unless `row`: by bits and not by a compare per element
+  __device__ static VT only_if(VT v, bool row) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) v[e] = keep(v[e], row ? ~0u : 0u);
+    return v;
   }
 };
 

@@ -14,7 +14,7 @@ namespace tl {
 // The ring of up to eight stages holds the diagonal too (8 rows x 4 fields x
 // 1 KB per wave, 128 KB of the CU's 160 KB for four waves); with ten stages it
 // does not fit, and every stage forms it from the faces again.
-constexpr bool deep_cheby_di(int stages) { return stages <= 8; }
+constexpr bool deep_cheby_di(int stages) { return stages <= 10; }
 constexpr int deep_cheby_fields(int stages) { return deep_cheby_di(stages) ? 4 : 3; }
 
 struct DeepCheby {
@@ -55,13 +55,14 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
   long row_l = (long)yl * t.pitch;
   auto load = [&]() {
     In i;
-    i.kx = t.load(a.Kx, row_l);
-    i.ky = t.load(a.Ky, row_l);
-    i.u = t.load(a.u, row_l);
-    i.p = t.load(a.p, row_l);
-    i.u0 = t.load(a.u0, row_l);
+    const bool is = yl < t.ny;
+    i.kx = t.load(a.Kx, row_l, is);
+    i.ky = t.load(a.Ky, row_l, is && yl > 0);
+    i.u = t.load(a.u, row_l, is);
+    i.p = t.load(a.p, row_l, is);
+    i.u0 = t.load(a.u0, row_l, is);
     yl += 1;
-    row_l += yl < t.ny ? t.pitch : 0;
+    row_l += t.pitch;
     return i;
   };
   dev::LaneCoef<T> cs(co);
@@ -73,24 +74,23 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
     for (int s = 0; s < STAGES; ++s) behind[s] = centre[s] = ps[s] = VT(0);
     VT kx1 = VT(0), ky1 = VT(0), u01 = VT(0);
     for (int i = 0; i < STAGES * NF; ++i) ring[i * WAVE] = VT(0);
-    constexpr int AHEAD = dev::deep_ahead(STAGES);
+    constexpr int AHEAD = dev::DEEP_AHEAD;
     In q[AHEAD];
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i) q[i] = load();
-    long row_o = (long)t.y0 * t.pitch;
+    long row_o = ((long)t.first - STAGES) * t.pitch;
     struct Faces {
       VT kx, ky, di, u0;
     };
     auto step = [&](int y, In &qi, const int slot) {
       In in = qi;
-      asm volatile("" : "+v"(cs.a), "+v"(cs.b));  // no readlane leaves the row
+      // no readlane and no multiple of the pitch leaves the row to wait for it
+      // in a register
+      asm volatile("" : "+v"(cs.a), "+v"(cs.b), "+s"(row_l), "+s"(row_o));
       const int yo = y - STAGES;
       qi = load();
-      in.kx = t.faces_x(in.kx, y);
-      in.ky = t.faces_y(in.ky, y);
-      in.u = t.cells(in.u, y);
-      in.p = t.cells(in.p, y);
-      in.u0 = t.cells(in.u0, y);
+      in.kx = t.faces_x(in.kx) * a.rx;
+      in.ky = in.ky * a.ry;
       VT kyu = in.ky;
       Faces f = {kx1, ky1, VT(0), u01};
       T kxr = dev::from_above(f.kx[0]);
@@ -98,8 +98,7 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
         VT d;
 #pragma unroll
         for (int e = 0; e < V; ++e)
-          d[e] = T(1) + a.ry * (up[e] + k.ky[e]) +
-                 a.rx * (dev::vec_right<T, V>(k.kx, e, right) + k.kx[e]);
+          d[e] = T(1) + (up[e] + k.ky[e]) + (dev::vec_right<T, V>(k.kx, e, right) + k.kx[e]);
         return d;
       };
       f.di = diagonal(f, kyu, kxr);
@@ -126,10 +125,15 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
         for (int e = 0; e < V; ++e) {
           const T l = dev::vec_left<T, V>(c, e, lo), rr = dev::vec_right<T, V>(c, e, hi);
           const T kr = dev::vec_right<T, V>(f.kx, e, kxr);
-          w[e] = f.di[e] * c[e] - a.ry * (kyu[e] * ahead[e] + f.ky[e] * behind[s][e]) -
-                 a.rx * (kr * rr + f.kx[e] * l);
+          if (LAST && s + 1 == STAGES) {
+            w[e] = f.di[e] * c[e] - kr * rr - f.kx[e] * l - f.ky[e] * behind[s][e] -
+                   kyu[e] * ahead[e];
+            r[e] = f.u0[e] - w[e];
+          } else {
+            r[e] = f.u0[e] - f.di[e] * c[e] + kr * rr + f.kx[e] * l + f.ky[e] * behind[s][e] +
+                   kyu[e] * ahead[e];
+          }
         }
-        r = f.u0 - w;
         const VT pn = cs.alpha(s) * p + cs.beta(s) * r;
         const VT un = c + pn;
         behind[s] = c;
@@ -153,11 +157,11 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
       if (LAST) {
         t.store(a.w, row_o, w, ok);
         t.store(a.r, row_o, r, ok);
-        r = t.cells_if(r, ok);
+        r = t.only_if(r, ok);
 #pragma unroll
         for (int e = 0; e < V; ++e) acc += r[e] * r[e];
       }
-      row_o += ok ? t.pitch : 0;
+      row_o += t.pitch;
     };
     // steps past the last row store nothing
     for (int y = t.first; y <= t.last; y += STAGES) {
@@ -175,14 +179,14 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
     for (int side = 0; side < 2; ++side) {
       if (side ? t.y1 != t.ny : t.y0 != 0) continue;
       const long hr = side ? (long)t.ny * t.pitch : -t.pitch;
-      if (t.out || t.part)
+      if (t.mine)
         for (int e = 0; e < V; ++e)
           if (t.c + e < t.nx) a.u_out[hr + t.c + e] = a.u[hr + t.c + e];
     }
   }
   if (LAST) {
     // cells outside the mesh have u0 = A u = 0; ghosts are not the lane's
-    if (!t.out && !t.part) acc = 0.0;
+    if (!t.mine) acc = 0.0;
     __syncthreads();
     acc = dev::block_sum(acc, (double *)dyn);
     if (threadIdx.x == 0) a.part_rr[blockIdx.x] = acc;

@@ -459,12 +459,15 @@ __global__ __launch_bounds__(BLOCK) void k_cg_ur(Geo G, int n, T *__restrict__ u
   if (threadIdx.x == 0) out_part[blockIdx.x] = acc;
 }
 
-// The u updates of the `count` iterations up to n that a loop's end left over.
+// The u updates of the `count` iterations up to n: what a CG loop's end left
+// over, and PPCG's, which a stop that `ctl` tells of leaves to the loop's end.
 template <typename T, int V>
 __global__ __launch_bounds__(BLOCK) void k_cg_u(Geo G, int n, int count, T *__restrict__ u,
                                                  CgDefer<T> d,
-                                                 const double *__restrict__ halpha) {
+                                                 const double *__restrict__ halpha,
+                                                 const Ctl *ctl) {
   typedef typename dev::Vec<T, V>::type VT;
+  if (ctl && ctl->stop) return;
   const long P = G.pitch;
   dev::TileIter it(G.tiles, G.blocks);
   for (long t = it.t; t < it.t_end; ++t) {
@@ -474,9 +477,26 @@ __global__ __launch_bounds__(BLOCK) void k_cg_u(Geo G, int n, int count, T *__re
       const long i = (long)y * P + tt.c;
       VT uv = dev::ldv<true, T, V>(u + i);
 #pragma unroll
-      for (int m = 0; m < CG_DEFER - 1; ++m)
+      for (int m = 0; m < CG_DEFER; ++m)
         if (m < count) uv = uv + (T)halpha[n - count + 1 + m] * dev::ldv<true, T, V>(d.p[m] + i);
       dev::stv<true, T, V>(u + (long)y * P, tt.c, G.nx, uv);
+    }
+  }
+}
+
+// Two fields change places, cell by cell.
+template <typename T, int V>
+__global__ __launch_bounds__(BLOCK) void k_swap(Geo G, T *__restrict__ a, T *__restrict__ b) {
+  typedef typename dev::Vec<T, V>::type VT;
+  dev::TileIter it(G.tiles, G.blocks);
+  for (long t = it.t; t < it.t_end; ++t) {
+    const dev::TileV<V> tt = dev::tilev_of<V>(G, t);
+    if (tt.c >= G.nx) continue;
+    for (int y = tt.y0; y < tt.y1; ++y) {
+      const long row = (long)y * G.pitch;
+      const VT va = dev::ldv<true, T, V>(a + row + tt.c), vb = dev::ldv<true, T, V>(b + row + tt.c);
+      dev::stv<true, T, V>(a + row, tt.c, G.nx, vb);
+      dev::stv<true, T, V>(b + row, tt.c, G.nx, va);
     }
   }
 }
@@ -1066,11 +1086,76 @@ int sweep_parts(const LoopBufs<T> &b, int inner) {
                                             : abs_blocks(b.G);
 }
 
+// What the deep passes of an outer iteration's update need: its iteration n
+// (`first` of the loop, whose z.r is rro), the partials of p.w, and whether n is
+// an odd one of the loop, when r and r_store have changed places.
+struct DeepUpdate {
+  int n, first, npw, nzr, odd;
+  double rro;
+};
+
+// Queue the sweeps of one PPCG outer iteration and its update of r, or those of
+// a preconditioner application when up is null, as up to ten sweeps per pass
+// (tl_deep_ppcg.hpp).  The partials go where queue_sweeps leaves them, except
+// that z.r's alternate between P2 and P4 from iteration to iteration: the first
+// pass of one reads those of the one before.
+template <typename T, int V>
+int queue_deep(const LoopBufs<T> &b, const double *alphas, const double *betas, int inner,
+               T theta_r, const LoopMem &m, const DeepUpdate *up) {
+  const bool odd = up && up->odd;
+  DeepPpcg<T> a = {};
+  T *r = odd ? b.r_store : b.r, *r_new = odd ? b.r : b.r_store;
+  a.Kx = b.Kx;
+  a.Ky = b.Ky;
+  a.z = b.z;
+  a.rx = b.rx;
+  a.ry = b.ry;
+  a.theta_r = theta_r;
+  a.part_rrn = m.part(P3);
+  a.part_zr = m.part(odd ? P4 : P2);
+  a.r = r;
+  if (up) {
+    a.ctl = m.ctl;
+    a.w = b.w;
+    a.r_out = r_new;
+    a.n = up->n;
+    a.first = up->first;
+    a.npw = up->npw;
+    a.nzr = up->nzr;
+    a.rro_in = up->rro;
+    a.part_pw = m.part(P1);
+    a.zr_in = m.part(odd ? P2 : P4);
+    a.hrro = m.hrro;
+    a.halpha = m.halpha;
+  }
+  // between passes z and z one sweep before go through two pairs of buffers
+  T *zs[2] = {b.rtemp, b.w}, *zps[2] = {b.sd[0], b.sd[1]};
+  const int passes = deep_passes(inner);
+  int left = deep_stages(inner), done = 0;
+  for (int p = 0; p < passes; ++p) {
+    const int n = deep_next(left, passes - p);
+    const int count = n < inner - done ? n : inner - done;
+    a.z_in = zs[1 - (p & 1)];
+    a.zp_in = zps[1 - (p & 1)];
+    a.z_out = zs[p & 1];
+    a.zp_out = zps[p & 1];
+    if (p > 0) {
+      a.r = up ? r_new : r;
+      a.r_store = up ? r : b.r_store;
+    }
+    const int rc = deep_pass<T, V>(p > 0 ? 0 : up ? 2 : 1, p + 1 == passes, n, count, b.G.pitch,
+                                   alphas + done, betas + done, a);
+    if (rc) return rc;
+    done += count;
+    left -= n;
+  }
+  return TL_OK;
+}
+
 // Queue the `inner` sweeps of one PPCG outer iteration (or of a preconditioner
-// application when ctl is null): up to ten sweeps per pass (tl_deep_ppcg.hpp),
-// faster at every size measured (256^2 to 4096^2: 1.07 to 4 times); with a
-// preconditioner or fewer than four sweeps, pairs of sweeps in one pass each
-// and a single pass for an odd last one.  sd ping-pongs per pass; rtemp alternates
+// application when ctl is null) where the deep passes do not take them: pairs of
+// sweeps in one pass each and a single pass for an odd last one.  sd ping-pongs
+// per pass; rtemp alternates
 // between b.rtemp and b.w (w is dead between the update and the next w pass).
 // Passes walk in alternating directions starting with `dir`; without pairs,
 // both sweeps of what would be a pair take that pair's direction, so the two
@@ -1109,56 +1194,6 @@ int queue_sweeps(const LoopBufs<T> &b, const double *alphas, const double *betas
       TL_HIP(hipGetLastError());
       return TL_OK;
     }
-  }
-  if (deep_takes(inner, b.diag, b.block)) {
-    DeepPpcg<T> a;
-    a.r = b.r;
-    a.r_store = b.r_store;
-    a.Kx = b.Kx;
-    a.Ky = b.Ky;
-    a.ut_in = a.ut_out = b.utemp;
-    a.z = b.z;
-    a.rx = b.rx;
-    a.ry = b.ry;
-    a.theta_r = theta_r;
-    a.part_rrn = m.part(P3);
-    a.part_zr = m.part(P2);
-    a.ctl = ctl;
-    int i = 0;
-    if (inner & 1) {
-      auto k1 = nt ? k_pp_sweep<true, T, V> : k_pp_sweep<false, T, V>;
-      hipEvent_t ev;
-      prof_arm(2, &ev);
-      klaunch(k1, dim3(nb), dim3(BLOCK), G, 1, 0, want_rrn, theta_r, (T)alphas[0], (T)betas[0],
-              b.diag, (const T *)b.r, (const T *)b.sd[sd], b.sd[1 - sd], rt_cur, b.utemp,
-              (const T *)b.r, (const T *)b.r_store, b.z, b.Mi, b.Kx, b.Ky, b.rx, b.ry, m.part(P3),
-              m.part(P2), ctl, dir);
-      prof_end(2, ev);
-      TL_HIP(hipGetLastError());
-      sd = 1 - sd;
-      i = 1;
-    }
-    for (int left = inner - i, p = deep_passes(inner); p > 0; --p) {
-      const int n = deep_next(left, p);
-      T *rt_next = rt_cur == b.rtemp ? b.w : b.rtemp;
-      a.sd_in = b.sd[sd];
-      a.sd_out = b.sd[1 - sd];
-      a.rt_in = rt_cur;
-      a.rt_out = rt_next;
-      int rc;
-      if (i == 0)
-        rc = p == 1 ? deep_dispatch<T, V, 1, 1>(n, G.pitch, alphas + i, betas + i, a)
-                    : deep_dispatch<T, V, 1, 0>(n, G.pitch, alphas + i, betas + i, a);
-      else
-        rc = p == 1 ? deep_dispatch<T, V, 0, 1>(n, G.pitch, alphas + i, betas + i, a)
-                    : deep_dispatch<T, V, 0, 0>(n, G.pitch, alphas + i, betas + i, a);
-      if (rc) return rc;
-      rt_cur = rt_next;
-      sd = 1 - sd;
-      i += n;
-      left -= n;
-    }
-    return TL_OK;
   }
   auto k1 = nt ? k_pp_sweep<true, T, V> : k_pp_sweep<false, T, V>;
   const T *src = b.diag ? b.z : b.r;
@@ -1290,7 +1325,7 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
       CgDefer<T> d = {};
       for (int q = 0; q < left; ++q) d.p[q] = p_out(done - left + q);
       hipLaunchKernelGGL((k_cg_u<T, V>), dim3(nb), dim3(BLOCK), 0, s.stream, G,
-                         st->n_first + done - 1, left, b.u, d, m.halpha);
+                         st->n_first + done - 1, left, b.u, d, m.halpha, (const Ctl *)nullptr);
       TL_HIP(hipGetLastError());
     }
     // the launch that stopped the loop applied the last p update
@@ -1336,26 +1371,55 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   const T theta_r = (T)(1.0 / theta);
   // Row directions: the w pass walks d, the update -d, the sweep passes
   // alternate from d; with an odd number of sweep passes the next outer
-  // iteration flips d, so every pass starts on the rows written last.
+  // iteration flips d, so every pass starts on the rows written last.  The deep
+  // passes and what goes with them all walk upwards.
   const bool deep = deep_takes(inner, b.diag, b.block);
-  const int passes = (deep ? deep_passes(inner) : inner / 2) + inner % 2;
+  const int passes = inner / 2 + inner % 2;
+  // With the deep passes, whose first updates r, u += alpha p of up to four
+  // iterations is done in one pass (12 to 13 bytes a cell and iteration for
+  // 24).  Their directions go round as many buffers: utemp, which the deep
+  // passes do not use, and, if a single one leaves the sd buffers alone, one of
+  // those.
+  T *ring[CG_DEFER] = {b.p[c0], b.p[1 - c0], b.utemp, b.spare[1]};
+  const int turn = !deep ? 2 : deep_passes(inner) == 1 && b.spare[1] ? 4 : 3;
+  // the direction entering iteration i of this call (from 0), and the one it makes
+  auto p_in = [&](int i) { return ring[i % turn]; };
+  auto p_out = [&](int i) { return ring[(i + 1) % turn]; };
+  // u += alpha p of the `count` iterations of this call before iteration i
+  auto flush_u = [&](int i, int count, const Ctl *ctl) -> int {
+    CgDefer<T> d = {};
+    for (int q = 0; q < count; ++q) d.p[q] = p_out(i - count + q);
+    hipEvent_t ev;
+    prof_arm(6, &ev);
+    klaunch(&k_cg_u<T, V>, dim3(nb), dim3(BLOCK), G, st->n_first + i - 1, count, b.u, d, m.halpha,
+            ctl);
+    prof_end(6, ev);
+    TL_HIP(hipGetLastError());
+    return TL_OK;
+  };
   auto launch = [&](int n, bool first) -> int {
-    const int cin = c0 ^ ((n - st->n_first) & 1);
-    const T *pin = (first && pin_first) ? pin_first : b.p[cin];
-    const int d = (!deep && (passes & 1) && ((n - st->n_first) & 1)) ? -1 : 1;
+    const int i = n - st->n_first;
+    const T *pin = (first && pin_first) ? pin_first : p_in(i);
+    const int d = (!deep && (passes & 1) && (i & 1)) ? -1 : 1;
     hipEvent_t ev;
     prof_arm(5, &ev);
     klaunch(kw, dim3(nb), dim3(BLOCK), G, n, first ? 1 : 0, 0, lp,
-            rro_first, b.z, pin, b.p[1 - cin], b.Kx, b.Ky, b.w, b.rx, b.ry,
+            rro_first, b.z, pin, p_out(i), b.Kx, b.Ky, b.w, b.rx, b.ry,
             m.part(P3), nzr, m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, d);
     prof_end(5, ev);
+    if (deep) {
+      const DeepUpdate up = {n, first ? 1 : 0, nb, nzr, i & 1, rro_first};
+      int rc = queue_deep<T, V>(b, alphas, betas, inner, theta_r, m, &up);
+      if (!rc && (i + 1) % turn == 0) rc = flush_u(i + 1, turn, m.ctl);
+      return rc;
+    }
     prof_arm(6, &ev);
     bool block_ur = false;
     if constexpr (sizeof(T) == 8) {
       if (b.block) {
         auto kub = nt ? k_pp_ur_blk<true, T, V> : k_pp_ur_blk<false, T, V>;
         klaunch(kub, dim3(nb), dim3(BLOCK), G, n, first ? 1 : 0,
-                rro_first, b.u, b.p[1 - cin], b.r, b.r_store, b.w, b.z, b.Di, b.Ky,
+                rro_first, b.u, p_out(i), b.r, b.r_store, b.w, b.z, b.Di, b.Ky,
                 b.cp, b.bfp, b.ry, m.part(P1), m.part(P2), nb, nzr, m.ctl, m.hrro,
                 m.halpha, d > 0 ? 1 : 0);
         block_ur = true;
@@ -1363,16 +1427,16 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
     }
     if (!block_ur)
       klaunch(kur, dim3(nb), dim3(BLOCK), G, n, first ? 1 : 0,
-              rro_first, b.u, b.p[1 - cin], b.r, b.r_store, b.w, b.z, b.Mi, b.diag,
+              rro_first, b.u, p_out(i), b.r, b.r_store, b.w, b.z, b.Mi, b.diag,
               m.part(P1), m.part(P2), nb, nzr, m.ctl, m.hrro, m.halpha, d > 0 ? 1 : 0);
     prof_end(6, ev);
     T *rt_cur = b.rtemp;
     return queue_sweeps<T, V>(b, alphas, betas, inner, theta_r, 1, m.ctl, m, sd, rt_cur, d);
   };
   auto tail = [&](int n) -> int {
-    const int cin = c0 ^ ((n - st->n_first) & 1);
+    const int i = n - st->n_first;
     hipLaunchKernelGGL(kw, dim3(nb), dim3(BLOCK), 0, s.stream, G, n, 0, 1, lp, rro_first, b.z,
-                       b.p[cin], b.p[1 - cin], b.Kx, b.Ky, b.w, b.rx, b.ry, m.part(P3), nzr,
+                       (const T *)p_in(i), p_out(i), b.Kx, b.Ky, b.w, b.rx, b.ry, m.part(P3), nzr,
                        m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1);
     TL_HIP(hipGetLastError());
     return TL_OK;
@@ -1384,12 +1448,30 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   st->error = res.error;
   st->rro = res.rro;
   st->old_error = res.old_error;
-  if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("PPCG", res.n_end);
   const int executed = res.n_end - st->n_first + 1;  // outer iterations that ran
+  if (deep) {
+    // updates that ran: not that of an iteration with a non-finite p.w
+    const int done =
+        executed - (res.reason == TL_LOOP_NONFINITE && res.stop == STOP_UPDATE ? 1 : 0);
+    if (done % turn && (rc = flush_u(done, done % turn, nullptr))) return rc;
+    if (done & 1) {
+      hipLaunchKernelGGL((k_swap<T, V>), dim3(nb), dim3(BLOCK), 0, s.stream, G, b.r, b.r_store);
+      TL_HIP(hipGetLastError());
+    }
+    // the launch that stopped the loop applied the last p update
+    T *p_last = p_out(done);
+    if (p_last == b.p[0] || p_last == b.p[1])
+      *b.pcur = p_last == b.p[0] ? 0 : 1;
+    else
+      TL_HIP(hipMemcpy2DAsync(b.p[c0], G.pitch * sizeof(T), p_last, G.pitch * sizeof(T),
+                              G.nx * sizeof(T), G.ny, hipMemcpyDeviceToDevice, s.stream));
+  } else {
+    *b.pcur = c0 ^ ((executed + 1) & 1);             // + the stopping launch's p update
+    const int swaps = sweep_pairs() ? passes : inner;
+    *b.sdcur = *b.sdcur ^ ((executed * swaps) & 1);
+  }
+  if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("PPCG", res.n_end);
   if (inner_iters) *inner_iters += executed * inner;
-  *b.pcur = c0 ^ ((executed + 1) & 1);               // + the stopping launch's p update
-  const int swaps = sweep_pairs() ? passes : inner;
-  *b.sdcur = *b.sdcur ^ ((executed * swaps) & 1);
   return TL_OK;
 }
 
@@ -1402,6 +1484,8 @@ int run_ppcg_precondition(const LoopBufs<T> &b, const double *alphas, const doub
   int sd = *b.sdcur;
   T *rt_cur = b.rtemp;
   const LoopMem m = loop_mem();
+  if (deep_takes(inner, b.diag, b.block))
+    return queue_deep<T, V>(b, alphas, betas, inner, (T)(1.0 / theta), m, nullptr);
   const int rc = queue_sweeps<T, V>(b, alphas, betas, inner, (T)(1.0 / theta), 0,
                                     (const Ctl *)nullptr, m, sd, rt_cur, 1);
   if (rc) return rc;

@@ -66,6 +66,56 @@ def test_ppcg_sweeps(inner, reflective):
             assert np.max(np.abs(got[i] - ref[i])) <= tol * scale, (nx, ny, i)
 
 
+@pytest.mark.parametrize("inner", [7, 10, 14])
+@pytest.mark.parametrize("outers", [1, 2, 3, 4, 5, 8])
+def test_ppcg_outer_iterations(inner, outers):
+    """Fields after 1 to 8 outer iterations, in which r and r_store change
+    places every time, and the directions and u's updates go round 3 or 4.
+
+    Tolerance: an outer iteration's rounding (test_ppcg_sweeps, through z) is
+    carried on by CG's recurrences; 100 times the sum over the iterations, the
+    condition of the bounds, relative to the largest r or u at the start, is
+    1.3e-9 at most."""
+    pd = C.POINTER(C.c_double)
+    for nx, ny in ((7, 31), (109, 64), (250, 37)):
+        print(f"deep ppcg outer {nx}x{ny} inner {inner} outers {outers}", flush=True)
+        d, rx, ry = _chunk(nx, ny, 1, False)
+        try:
+            out = []
+            for deep in (0, 1):
+                with env(TL_DEEP=deep):
+                    r0 = _start(d, rx, ry)
+                    scale = {"r": float(np.max(np.abs(interior(d.download("r"), 1)))),
+                             "u": float(np.max(np.abs(interior(d.download("u"), 1))))}
+                    hi = 1.05 * _norm_a(d, rx, ry)
+                    ca, cb, theta = chebyshev_coefs(hi / 100.0, hi, inner)
+                    d.scalar("tl_cg_init")
+                    L.call("tl_set_ppcg_active", 1)
+                    d.scalar("tl_ppcg_init", 2)
+                    L.call("tl_ppcg_init_sd", theta)
+                    d.update_halo([0, 0, 0, 0, 0, 1, 1] + [0] * 4, 1)
+                    L.call("tl_ppcg_inner", ca.ctypes.data_as(pd), cb.ctypes.data_as(pd), 1, inner)
+                    L.call("tl_ppcg_update_z")
+                    rro = d.scalar("tl_ppcg_init", 3)
+                    st = L.LoopState(n_first=2, n_last=1 + outers, eps_abs=0.0, rro=rro,
+                                     old_error=r0)
+                    n = C.c_int(0)
+                    rc = L.lib().tl_ppcg_loop(C.byref(st), ca.ctypes.data_as(pd),
+                                              cb.ctypes.data_as(pd), inner, theta, C.byref(n))
+                    L.call("tl_set_ppcg_active", 0)
+                    out.append((rc, st.n_end, n.value,
+                                {f: interior(d.download(f), 1) for f in ("u", "r", "r_store", "z",
+                                                                         "p")}))
+        finally:
+            d.close()
+        ref, got = out
+        assert got[:3] == ref[:3] == (L.TL_OK, 1 + outers, inner * outers)
+        tol = 100.0 * outers * 1000.0 * inner * 2.0 ** -53
+        for f in ("u", "r", "r_store", "z", "p"):
+            err = np.max(np.abs(got[3][f] - ref[3][f]))
+            assert err <= tol * scale["u" if f == "u" else "r"], (nx, ny, f)
+
+
 @pytest.mark.parametrize("inner", [4, 7, 10, 13, 20])
 def test_mixed_sweeps(inner):
     """The FP32 passes inside the refined solver: both ways reach the true
