@@ -70,6 +70,18 @@ struct ResCg {
 // < 0: -(error code)
 template <typename T>
 int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out);
+// The same for the Jacobi iterations of tl_jacobi_loop, u read and written in
+// place.
+struct ResJacobi {
+  double *u;
+  const double *u0, *Kx, *Ky;
+  double rx, ry;
+  int n_first, n_last, n_pause;
+  double eps_abs;
+  Ctl *ctl;
+  double *herr;
+};
+int resident_jacobi(ResJacobi a, long pitch, Ctl *out);
 constexpr int RES_PAUSED = 0;  // reason of a launch that stopped for the host only
 
 bool use_nontemporal();

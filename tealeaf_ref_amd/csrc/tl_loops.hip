@@ -1148,7 +1148,21 @@ extern "C" int tl_jacobi_loop(tl_loop_state *st) {
   // outside the mesh, as the reference reads the never-written halo of un);
   // the per-cell walk otherwise
   const bool vec = s.zb_all;
-  if (vec && sweep_pairs()) return jacobi_loop_pairs(st);
+  if (vec) {
+    const ResJacobi a = {s.u[s.ucur].p11, s.u0.p11,  s.Kx.p11, s.Ky.p11,    s.rx,
+                         s.ry,            st->n_first, st->n_last, 0, st->eps_abs,
+                         (Ctl *)s.ctl,    loop_mem().herr};
+    Ctl res;
+    const int ran = resident_jacobi(a, s.pitch, &res);
+    if (ran < 0) return -ran;
+    if (ran) {
+      st->n_end = res.n_end;
+      st->reason = res.reason;
+      st->error = res.error;
+      return res.reason == TL_LOOP_NONFINITE ? nonfinite_fail("Jacobi", res.n_end) : TL_OK;
+    }
+    if (sweep_pairs()) return jacobi_loop_pairs(st);
+  }
   const Geo G = vec ? geo(2 * BLOCK) : geo(BLOCK);
   const int nb = G.blocks < 0 ? -G.blocks : G.blocks;
   const int u0c = s.ucur;

@@ -260,6 +260,143 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Jacobi: iterations n_first.. of tl_jacobi_loop in one launch
+// ---------------------------------------------------------------------------
+// One exchange per iteration carries the halos of the new u and the sum of
+// |u - un|, so that the exit test of an iteration is settled before the next
+// one begins.  Cells outside the mesh are zero: with external faces whose
+// coefficients are zero nothing crosses them, and reflective faces, whose
+// coefficients are not, are to read zero there (as k_jl_v, ZE); what is held
+// for them is 1 / Di = 0.  The quotient by Di is the product with 1 / Di
+// corrected by its remainder, which gives the division's rounding in three
+// operations for about ten.
+//
+// What bounds it: the exchange, 2.1 us of 3.7 with 225 blocks of five rows
+// (1100x1000: a step of 1000 iterations 14.6 -> 3.8 ms against the pass kernels;
+// 512^2 5.6 -> 2.9, 100^2 3.0 -> 1.2).
+template <int R>
+struct JacobiPlan {
+  static constexpr bool U0_LDS = R >= 6;  // of 256 registers a field takes 4 a row
+  static constexpr size_t BYTES = U0_LDS ? (size_t)R * RES_THREADS * 2 * sizeof(double) : 0;
+};
+
+template <int R>
+__global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi a) {
+  typedef double T;
+  typedef typename dev::Vec<T, 2>::type VT;
+  extern __shared__ char dyn[];
+  __shared__ ResShared<T, R, 2> sh;
+  if (threadIdx.x < 2) sh.dead[threadIdx.x] = 0;
+  const ResTile<T, R> t(g);
+  VT u[R], rdi[R], kx[R], ky[R + 1];
+  Kept<T, R, JacobiPlan<R>::U0_LDS> u0(dyn, 0);
+  T *kxr = sh.kxr[t.wave];
+  // the faces, which the row above and the column right of the mesh have too
+#pragma unroll
+  for (int j = 0; j <= R; ++j) {
+    const int y = t.y0 + j;
+    ky[j] = VT(0);
+    if (t.okx && y <= g.ny) {
+      ky[j] = *(const VT *)t.at(a.Ky, g, t.c, y) * a.ry;
+      if (!t.oky) ky[j].y = T(0);
+    }
+    if (j == R) break;
+    u[j] = t.load(a.u, g, y);
+    u0.set(j, t.load(a.u0, g, y));
+    kx[j] = VT(0);
+    if (t.c <= g.nx && y < g.ny) {
+      kx[j] = *(const VT *)t.at(a.Kx, g, t.c, y) * a.rx;
+      if (t.c == g.nx) kx[j].y = T(0);
+    }
+    if (t.lane == WAVE - 1)
+      kxr[j] = (y < g.ny && t.c + 2 <= g.nx) ? *t.at(a.Kx, g, t.c + 2, y) * a.rx : T(0);
+  }
+  __builtin_amdgcn_wave_barrier();
+  auto right_face = [&](int j) {
+    const T kr = dev::lane_above(kx[j].x), gk = kxr[j];
+    return t.lane == WAVE - 1 ? gk : kr;
+  };
+  auto diagonal = [&](int j, T kr) {
+    VT d;
+    d.x = T(1) + (kx[j].x + kx[j].y) + (ky[j].x + ky[j + 1].x);
+    d.y = T(1) + (kx[j].y + kr) + (ky[j].y + ky[j + 1].y);
+    return d;
+  };
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const VT d = diagonal(j, right_face(j));
+    const bool in = t.y0 + j < g.ny;
+    rdi[j].x = in && t.okx ? T(1) / d.x : T(0);
+    rdi[j].y = in && t.oky ? T(1) / d.y : T(0);
+  }
+  ResGhost<T> gh = load_ghosts<T, R>(t, g, a.u);
+  const bool lead = t.blk == 0 && threadIdx.x == 0;
+  T *side = sh.side[t.wave];
+  double err = 0.0;
+  int reason = 0, n = a.n_first;
+  bool dead = false;
+  unsigned s = 0;
+  __syncthreads();
+  for (;; ++n) {
+    if (t.lane < 2 * R) side[t.lane] = gh.side;
+    __builtin_amdgcn_wave_barrier();
+    double acc = 0.0;
+    VT dn = gh.dn;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const VT c = u[j];
+      // taller tiles form the diagonal anew: no registers to hold it
+      if (R >= 6) {
+        asm volatile("" : "+v"(kx[j].x), "+v"(ky[j].x));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      T l = dev::lane_below(c.y), r = dev::lane_above(c.x);
+      const T gl = side[j], gr = side[R + j], kr = right_face(j);
+      l = t.lane == 0 ? gl : l;
+      r = t.lane == WAVE - 1 ? gr : r;
+      const VT up = j + 1 < R ? u[j + 1 < R ? j + 1 : j] : gh.up;
+      VT b = u0.get(j) + ky[j] * dn + ky[j + 1] * up;
+      b.x = b.x + kx[j].x * l + kx[j].y * c.y;
+      b.y = b.y + kx[j].y * c.x + kr * r;
+      const VT q = b * rdi[j];
+      const VT rem = b - diagonal(j, kr) * q;
+      const VT v = q + rem * rdi[j];
+      acc += fabs(v.x - c.x) + fabs(v.y - c.y);
+      dn = c;
+      u[j] = v;
+    }
+    double sum;
+    if (!dev::res_exchange<true, true>(t, g, sh, s++, acc, &sum, &u, &gh)) {
+      dead = true;
+      break;
+    }
+    err = sqrt(fabs(sum));
+    if (lead) a.herr[n] = err;
+    const bool conv = err < a.eps_abs, bad = !isfinite(err);
+    if (conv || bad || n == a.n_last || n == a.n_pause) {
+      reason = conv               ? TL_LOOP_CONVERGED
+               : bad              ? TL_LOOP_NONFINITE
+               : n == a.n_last    ? TL_LOOP_MAXITERS
+                                  : RES_PAUSED;
+      break;
+    }
+  }
+  if (dead) {
+    if (threadIdx.x == 0) *g.abort_flag = 1;
+    return;
+  }
+  const int col = t.col_anew();
+#pragma unroll
+  for (int j = 0; j < R; ++j) t.store(a.u, g, col, t.y0 + j, u[j]);
+  if (lead) {
+    a.ctl->stop = 1;
+    a.ctl->reason = reason;
+    a.ctl->n_end = n;
+    a.ctl->error = err;
+  }
+}
+
 }  // namespace
 
 namespace tl {
@@ -283,8 +420,9 @@ __global__ void k_res_clear(u64 *__restrict__ p, long n) {
 constexpr long RES_WORDS = (long)(RES_PARTS + RES_HALOS) + 16;
 
 // Rows per lane for an nx x ny mesh, of the counts in `rows` (ascending): 0
-// when no tiling has at most one block per CU.
-int res_rows(int nx, int ny, const int *rows, int nrows) {
+// when no tiling has at most one block per CU.  `syncs` exchanges and `row` us
+// of arithmetic per row make an iteration.
+int res_rows(int nx, int ny, const int *rows, int nrows, int syncs = 2, double row = 0.2) {
   const State &s = S();
   const int forced = env_int("TL_RES_ROWS", 0);
   const int cap = s.cus < RES_MAX_BLOCKS ? s.cus : RES_MAX_BLOCKS;
@@ -296,12 +434,12 @@ int res_rows(int nx, int ny, const int *rows, int nrows) {
     const long ty = (ny + (long)RES_WAVES * R - 1) / ((long)RES_WAVES * R), nb = tx * ty;
     if (nb > cap) continue;
     if (forced == R) return R;
-    // time of an iteration in us: two exchanges, dearer with more blocks, and
-    // the arithmetic of R rows.  Measured per step: 512^2 3.04 ms with R = 1
+    // time of an iteration in us: the exchanges, dearer with more blocks, and
+    // the arithmetic of R rows.  Measured with CG, per step: 512^2 3.04 ms with R = 1
     // (256 blocks), 2.50 with 2, 2.43 with 4, 2.92 with 8; 250^2 (ten steps)
     // 12.5 ms with 1, 12.2 with 2, 13.0 with 4, 16.2 with 8
     const double sync = nb == 1 ? 0.4 : (nb <= 8 ? 1.2 : (nb <= 128 ? 1.4 : 2.1));
-    const double cost = 2.0 * sync + 0.2 * R;
+    const double cost = syncs * sync + row * R;
     if (!best || cost < best_cost) {
       best = R;
       best_cost = cost;
@@ -465,5 +603,31 @@ int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out) {
 }
 template int resident_cg<double>(ResCg<double>, int, long, Ctl *);
 template int resident_cg<float>(ResCg<float>, int, long, Ctl *);
+
+int resident_jacobi(ResJacobi a, long pitch, Ctl *out) {
+  State &s = S();
+  if (!resident_on()) return 0;
+  // with eight rows the kernel spills vector registers (see CgPlan)
+  static constexpr int ROWS[] = {1, 2, 3, 4, 5, 6};
+  const int R = res_rows(s.nx, s.ny, ROWS, 6, 1, 0.2);
+  if (!R) return 0;
+  ResGeo g = res_geo(R, pitch);
+  const int n_first = a.n_first, chunk = res_chunk();
+  for (;;) {
+    const long left = (long)a.n_last - a.n_first + 1;
+    const long run = left < chunk ? left : chunk;
+    a.n_pause = (int)(a.n_first + run - 1);
+    int rc;
+    if ((rc = res_tags(run, &g.epoch))) return -rc;
+#define CASE(RR) R == RR ? res_launch(&k_res_jacobi<RR>, g, a, JacobiPlan<RR>::BYTES)
+    rc = CASE(1) : CASE(2) : CASE(3) : CASE(4) : CASE(5)
+         : res_launch(&k_res_jacobi<6>, g, a, JacobiPlan<6>::BYTES);
+#undef CASE
+    if (rc == RES_REFUSED) return a.n_first == n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
+    if (rc || (rc = res_result(g, a.ctl, out))) return -rc;
+    if (out->reason != RES_PAUSED) return 1;
+    a.n_first = out->n_end + 1;
+  }
+}
 
 }  // namespace tl

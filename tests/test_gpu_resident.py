@@ -149,6 +149,71 @@ def test_cg_in_several_launches():
     assert np.array_equal(u1, u0)
 
 
+def _errors(k):
+    """Exit-test errors of iterations 1..k (the library's array starts at 0)."""
+    err = np.zeros(k + 1)
+    L.call("tl_loop_errors", 1, k, err.ctypes.data_as(C.POINTER(C.c_double)))
+    return err[1:]
+
+
+@pytest.mark.parametrize("rows", [0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("reflective", [False, True])
+def test_jacobi_matches_passes(reflective, rows):
+    """u after a number of Jacobi iterations, in one launch and in several.
+
+    Tolerance: an iteration's rounding is at most 10 operations' on terms of at
+    most the largest u, and an iteration never increases the largest
+    difference of two iterates (its row sums are below 1), so after k
+    iterations the two differ by at most 2 * 10 k 2^-53 max|u|.  The sum of |u -
+    un| then differs by at most twice that per cell, besides its own rounding."""
+    k = 37
+    for nx, ny in SIZES[1:]:  # 1x1 has converged before the first iteration
+        print(f"resident jacobi {nx}x{ny} refl {reflective} rows {rows}", flush=True)
+        d, rx, ry = _chunk(nx, ny, 1, reflective)
+        try:
+            out = []
+            for kw in ({"TL_RESIDENT": 0}, {"TL_RES_ROWS": rows},
+                       {"TL_RES_ROWS": rows, "TL_RES_CHUNK": 10}):
+                with env(**kw):
+                    _start(d, rx, ry)
+                    st = L.LoopState(n_first=1, n_last=k, eps_abs=0.0)
+                    assert L.lib().tl_jacobi_loop(C.byref(st)) == L.TL_OK
+                    out.append((st.n_end, st.reason, _errors(k), interior(d.download("u"), 1)))
+        finally:
+            d.close()
+        ref = out[0]
+        big = float(np.max(np.abs(ref[3])))
+        tol = 20.0 * k * 2.0 ** -53 * big
+        for got in out[1:]:
+            assert got[:2] == ref[:2] == (k, L.LOOP_MAXITERS)
+            assert np.max(np.abs(got[3] - ref[3])) <= tol
+            assert np.max(np.abs(got[2] ** 2 - ref[2] ** 2)) <= 2 * tol * nx * ny * 1.01
+        assert np.array_equal(out[1][3], out[2][3])
+
+
+def test_jacobi_exit():
+    """The exit test of an iteration ends the loop there."""
+    d, rx, ry = _chunk(300, 200, 1, False)
+    try:
+        out = []
+        for resident in (0, 1):
+            with env(TL_RESIDENT=resident):
+                _start(d, rx, ry)
+                st = L.LoopState(n_first=1, n_last=60, eps_abs=0.0)
+                assert L.lib().tl_jacobi_loop(C.byref(st)) == L.TL_OK
+                err = _errors(60)
+                for n in (1, 8, 41):  # a bound between the errors of n - 1 and n
+                    eps = 2.0 * err[0] if n == 1 else 0.5 * (err[n - 2] + err[n - 1])
+                    _start(d, rx, ry)
+                    st = L.LoopState(n_first=1, n_last=60, eps_abs=eps)
+                    assert L.lib().tl_jacobi_loop(C.byref(st)) == L.TL_OK
+                    out.append((st.n_end, st.reason))
+                assert out[-3:] == [(n, L.LOOP_CONVERGED) for n in (1, 8, 41)]
+    finally:
+        d.close()
+    assert out[:3] == out[3:]
+
+
 def test_wait_that_runs_out_is_an_error():
     """Every wait of the launch is made to run out (a negative limit): all
     blocks leave the kernel, the call fails, and the next one runs."""
