@@ -60,7 +60,8 @@ __device__ inline ResGhost<T> load_ghosts(const ResTile<T, R> &t, const ResGeo &
 // What bounds it: the two exchanges of an iteration, about 1.4 us each of 4.6
 // (512^2), and with 16 cells per lane the arithmetic (3 of 6 us).  Against
 // the pass kernels: 512^2 step 5.7 -> 2.5 ms, 777x1031 with jac_diag 23.0 ->
-// 4.8 ms, the 1024^2 adjoint's CG solves 155 -> 43 ms.
+// 4.8 ms, 1500x997 with jac_block (eight rows) 87.5 -> 19 ms, the 1024^2 adjoint's
+// CG solves 155 -> 41 ms.
 enum Where { REGS, MEMORY };
 template <typename T, int R, int PREC>
 struct CgPlan {
@@ -92,12 +93,16 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
   Kept<T, R, Plan::U_LDS> u(dyn, 0);
   // Mi of the diagonal preconditioner, where it is kept
   Kept<T, Plan::M == MEMORY || !HAS_Z ? 1 : R, false> m(dyn, 0);
+  // what goes to LDS first, while there are registers to pass through
+  if (Plan::KY_LDS) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < R; ++j) u.set(j, t.load(a.u, g, t.y0 + j));
+  if (Plan::U_LDS) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j = 0; j < R; ++j) {
     const int y = t.y0 + j;
     r[j] = t.load(a.r, g, y);
     p[j] = t.load(a.pin, g, y);
-    u.set(j, t.load(a.u, g, y));
     if constexpr (HAS_Z && Plan::M != MEMORY) m.set(j, t.load(a.Mi, g, y));
   }
   ResGhost<T> pg = load_ghosts<T, R>(t, g, a.pin);
@@ -149,6 +154,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
       r[j] = r[j] - al * w[j];
     }
     bool ok;
+    const int yn = t.row_anew();
     if constexpr (PREC == TL_PREC_NONE) {
 #pragma unroll
       for (int j = 0; j < R; ++j) {
@@ -160,29 +166,33 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
       if constexpr (PREC == TL_PREC_JAC_DIAG) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-          if constexpr (Plan::M == MEMORY) z[j] = t.load(a.Mi, g, t.y0 + j) * r[j];
+          if constexpr (Plan::M == MEMORY) z[j] = t.load(a.Mi, g, yn + j) * r[j];
           else z[j] = m.get(j) * r[j];
         }
       } else {
         // 4-row Thomas solve (tea_block_solve, kernels/tea_leaf_common_kernel.f90:
-        // 378-468); cells outside the mesh have r = 0, bfp = cp = 0 and Di = 1
+        // 378-468); cells outside the mesh have r = 0, bfp = 0 and Di = 1.  cp
+        // above the first row is formed as k_block_init forms it.
 #pragma unroll
         for (int b = 0; b < R; b += 4) {
           __builtin_amdgcn_sched_barrier(0);  // one group's loads at a time
-          VT di = t.load(a.Di, g, t.y0 + b);
+          VT di = t.load(a.Di, g, yn + b), bf[3];
+          const VT c0 = t.load(a.cp, g, yn + b);
+#pragma unroll
+          for (int q = 1; q < 4; ++q) bf[q - 1] = t.load(a.bfp, g, yn + b + q);
           if (!t.okx || b >= t.rows) di.x = T(1);
           if (!t.oky || b >= t.rows) di.y = T(1);
           z[b] = r[b] / di;
 #pragma unroll
           for (int q = 1; q < 4; ++q)
-            z[b + q] = (r[b + q] - (-k.ky(b + q) * a.ry) * z[b + q - 1]) *
-                       t.load(a.bfp, g, t.y0 + b + q);
+            z[b + q] = (r[b + q] - (-k.ky(b + q) * a.ry) * z[b + q - 1]) * bf[q - 1];
           // back substitution; the last row of a short block has no row above
 #pragma unroll
           for (int q = 2; q >= 0; --q) {
-            const VT c = t.load(a.cp, g, t.y0 + b + q);
+            const VT c = q > 0 ? (-k.ky(b + q + 1) * a.ry) * bf[q > 0 ? q - 1 : 0] : c0;
             z[b + q] = b + q + 1 < t.rows ? z[b + q] - c * z[b + q + 1] : z[b + q];
           }
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
 #pragma unroll
@@ -235,11 +245,11 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
   }
   // the fields as the loop leaves them; w = A p of the last iteration is
   // formed again rather than held through it
-  const int col = t.col_anew();
-  apply_p([&](int j, VT wv) { t.store(a.w, g, col, t.y0 + j, wv); });
+  const int col = t.col_anew(), row = t.row_anew();
+  apply_p([&](int j, VT wv) { t.store(a.w, g, col, row + j, wv); });
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const int y = t.y0 + j;
+    const int y = row + j;
     t.store(a.u, g, col, y, u.get(j));
     t.store(a.r, g, col, y, r[j]);
     VT pj = p[j];
@@ -292,6 +302,10 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
   VT u[R], rdi[R], kx[R], ky[R + 1];
   Kept<T, R, JacobiPlan<R>::U0_LDS> u0(dyn, 0);
   T *kxr = sh.kxr[t.wave];
+  // what goes to LDS first, while there are registers to pass through
+#pragma unroll
+  for (int j = 0; j < R; ++j) u0.set(j, t.load(a.u0, g, t.y0 + j));
+  if (JacobiPlan<R>::U0_LDS) __builtin_amdgcn_sched_barrier(0);
   // the faces, which the row above and the column right of the mesh have too
 #pragma unroll
   for (int j = 0; j <= R; ++j) {
@@ -303,7 +317,6 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
     }
     if (j == R) break;
     u[j] = t.load(a.u, g, y);
-    u0.set(j, t.load(a.u0, g, y));
     kx[j] = VT(0);
     if (t.c <= g.nx && y < g.ny) {
       kx[j] = *(const VT *)t.at(a.Kx, g, t.c, y) * a.rx;
@@ -386,9 +399,9 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
     if (threadIdx.x == 0) *g.abort_flag = 1;
     return;
   }
-  const int col = t.col_anew();
+  const int col = t.col_anew(), row = t.row_anew();
 #pragma unroll
-  for (int j = 0; j < R; ++j) t.store(a.u, g, col, t.y0 + j, u[j]);
+  for (int j = 0; j < R; ++j) t.store(a.u, g, col, row + j, u[j]);
   if (lead) {
     a.ctl->stop = 1;
     a.ctl->reason = reason;
@@ -419,10 +432,25 @@ __global__ void k_res_clear(u64 *__restrict__ p, long n) {
 
 constexpr long RES_WORDS = (long)(RES_PARTS + RES_HALOS) + 16;
 
+// What a tiling costs an iteration, in us: `block` for every block, which all
+// others wait for, `row` for every row a lane holds, `memory` more where
+// preconditioner fields are read again (from `from` rows on).  Fitted to steps
+// of 400 CG iterations: 512^2 with 128, 88, 64, 44 and 32 blocks of 2, 3, 4, 6
+// and 8 rows 2.24, 2.15, 2.12, 2.39 and 2.61 ms; 640^2 with 200, 100 and 50
+// blocks of 2, 4 and 8 rows 2.66, 2.25 and 2.66; 777^2 with jac_diag and 231,
+// 154 and 119 blocks of 4, 6 and 8 rows 2.68, 2.86 and 2.92; and of 1000 Jacobi
+// iterations: 512^2 with 256, 128, 64 and 44 blocks of 1, 2, 4 and 6 rows 3.23,
+// 2.88, 2.94 and 3.43 ms.  A single block waits for none.
+struct ResCost {
+  double block, row, memory;
+  int from;
+};
+constexpr ResCost CG_COST = {0.019, 0.42, 0.0, 0}, CG_PREC_COST = {0.019, 0.42, 1.0, 6},
+                  JACOBI_COST = {0.0045, 0.17, 0.0, 0};
+
 // Rows per lane for an nx x ny mesh, of the counts in `rows` (ascending): 0
-// when no tiling has at most one block per CU.  `syncs` exchanges and `row` us
-// of arithmetic per row make an iteration.
-int res_rows(int nx, int ny, const int *rows, int nrows, int syncs = 2, double row = 0.2) {
+// when no tiling has at most one block per CU.
+int res_rows(int nx, int ny, const int *rows, int nrows, const ResCost &c) {
   const State &s = S();
   const int forced = env_int("TL_RES_ROWS", 0);
   const int cap = s.cus < RES_MAX_BLOCKS ? s.cus : RES_MAX_BLOCKS;
@@ -434,12 +462,8 @@ int res_rows(int nx, int ny, const int *rows, int nrows, int syncs = 2, double r
     const long ty = (ny + (long)RES_WAVES * R - 1) / ((long)RES_WAVES * R), nb = tx * ty;
     if (nb > cap) continue;
     if (forced == R) return R;
-    // time of an iteration in us: the exchanges, dearer with more blocks, and
-    // the arithmetic of R rows.  Measured with CG, per step: 512^2 3.04 ms with R = 1
-    // (256 blocks), 2.50 with 2, 2.43 with 4, 2.92 with 8; 250^2 (ten steps)
-    // 12.5 ms with 1, 12.2 with 2, 13.0 with 4, 16.2 with 8
-    const double sync = nb == 1 ? 0.4 : (nb <= 8 ? 1.2 : (nb <= 128 ? 1.4 : 2.1));
-    const double cost = syncs * sync + row * R;
+    const double cost = (nb > 1 ? 1.5 + c.block * nb : 0.0) + c.row * R +
+                        (c.memory > 0.0 && R >= c.from ? c.memory : 0.0);
     if (!best || cost < best_cost) {
       best = R;
       best_cost = cost;
@@ -448,14 +472,15 @@ int res_rows(int nx, int ny, const int *rows, int nrows, int syncs = 2, double r
   return best;
 }
 
-constexpr int ROWS64[] = {1, 2, 3, 4, 6, 8}, ROWS64_BLK[] = {4};
+constexpr int ROWS64[] = {1, 2, 3, 4, 6, 8}, ROWS64_BLK[] = {4, 8};
 constexpr int ROWS32[] = {1, 2, 3, 4, 6, 8, 12, 16};
 
 template <typename T>
 int rows_for(int nx, int ny, int prec) {
-  if (sizeof(T) == 4) return res_rows(nx, ny, ROWS32, 8);
-  return prec == TL_PREC_JAC_BLOCK ? res_rows(nx, ny, ROWS64_BLK, 1)
-                                   : res_rows(nx, ny, ROWS64, prec == TL_PREC_NONE ? 6 : 5);
+  if (sizeof(T) == 4) return res_rows(nx, ny, ROWS32, 8, CG_COST);
+  const ResCost &c = prec == TL_PREC_NONE ? CG_COST : CG_PREC_COST;
+  return prec == TL_PREC_JAC_BLOCK ? res_rows(nx, ny, ROWS64_BLK, 2, c)
+                                   : res_rows(nx, ny, ROWS64, 6, c);
 }
 
 constexpr int RES_REFUSED = -1;
@@ -556,7 +581,9 @@ int cg_dispatch(int R, int prec, const ResGeo &g, const ResCg<T> &a) {
     CASE(3, TL_PREC_JAC_DIAG);
     CASE(4, TL_PREC_JAC_DIAG);
     CASE(6, TL_PREC_JAC_DIAG);
+    CASE(8, TL_PREC_JAC_DIAG);
     CASE(4, TL_PREC_JAC_BLOCK);
+    CASE(8, TL_PREC_JAC_BLOCK);
   }
 #undef CASE
   return fail(TL_ERR_STATE, "solver loop: no kernel for this tiling");
@@ -609,7 +636,7 @@ int resident_jacobi(ResJacobi a, long pitch, Ctl *out) {
   if (!resident_on()) return 0;
   // with eight rows the kernel spills vector registers (see CgPlan)
   static constexpr int ROWS[] = {1, 2, 3, 4, 5, 6};
-  const int R = res_rows(s.nx, s.ny, ROWS, 6, 1, 0.2);
+  const int R = res_rows(s.nx, s.ny, ROWS, 6, JACOBI_COST);
   if (!R) return 0;
   ResGeo g = res_geo(R, pitch);
   const int n_first = a.n_first, chunk = res_chunk();

@@ -181,21 +181,36 @@ struct ResTile {
     const char *row = (const char *)f + (unsigned)y * g.pitch * (unsigned)sizeof(T);
     return (const T *)(row + (unsigned)col * (unsigned)sizeof(T));
   }
-  __device__ VT load(const T *f, const ResGeo &g, int y) const {  // 0 outside the mesh
-    VT v = VT(0);
-    if (okx && y >= 0 && y < g.ny) {
-      v = *(const VT *)at(f, g, c, y);
-      if (!oky) v.y = T(0);
-    }
-    return v;
+  // Row y of a field through a buffer descriptor whose length is the mesh's
+  // width, or 0 for a row that is none: what is read outside the mesh is zero
+  // and what is written there is dropped, in the hardware.
+  __device__ static __amdgpu_buffer_rsrc_t desc(const T *f, const ResGeo &g, int y) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)at(f, g, 0, y), 0,
+                                             y >= 0 && y < g.ny ? g.nx * (int)sizeof(T) : 0,
+                                             0x00027000);
+  }
+  __device__ VT load(const T *f, const ResGeo &g, int y) const {
+    const int off = c * (int)sizeof(T);
+    if constexpr (sizeof(T) == 8)
+      return __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b128(desc(f, g, y), off, 0, 0));
+    else
+      return __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b64(desc(f, g, y), off, 0, 0));
   }
   // column `col` is c, handed in anew after the loop so that no address of
   // the first loads is kept in registers for the stores
   __device__ void store(T *f, const ResGeo &g, int col, int y, VT v) const {
-    if (y >= g.ny) return;
-    T *q = const_cast<T *>(at(f, g, col, y));
-    if (col + 1 < g.nx) *(VT *)q = v;
-    else if (col < g.nx) *q = v.x;
+    typedef unsigned U __attribute__((ext_vector_type(sizeof(VT) / 4)));
+    const int off = col * (int)sizeof(T);
+    if constexpr (sizeof(T) == 8)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U, v), desc(f, g, y), off, 0, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U, v), desc(f, g, y), off, 0, 0);
+  }
+  // the first row, anew for the same reason (and no row's address in scalar ones)
+  __device__ int row_anew() const {
+    int y = y0;
+    asm volatile("" : "+s"(y));
+    return y;
   }
   __device__ int col_anew() const {
     int col = c;
@@ -292,6 +307,10 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
   const unsigned tag = g.epoch + s;
   const int buf = s & 1;
   const int nb = g.tx * g.ty;
+  // the tallest tiles form their addresses anew in every exchange: no registers
+  // to hold them through the loop
+  int lane = t.lane;
+  if (R * sizeof(T) >= 64) asm volatile("" : "+v"(lane));
   u64 *parts = g.part + buf * (RES_MAX_BLOCKS * RES_PART_WORDS);
   u64 *halos = g.halo + buf * (RES_MAX_BLOCKS * RES_HALO_WORDS);
   constexpr int W = res_words<T>();
@@ -300,44 +319,44 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
                 RUN_R = RUN_L + W * SIDE;
   if constexpr (HALO) {
     const VT vb = (*v)[0], vt = (*v)[R - 1];
-    sh.bottom[eb][t.wave][t.lane] = vb;
-    sh.top[eb][t.wave][t.lane] = vt;
+    sh.bottom[eb][t.wave][lane] = vb;
+    sh.top[eb][t.wave][lane] = vt;
     u64 *mine = halos + t.blk * RES_HALO_WORDS;
     if (t.wave == 0 && t.below) {
-      put_value<T>(mine, RES_COLS, RUN_B + t.lane, vb.x, tag);
-      put_value<T>(mine, RES_COLS, RUN_B + WAVE + t.lane, vb.y, tag);
+      put_value<T>(mine, RES_COLS, RUN_B + lane, vb.x, tag);
+      put_value<T>(mine, RES_COLS, RUN_B + WAVE + lane, vb.y, tag);
     }
     if (t.wave == RES_WAVES - 1 && t.above) {
-      put_value<T>(mine, RES_COLS, RUN_T + t.lane, vt.x, tag);
-      put_value<T>(mine, RES_COLS, RUN_T + WAVE + t.lane, vt.y, tag);
+      put_value<T>(mine, RES_COLS, RUN_T + lane, vt.x, tag);
+      put_value<T>(mine, RES_COLS, RUN_T + WAVE + lane, vt.y, tag);
     }
     // the wave's edge columns, moved to lanes 0..2R-1
     T *sd = sh.side[t.wave];
-    if (t.lane == 0 || t.lane == WAVE - 1) {
-      const int off = t.lane == 0 ? 0 : R;
+    if (lane == 0 || lane == WAVE - 1) {
+      const int off = lane == 0 ? 0 : R;
 #pragma unroll
-      for (int j = 0; j < R; ++j) sd[off + j] = t.lane == 0 ? (*v)[j].x : (*v)[j].y;
+      for (int j = 0; j < R; ++j) sd[off + j] = lane == 0 ? (*v)[j].x : (*v)[j].y;
     }
     __builtin_amdgcn_wave_barrier();
-    if (t.lane < 2 * R) {
-      const T e = sd[t.lane];
-      const bool lft = t.lane < R;
-      const int i = t.wave * R + (lft ? t.lane : t.lane - R);
+    if (lane < 2 * R) {
+      const T e = sd[lane];
+      const bool lft = lane < R;
+      const int i = t.wave * R + (lft ? lane : lane - R);
       if (lft ? t.left : t.right) put_value<T>(mine, SIDE, (lft ? RUN_L : RUN_R) + i, e, tag);
     }
   }
   if constexpr (SUM) {
     part = wave_total(part);
-    if (t.lane == 0) sh.red[buf][t.wave] = part;
+    if (lane == 0) sh.red[buf][t.wave] = part;
   }
   __syncthreads();
   double own = 0.0;
   if constexpr (SUM) {
 #pragma unroll
     for (int i = 0; i < RES_WAVES; ++i) own += sh.red[buf][i];
-    if (nb > 1 && t.wave == 0 && t.lane < 2) {
+    if (nb > 1 && t.wave == 0 && lane < 2) {
       const u64 b = __builtin_bit_cast(u64, own);
-      put(parts, t.blk * RES_PART_WORDS + t.lane, t.lane == 0 ? (unsigned)b : (unsigned)(b >> 32),
+      put(parts, t.blk * RES_PART_WORDS + lane, lane == 0 ? (unsigned)b : (unsigned)(b >> 32),
           tag);
     }
   }
@@ -345,9 +364,9 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
   // (waves 0 and 7 are busy with the rows), lanes 0..2R-1 of every wave one
   // ghost cell of the sides
   if constexpr (HALO) {
-    gh->dn = t.wave > 0 ? sh.top[eb][t.wave > 0 ? t.wave - 1 : 0][t.lane] : VT(0);
+    gh->dn = t.wave > 0 ? sh.top[eb][t.wave > 0 ? t.wave - 1 : 0][lane] : VT(0);
     gh->up = t.wave < RES_WAVES - 1
-                 ? sh.bottom[eb][t.wave < RES_WAVES - 1 ? t.wave + 1 : 0][t.lane]
+                 ? sh.bottom[eb][t.wave < RES_WAVES - 1 ? t.wave + 1 : 0][lane]
                  : VT(0);
     gh->side = T(0);
   }
@@ -355,18 +374,18 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
   const bool want_p = SUM && nb > 1 && from >= 0 && from < nb;
   const bool want_b = HALO && t.wave == 0 && t.below;
   const bool want_t = HALO && t.wave == RES_WAVES - 1 && t.above;
-  const bool lft = t.lane < R;
-  const bool want_s = HALO && t.lane < 2 * R && (lft ? t.left : t.right);
+  const bool lft = lane < R;
+  const bool want_s = HALO && lane < 2 * R && (lft ? t.left : t.right);
   double q = 0.0;
   if (want_p || want_b || want_t || want_s) {
     const unsigned pp = (want_p ? from : 0) * RES_PART_WORDS;
     unsigned pr = 0, ps = 0;
     if constexpr (HALO) {
-      if (want_b) pr = (t.blk - g.tx) * RES_HALO_WORDS + RUN_T + t.lane;
-      if (want_t) pr = (t.blk + g.tx) * RES_HALO_WORDS + RUN_B + t.lane;
+      if (want_b) pr = (t.blk - g.tx) * RES_HALO_WORDS + RUN_T + lane;
+      if (want_t) pr = (t.blk + g.tx) * RES_HALO_WORDS + RUN_B + lane;
       if (want_s)
         ps = (lft ? t.blk - 1 : t.blk + 1) * RES_HALO_WORDS + (lft ? RUN_R : RUN_L) + t.wave * R +
-             (lft ? t.lane : t.lane - R);
+             (lft ? lane : lane - R);
     }
     Words<double> a = {};
     Words<T> r0 = {}, r1 = {}, sw = {};
@@ -414,7 +433,7 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
       const int waves = (nb + WAVE - 1) / WAVE;  // waves 1..waves hold partials
       if (t.wave >= 1 && t.wave <= waves) {
         q = wave_total(q);
-        if (t.lane == 0) sh.tot[buf][t.wave - 1] = q;
+        if (lane == 0) sh.tot[buf][t.wave - 1] = q;
       }
       __syncthreads();
       own = 0.0;
