@@ -82,6 +82,15 @@ struct ResJacobi {
   double *herr;
 };
 int resident_jacobi(ResJacobi a, long pitch, Ctl *out);
+// The same for `count` Chebyshev iterations without a preconditioner
+// (cheby_run_deep's contract); u and p read and written in place.
+struct ResCheby {
+  double *u, *p, *w, *r;
+  const double *u0, *Kx, *Ky;
+  double rx, ry;
+};
+int resident_cheby(const ResCheby &a, const double *alphas, const double *betas, int count,
+                   long pitch, bool want_norm, double *norm);
 constexpr int RES_PAUSED = 0;  // reason of a launch that stopped for the host only
 
 bool use_nontemporal();

@@ -589,12 +589,17 @@ int cheby_run_block(const double *ch_alphas, const double *ch_betas, int step_fi
   return 1;
 }
 
-// Chebyshev iterations without a preconditioner, an even count of at most
-// DEEP_MAX per pass after a single one where `count` is odd
-// (cheby_run_fused's contract).
+// Chebyshev iterations without a preconditioner: on the chip where the mesh
+// fits, else an even count of at most DEEP_MAX per pass after a single one where
+// `count` is odd (cheby_run_fused's contract).
 int cheby_run_deep(const double *ch_alphas, const double *ch_betas, int step_first, int count,
                    int want_norm, double *norm) {
   State &s = S();
+  const ResCheby f = {s.u[s.ucur].p11, s.p[s.pcur].p11, s.w.p11, s.r.p11, s.u0.p11,
+                      s.Kx.p11,        s.Ky.p11,        s.rx,    s.ry};
+  const int ran = resident_cheby(f, ch_alphas + step_first - 1, ch_betas + step_first - 1, count,
+                                 s.pitch, want_norm, norm);
+  if (ran) return ran;
   int done = 0, nparts = 0;
   if (count & 1) {
     const Geo G = geo(2 * BLOCK);

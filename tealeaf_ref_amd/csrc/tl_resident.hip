@@ -283,12 +283,13 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
 // operations for about ten.
 //
 // What bounds it: the exchange, 2.1 us of 3.7 with 225 blocks of five rows
-// (1100x1000: a step of 1000 iterations 14.6 -> 3.8 ms against the pass kernels;
-// 512^2 5.6 -> 2.9, 100^2 3.0 -> 1.2).
+// (1100x1000: a step of 1000 iterations 14.6 -> 3.9 ms against the pass kernels;
+// 1400^2 18.3 -> 4.8, 512^2 5.6 -> 2.9, 100^2 3.0 -> 1.2).
 template <int R>
 struct JacobiPlan {
-  static constexpr bool U0_LDS = R >= 6;  // of 256 registers a field takes 4 a row
-  static constexpr size_t BYTES = U0_LDS ? (size_t)R * RES_THREADS * 2 * sizeof(double) : 0;
+  // of 256 registers a field takes 4 a row
+  static constexpr bool KY_LDS = R >= 8, U0_LDS = R >= 8;
+  static constexpr size_t BYTES = KY_LDS ? (size_t)2 * R * RES_THREADS * 2 * sizeof(double) : 0;
 };
 
 template <int R>
@@ -296,27 +297,29 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
   typedef double T;
   typedef typename dev::Vec<T, 2>::type VT;
   extern __shared__ char dyn[];
-  __shared__ ResShared<T, R, 2> sh;
+  __shared__ ResShared<T, R, 1> sh;
   if (threadIdx.x < 2) sh.dead[threadIdx.x] = 0;
   const ResTile<T, R> t(g);
-  VT u[R], rdi[R], kx[R], ky[R + 1];
-  Kept<T, R, JacobiPlan<R>::U0_LDS> u0(dyn, 0);
+  VT u[R], rdi[R], kx[R], ky_top = VT(0);
+  Kept<T, R, JacobiPlan<R>::U0_LDS> u0(dyn, 1);
+  Kept<T, R, JacobiPlan<R>::KY_LDS> ky_in(dyn, 0);
   T *kxr = sh.kxr[t.wave];
-  // what goes to LDS first, while there are registers to pass through
-#pragma unroll
-  for (int j = 0; j < R; ++j) u0.set(j, t.load(a.u0, g, t.y0 + j));
-  if (JacobiPlan<R>::U0_LDS) __builtin_amdgcn_sched_barrier(0);
   // the faces, which the row above and the column right of the mesh have too
 #pragma unroll
   for (int j = 0; j <= R; ++j) {
     const int y = t.y0 + j;
-    ky[j] = VT(0);
+    VT v = VT(0);
     if (t.okx && y <= g.ny) {
-      ky[j] = *(const VT *)t.at(a.Ky, g, t.c, y) * a.ry;
-      if (!t.oky) ky[j].y = T(0);
+      v = *(const VT *)t.at(a.Ky, g, t.c, y) * a.ry;
+      if (!t.oky) v.y = T(0);
     }
-    if (j == R) break;
-    u[j] = t.load(a.u, g, y);
+    if (j < R) ky_in.set(j < R ? j : 0, v);
+    else ky_top = v;
+  }
+  if (JacobiPlan<R>::KY_LDS) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int y = t.y0 + j;
     kx[j] = VT(0);
     if (t.c <= g.nx && y < g.ny) {
       kx[j] = *(const VT *)t.at(a.Kx, g, t.c, y) * a.rx;
@@ -325,23 +328,29 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
     if (t.lane == WAVE - 1)
       kxr[j] = (y < g.ny && t.c + 2 <= g.nx) ? *t.at(a.Kx, g, t.c + 2, y) * a.rx : T(0);
   }
+  auto ky = [&](int j) { return j < R ? ky_in.get(j < R ? j : 0) : ky_top; };
   __builtin_amdgcn_wave_barrier();
   auto right_face = [&](int j) {
     const T kr = dev::lane_above(kx[j].x), gk = kxr[j];
     return t.lane == WAVE - 1 ? gk : kr;
   };
-  auto diagonal = [&](int j, T kr) {
+  auto diagonal = [&](int j, T kr, VT kd, VT ku) {
     VT d;
-    d.x = T(1) + (kx[j].x + kx[j].y) + (ky[j].x + ky[j + 1].x);
-    d.y = T(1) + (kx[j].y + kr) + (ky[j].y + ky[j + 1].y);
+    d.x = T(1) + (kx[j].x + kx[j].y) + (kd.x + ku.x);
+    d.y = T(1) + (kx[j].y + kr) + (kd.y + ku.y);
     return d;
   };
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const VT d = diagonal(j, right_face(j));
+    const VT d = diagonal(j, right_face(j), ky(j), ky(j + 1));
     const bool in = t.y0 + j < g.ny;
     rdi[j].x = in && t.okx ? T(1) / d.x : T(0);
     rdi[j].y = in && t.oky ? T(1) / d.y : T(0);
+  }
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    u[j] = t.load(a.u, g, t.y0 + j);
+    u0.set(j, t.load(a.u0, g, t.y0 + j));
   }
   ResGhost<T> gh = load_ghosts<T, R>(t, g, a.u);
   const bool lead = t.blk == 0 && threadIdx.x == 0;
@@ -355,13 +364,13 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
     if (t.lane < 2 * R) side[t.lane] = gh.side;
     __builtin_amdgcn_wave_barrier();
     double acc = 0.0;
-    VT dn = gh.dn;
+    VT dn = gh.dn, kd = ky(0);
 #pragma unroll
     for (int j = 0; j < R; ++j) {
       const VT c = u[j];
       // taller tiles form the diagonal anew: no registers to hold it
       if (R >= 6) {
-        asm volatile("" : "+v"(kx[j].x), "+v"(ky[j].x));
+        asm volatile("" : "+v"(kx[j].x));
         __builtin_amdgcn_sched_barrier(0);
       }
       T l = dev::lane_below(c.y), r = dev::lane_above(c.x);
@@ -369,14 +378,18 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
       l = t.lane == 0 ? gl : l;
       r = t.lane == WAVE - 1 ? gr : r;
       const VT up = j + 1 < R ? u[j + 1 < R ? j + 1 : j] : gh.up;
-      VT b = u0.get(j) + ky[j] * dn + ky[j + 1] * up;
+      const VT ku = ky(j + 1);
+      VT b = u0.get(j) + kd * dn + ku * up;
       b.x = b.x + kx[j].x * l + kx[j].y * c.y;
       b.y = b.y + kx[j].y * c.x + kr * r;
       const VT q = b * rdi[j];
-      const VT rem = b - diagonal(j, kr) * q;
-      const VT v = q + rem * rdi[j];
+      const VT rem = b - diagonal(j, kr, kd, ku) * q;
+      VT v = q + rem * rdi[j];
       acc += fabs(v.x - c.x) + fabs(v.y - c.y);
+      // ... and finish a row before the next, or all rows' operands wait together
+      if (R >= 6) asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(acc));
       dn = c;
+      kd = ku;
       u[j] = v;
     }
     double sum;
@@ -384,6 +397,9 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
       dead = true;
       break;
     }
+    // with other blocks the exchange ends with a barrier, after which the waves'
+    // edge rows in LDS may be written again
+    if (g.tx * g.ty == 1) __syncthreads();
     err = sqrt(fabs(sum));
     if (lead) a.herr[n] = err;
     const bool conv = err < a.eps_abs, bad = !isfinite(err);
@@ -410,6 +426,113 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Chebyshev: iterations of tl_cheby_run, up to RES_CHEBY_STEPS in one launch
+// ---------------------------------------------------------------------------
+// An iteration (kernels/tea_leaf_cheby_kernel.f90:111-200) needs the halos of u
+// alone, so its exchange is with the neighbouring blocks only; the sum r.r is
+// formed once, at the end of a run.
+//
+// What bounds it: the exchange with the neighbours, 0.9 us of 1.4 (256^2, one row
+// a lane), and from four rows on the arithmetic.  A step of 25 CG and 975
+// Chebyshev iterations against passes of ten: 256^2 3.3 -> 2.0 ms, 512^2 3.5 ->
+// 2.2, 1024^2 4.6 -> 2.8, 1400^2 5.2 -> 4.0.
+constexpr int RES_CHEBY_STEPS = 128;  // coefficients that go along as arguments
+struct ChebyArgs {
+  ResCheby f;
+  int count;
+  bool last;               // of the run: w, r and r.r are wanted
+  double *norm;            // host memory
+  double a[RES_CHEBY_STEPS], b[RES_CHEBY_STEPS];
+};
+template <int R>
+struct ChebyPlan {
+  static constexpr bool KY_LDS = R >= 8;  // of 256 registers a field takes 4 a row
+  static constexpr size_t BYTES = KY_LDS ? (size_t)R * RES_THREADS * 2 * sizeof(double) : 0;
+};
+
+template <int R>
+__global__ __launch_bounds__(RES_THREADS) void k_res_cheby(ResGeo g, ChebyArgs a) {
+  typedef double T;
+  typedef typename dev::Vec<T, 2>::type VT;
+  extern __shared__ char dyn[];
+  __shared__ ResShared<T, R, 2> sh;
+  if (threadIdx.x < 2) sh.dead[threadIdx.x] = 0;
+  const ResTile<T, R> t(g);
+  ResFaces<T, R, ChebyPlan<R>::KY_LDS> k;
+  T *kxr = sh.kxr[t.wave], *side = sh.side[t.wave];
+  k.load(t, g, a.f.Kx, a.f.Ky, kxr, (VT *)dyn + threadIdx.x);
+  if (ChebyPlan<R>::KY_LDS) __builtin_amdgcn_sched_barrier(0);
+  VT u[R], p[R], u0[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    u[j] = t.load(a.f.u, g, t.y0 + j);
+    p[j] = t.load(a.f.p, g, t.y0 + j);
+    u0[j] = t.load(a.f.u0, g, t.y0 + j);
+  }
+  ResGhost<T> gh = load_ghosts<T, R>(t, g, a.f.u);
+  __syncthreads();
+  double acc = 0.0;
+  const int col = t.col_anew();
+  for (int n = 0;; ++n) {
+    const bool end = n + 1 == a.count, out = end && a.last;
+    const T al = a.a[n], be = a.b[n];
+    if (t.lane < 2 * R) side[t.lane] = gh.side;
+    __builtin_amdgcn_wave_barrier();
+    const int row = t.row_anew();
+    VT dn = gh.dn, kd = k.ky(0);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      if (R >= 6) __builtin_amdgcn_sched_barrier(0);
+      const VT c = u[j];
+      T l = dev::lane_below(c.y), r = dev::lane_above(c.x), kr = dev::lane_above(k.kx[j].x);
+      const T gl = side[j], gr = side[R + j], gk = kxr[j];
+      l = t.lane == 0 ? gl : l;
+      r = t.lane == WAVE - 1 ? gr : r;
+      kr = t.lane == WAVE - 1 ? gk : kr;
+      const VT up = j + 1 < R ? u[j + 1 < R ? j + 1 : j] : gh.up, ku = k.ky(j + 1);
+      VT w;
+      w.x = dev::op_cell<false>(c.x, l, c.y, dn.x, up.x, k.kx[j].x, k.kx[j].y, kd.x, ku.x, a.f.rx,
+                           a.f.ry);
+      w.y = dev::op_cell<false>(c.y, c.x, r, dn.y, up.y, k.kx[j].y, kr, kd.y, ku.y, a.f.rx, a.f.ry);
+      const VT res = u0[j] - w;
+      if (out) {
+        t.store(a.f.w, g, col, row + j, w);
+        t.store(a.f.r, g, col, row + j, res);
+        acc += res.x * res.x + res.y * res.y;
+      }
+      p[j] = al * p[j] + be * res;
+      u[j] = c + p[j];
+      dn = c;
+      kd = ku;
+    }
+    if (end) break;
+    if (!dev::res_exchange<true, false>(t, g, sh, (unsigned)n, 0.0, (double *)nullptr, &u, &gh)) {
+      if (threadIdx.x == 0) *g.abort_flag = 1;
+      return;
+    }
+  }
+  const int row = t.row_anew();
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    t.store(a.f.u, g, col, row + j, u[j]);
+    t.store(a.f.p, g, col, row + j, p[j]);
+  }
+  if (!a.last) {
+    // a wait that ran out in the last exchange: there is none after it to tell
+    __syncthreads();
+    if (threadIdx.x == 0 && (sh.dead[0] || sh.dead[1])) *g.abort_flag = 1;
+  } else {
+    double rr;
+    if (!dev::res_exchange<false, true>(t, g, sh, (unsigned)a.count, acc, &rr,
+                                        (const VT(*)[R]) nullptr, (ResGhost<T> *)nullptr)) {
+      if (threadIdx.x == 0) *g.abort_flag = 1;
+      return;
+    }
+    if (t.blk == 0 && threadIdx.x == 0) *a.norm = rr;
+  }
+}
+
 }  // namespace
 
 namespace tl {
@@ -430,7 +553,21 @@ __global__ void k_res_clear(u64 *__restrict__ p, long n) {
     p[i] = 0;
 }
 
-constexpr long RES_WORDS = (long)(RES_PARTS + RES_HALOS) + 16;
+constexpr long RES_WORDS = (long)(RES_PARTS + RES_HALOS);
+
+// What a launch tells the host, in the pinned memory of the loops' control
+// block copies (drive uses the first three): the kernel writes it there itself,
+// and the host needs to wait for the stream only.
+struct ResHost {
+  Ctl *ctl;
+  int *abort_flag;
+  double *norm;
+};
+ResHost res_host() {
+  Ctl *hc = (Ctl *)S().hctl;
+  static_assert(3 * sizeof(Ctl) + 16 <= 256, "pinned memory of the control block");
+  return {&hc[2], (int *)(hc + 3), (double *)(hc + 3) + 1};
+}
 
 // What a tiling costs an iteration, in us: `block` for every block, which all
 // others wait for, `row` for every row a lane holds, `memory` more where
@@ -440,13 +577,15 @@ constexpr long RES_WORDS = (long)(RES_PARTS + RES_HALOS) + 16;
 // blocks of 2, 4 and 8 rows 2.66, 2.25 and 2.66; 777^2 with jac_diag and 231,
 // 154 and 119 blocks of 4, 6 and 8 rows 2.68, 2.86 and 2.92; and of 1000 Jacobi
 // iterations: 512^2 with 256, 128, 64 and 44 blocks of 1, 2, 4 and 6 rows 3.23,
-// 2.88, 2.94 and 3.43 ms.  A single block waits for none.
+// 2.88, 2.94 and 3.43 ms, 1100^2 with 252 and 207 blocks of 5 and 6 rows 3.96 and
+// 4.18.  Chebyshev's blocks wait for their neighbours only: 256^2 with 1, 2, 4 and
+// 8 rows 2.03, 2.20, 2.47 and 3.65 ms.  A single block waits for none.
 struct ResCost {
   double block, row, memory;
   int from;
 };
 constexpr ResCost CG_COST = {0.019, 0.42, 0.0, 0}, CG_PREC_COST = {0.019, 0.42, 1.0, 6},
-                  JACOBI_COST = {0.0045, 0.17, 0.0, 0};
+                  JACOBI_COST = {0.0035, 0.2, 0.0, 0}, CHEBY_COST = {0.0, 0.2, 0.0, 0};
 
 // Rows per lane for an nx x ny mesh, of the counts in `rows` (ascending): 0
 // when no tiling has at most one block per CU.
@@ -517,7 +656,7 @@ ResGeo res_geo(int R, long pitch) {
   g.ty = (s.ny + RES_WAVES * R - 1) / (RES_WAVES * R);
   g.part = s.res_mem;
   g.halo = s.res_mem + RES_PARTS;
-  g.abort_flag = (int *)(s.res_mem + RES_PARTS + RES_HALOS);
+  g.abort_flag = res_host().abort_flag;
   g.limit = 2000000000LL;  // 20 s
   if (const char *e = getenv("TL_RES_LIMIT")) g.limit = atoll(e);
   return g;
@@ -536,20 +675,13 @@ int res_tags(long exchanges, unsigned *epoch) {
   return TL_OK;
 }
 
-// The control block of a finished launch, and whether a wait ran out.
-int res_result(const ResGeo &g, Ctl *dctl, Ctl *out) {
-  State &s = S();
-  Ctl *hc = (Ctl *)s.hctl;
-  int *ha = (int *)(hc + 3);
-  TL_HIP(hipMemcpyAsync(&hc[2], dctl, sizeof(Ctl), hipMemcpyDeviceToHost, s.stream));
-  TL_HIP(hipMemcpyAsync(ha, g.abort_flag, sizeof(int), hipMemcpyDeviceToHost, s.stream));
-  TL_HIP(hipStreamSynchronize(s.stream));
-  if (*ha) {
-    hipLaunchKernelGGL(k_res_clear, dim3(1), dim3(1), 0, s.stream, (u64 *)g.abort_flag, 1L);
-    return fail(TL_ERR_HIP, "solver loop: a block waited too long for the others");
-  }
-  *out = hc[2];
-  return TL_OK;
+// Wait for a launch; whether a wait of a block ran out.
+int res_wait() {
+  int *flag = res_host().abort_flag;
+  TL_HIP(hipStreamSynchronize(S().stream));
+  if (!*flag) return TL_OK;
+  *flag = 0;
+  return fail(TL_ERR_HIP, "solver loop: a block waited too long for the others");
 }
 
 // iterations of one launch: long loops come back to the host in between
@@ -611,6 +743,7 @@ int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out) {
   const int R = rows_for<T>(s.nx, s.ny, prec);
   if (!R) return 0;
   ResGeo g = res_geo(R, pitch);
+  a.ctl = res_host().ctl;
   const int n_first = a.n_first, chunk = res_chunk();
   for (;;) {
     const long left = (long)a.n_last - a.n_first + 1;
@@ -620,7 +753,8 @@ int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out) {
     if ((rc = res_tags(2 * run, &g.epoch))) return -rc;
     rc = cg_dispatch<T>(R, prec, g, a);
     if (rc == RES_REFUSED) return a.n_first == n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
-    if (rc || (rc = res_result(g, a.ctl, out))) return -rc;
+    if (rc || (rc = res_wait())) return -rc;
+    *out = *a.ctl;
     if (out->reason != RES_PAUSED) return 1;
     // p has been updated: the next launch starts as a first iteration does
     a.n_first = out->n_end + 1;
@@ -634,11 +768,11 @@ template int resident_cg<float>(ResCg<float>, int, long, Ctl *);
 int resident_jacobi(ResJacobi a, long pitch, Ctl *out) {
   State &s = S();
   if (!resident_on()) return 0;
-  // with eight rows the kernel spills vector registers (see CgPlan)
-  static constexpr int ROWS[] = {1, 2, 3, 4, 5, 6};
-  const int R = res_rows(s.nx, s.ny, ROWS, 6, JACOBI_COST);
+  static constexpr int ROWS[] = {1, 2, 3, 4, 5, 6, 8};
+  const int R = res_rows(s.nx, s.ny, ROWS, 7, JACOBI_COST);
   if (!R) return 0;
   ResGeo g = res_geo(R, pitch);
+  a.ctl = res_host().ctl;
   const int n_first = a.n_first, chunk = res_chunk();
   for (;;) {
     const long left = (long)a.n_last - a.n_first + 1;
@@ -647,14 +781,46 @@ int resident_jacobi(ResJacobi a, long pitch, Ctl *out) {
     int rc;
     if ((rc = res_tags(run, &g.epoch))) return -rc;
 #define CASE(RR) R == RR ? res_launch(&k_res_jacobi<RR>, g, a, JacobiPlan<RR>::BYTES)
-    rc = CASE(1) : CASE(2) : CASE(3) : CASE(4) : CASE(5)
-         : res_launch(&k_res_jacobi<6>, g, a, JacobiPlan<6>::BYTES);
+    rc = CASE(1) : CASE(2) : CASE(3) : CASE(4) : CASE(5) : CASE(6)
+         : res_launch(&k_res_jacobi<8>, g, a, JacobiPlan<8>::BYTES);
 #undef CASE
     if (rc == RES_REFUSED) return a.n_first == n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
-    if (rc || (rc = res_result(g, a.ctl, out))) return -rc;
+    if (rc || (rc = res_wait())) return -rc;
+    *out = *a.ctl;
     if (out->reason != RES_PAUSED) return 1;
     a.n_first = out->n_end + 1;
   }
+}
+
+int resident_cheby(const ResCheby &f, const double *alphas, const double *betas, int count,
+                   long pitch, bool want_norm, double *norm) {
+  State &s = S();
+  if (!resident_on()) return 0;
+  const int R = res_rows(s.nx, s.ny, ROWS64, 6, CHEBY_COST);
+  if (!R) return 0;
+  ResGeo g = res_geo(R, pitch);
+  ChebyArgs a;
+  a.f = f;
+  a.norm = res_host().norm;
+  int rc;
+  for (int done = 0; done < count; done += a.count) {
+    a.count = count - done < RES_CHEBY_STEPS ? count - done : RES_CHEBY_STEPS;
+    a.last = done + a.count == count;
+    memcpy(a.a, alphas + done, sizeof(double) * a.count);
+    memcpy(a.b, betas + done, sizeof(double) * a.count);
+    if ((rc = res_tags(a.count + 1, &g.epoch))) return -rc;
+#define CASE(RR) R == RR ? res_launch(&k_res_cheby<RR>, g, a, ChebyPlan<RR>::BYTES)
+    rc = CASE(1) : CASE(2) : CASE(3) : CASE(4) : CASE(6)
+         : res_launch(&k_res_cheby<8>, g, a, ChebyPlan<8>::BYTES);
+#undef CASE
+    if (rc == RES_REFUSED) return done == 0 ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
+    if (rc) return -rc;
+  }
+  if (want_norm) {
+    if ((rc = res_wait())) return -rc;
+    *norm = *a.norm;
+  }
+  return 1;
 }
 
 }  // namespace tl

@@ -277,6 +277,7 @@ extern "C" int tl_init(int nx, int ny, int halo, int device) {
   TL_HIP(hipMalloc(&s.ctl, 64));
   TL_HIP(hipMemsetAsync(s.ctl, 0, 64, s.stream));
   TL_HIP(hipHostMalloc(&s.hctl, 256, hipHostMallocDefault));
+  memset(s.hctl, 0, 256);
   // the exchange buffers of the on-chip loops: zeros, since their tags start at 1
   if ((s.res_words = resident_words(nx, ny))) {
     TL_HIP(hipMalloc((void **)&s.res_mem, sizeof(*s.res_mem) * (size_t)s.res_words));

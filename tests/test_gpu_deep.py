@@ -12,7 +12,7 @@ import pytest
 from helpers import interior
 from tealeaf_ref_amd import _lib as L
 from tealeaf_ref_amd.adjoint import chebyshev_coefs
-from test_gpu_resident import _chunk, _norm_a, _start, env
+from test_gpu_resident import SIZES as TILE_SIZES, _chunk, _norm_a, _start, env
 
 pytestmark = pytest.mark.gpu
 
@@ -138,21 +138,20 @@ def test_mixed_sweeps(inner):
         assert np.linalg.norm(us[1] - us[0]) <= 2e-10 * r0 * 1.01
 
 
-@pytest.mark.parametrize("count", [2, 3, 4, 5, 6, 8, 9, 10, 12, 17, 24, 31])
-def test_cheby_iterations(count):
-    """u, p, w and r after `count` iterations, and u's halo ring, which the
-    passes carry along unread.
+def _cheby(sizes, count, envs):
+    """u, p, w and r after `count` iterations, and u's halo ring, which no way
+    of running them changes, under two environments.
 
     Tolerance as in test_ppcg_sweeps, relative to the largest u and p; w and r
     hold u's rounding times |A|."""
     pd = C.POINTER(C.c_double)
-    for nx, ny in SIZES:
-        print(f"deep chebyshev {nx}x{ny} count {count}", flush=True)
+    for nx, ny in sizes:
+        print(f"chebyshev {nx}x{ny} count {count} {envs[1]}", flush=True)
         d, rx, ry = _chunk(nx, ny, 1, False)
         try:
             out = []
-            for deep in (0, 1):
-                with env(TL_DEEP=deep):
+            for kw in envs:
+                with env(**kw):
                     _start(d, rx, ry)
                     hi = 1.05 * _norm_a(d, rx, ry)
                     ca, cb, theta = chebyshev_coefs(hi / 100.0, hi, count + 1)
@@ -178,3 +177,16 @@ def test_cheby_iterations(count):
         ring[1:-1, 1:-1] = False
         ring[0, [0, -1]] = ring[-1, [0, -1]] = False  # corners are not carried
         assert np.array_equal(got[5][ring], ref[5][ring])
+
+
+@pytest.mark.parametrize("count", [2, 3, 4, 5, 6, 8, 9, 10, 12, 17, 24, 31])
+def test_cheby_iterations(count):
+    """Passes of many iterations against passes of one and two."""
+    _cheby(SIZES, count, ({"TL_DEEP": 0}, {"TL_RESIDENT": 0}))
+
+
+@pytest.mark.parametrize("rows,count", [(1, 2), (2, 3), (3, 10), (4, 128), (6, 129), (8, 41),
+                                        (0, 300)])
+def test_cheby_on_chip(rows, count):
+    """The whole run on the chip (128 iterations a launch) against the passes."""
+    _cheby(TILE_SIZES[1:], count, ({"TL_RESIDENT": 0}, {"TL_RES_ROWS": rows}))

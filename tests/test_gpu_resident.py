@@ -156,7 +156,7 @@ def _errors(k):
     return err[1:]
 
 
-@pytest.mark.parametrize("rows", [0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("rows", [0, 1, 2, 3, 4, 5, 6, 8])
 @pytest.mark.parametrize("reflective", [False, True])
 def test_jacobi_matches_passes(reflective, rows):
     """u after a number of Jacobi iterations, in one launch and in several.
