@@ -278,13 +278,27 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
 // one begins.  Cells outside the mesh are zero: with external faces whose
 // coefficients are zero nothing crosses them, and reflective faces, whose
 // coefficients are not, are to read zero there (as k_jl_v, ZE); what is held
-// for them is 1 / Di = 0.  The quotient by Di is the product with 1 / Di
-// corrected by its remainder, which gives the division's rounding in three
-// operations for about ten.
+// for them is 1 / Di = 0.  Every operation is rounded as the reference's, so that
+// the iterates are the reference's to the bit and an exit at a fixed point of
+// the rounding comes at its iteration: no products are fused, and the quotient
+// by Di is the product with the rounded 1 / Di, corrected by its remainder
+// (Markstein 1990), the division's own result in three operations for about ten.
 //
 // What bounds it: the exchange, 2.1 us of 3.7 with 225 blocks of five rows
 // (1100x1000: a step of 1000 iterations 14.6 -> 3.9 ms against the pass kernels;
 // 1400^2 18.3 -> 4.8, 512^2 5.6 -> 2.9, 100^2 3.0 -> 1.2).
+// tea_leaf_jacobi_kernel.f90:60-66
+__device__ inline double jacobi_num(double s0, double l, double r, double d, double u, double kxl,
+                                    double kxr, double kyd, double kyu, double rx, double ry) {
+#pragma clang fp contract(off)
+  return s0 + rx * (kxr * r + kxl * l) + ry * (kyu * u + kyd * d);
+}
+__device__ inline double jacobi_den(double kxl, double kxr, double kyd, double kyu, double rx,
+                                    double ry) {
+#pragma clang fp contract(off)
+  return 1.0 + rx * (kxl + kxr) + ry * (kyd + kyu);
+}
+
 template <int R>
 struct JacobiPlan {
   // of 256 registers a field takes 4 a row
@@ -310,7 +324,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
     const int y = t.y0 + j;
     VT v = VT(0);
     if (t.okx && y <= g.ny) {
-      v = *(const VT *)t.at(a.Ky, g, t.c, y) * a.ry;
+      v = *(const VT *)t.at(a.Ky, g, t.c, y);
       if (!t.oky) v.y = T(0);
     }
     if (j < R) ky_in.set(j < R ? j : 0, v);
@@ -322,11 +336,11 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
     const int y = t.y0 + j;
     kx[j] = VT(0);
     if (t.c <= g.nx && y < g.ny) {
-      kx[j] = *(const VT *)t.at(a.Kx, g, t.c, y) * a.rx;
+      kx[j] = *(const VT *)t.at(a.Kx, g, t.c, y);
       if (t.c == g.nx) kx[j].y = T(0);
     }
     if (t.lane == WAVE - 1)
-      kxr[j] = (y < g.ny && t.c + 2 <= g.nx) ? *t.at(a.Kx, g, t.c + 2, y) * a.rx : T(0);
+      kxr[j] = (y < g.ny && t.c + 2 <= g.nx) ? *t.at(a.Kx, g, t.c + 2, y) : T(0);
   }
   auto ky = [&](int j) { return j < R ? ky_in.get(j < R ? j : 0) : ky_top; };
   __builtin_amdgcn_wave_barrier();
@@ -336,8 +350,8 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
   };
   auto diagonal = [&](int j, T kr, VT kd, VT ku) {
     VT d;
-    d.x = T(1) + (kx[j].x + kx[j].y) + (kd.x + ku.x);
-    d.y = T(1) + (kx[j].y + kr) + (kd.y + ku.y);
+    d.x = jacobi_den(kx[j].x, kx[j].y, kd.x, ku.x, a.rx, a.ry);
+    d.y = jacobi_den(kx[j].y, kr, kd.y, ku.y, a.rx, a.ry);
     return d;
   };
 #pragma unroll
@@ -379,12 +393,14 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
       r = t.lane == WAVE - 1 ? gr : r;
       const VT up = j + 1 < R ? u[j + 1 < R ? j + 1 : j] : gh.up;
       const VT ku = ky(j + 1);
-      VT b = u0.get(j) + kd * dn + ku * up;
-      b.x = b.x + kx[j].x * l + kx[j].y * c.y;
-      b.y = b.y + kx[j].y * c.x + kr * r;
-      const VT q = b * rdi[j];
-      const VT rem = b - diagonal(j, kr, kd, ku) * q;
-      VT v = q + rem * rdi[j];
+      const VT s0 = u0.get(j);
+      VT b;
+      b.x = jacobi_num(s0.x, l, c.y, dn.x, up.x, kx[j].x, kx[j].y, kd.x, ku.x, a.rx, a.ry);
+      b.y = jacobi_num(s0.y, c.x, r, dn.y, up.y, kx[j].y, kr, kd.y, ku.y, a.rx, a.ry);
+      const VT q = b * rdi[j], di = diagonal(j, kr, kd, ku);
+      VT v;
+      v.x = fma(fma(-di.x, q.x, b.x), rdi[j].x, q.x);
+      v.y = fma(fma(-di.y, q.y, b.y), rdi[j].y, q.y);
       acc += fabs(v.x - c.x) + fabs(v.y - c.y);
       // ... and finish a row before the next, or all rows' operands wait together
       if (R >= 6) asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(acc));

@@ -156,6 +156,21 @@ def _errors(k):
     return err[1:]
 
 
+def _jacobi(u, u0, kx, ky, rx, ry, k):
+    """k iterations of tea_leaf_jacobi_kernel.f90:60-66, in its order of
+    operations, reading zero outside the mesh."""
+    c = (slice(1, -1), slice(1, -1))
+    kl, kr, kd, ku = kx[c], kx[1:-1, 2:], ky[c], ky[2:, 1:-1]
+    un = np.zeros_like(u)
+    un[c] = u[c]
+    for _ in range(k):
+        v = ((u0[c] + rx * (kr * un[1:-1, 2:] + kl * un[1:-1, :-2]) +
+              ry * (ku * un[2:, 1:-1] + kd * un[:-2, 1:-1])) /
+             (1.0 + rx * (kl + kr) + ry * (kd + ku)))
+        un[c] = v
+    return un[c]
+
+
 @pytest.mark.parametrize("rows", [0, 1, 2, 3, 4, 5, 6, 8])
 @pytest.mark.parametrize("reflective", [False, True])
 def test_jacobi_matches_passes(reflective, rows):
@@ -165,7 +180,8 @@ def test_jacobi_matches_passes(reflective, rows):
     most the largest u, and an iteration never increases the largest
     difference of two iterates (its row sums are below 1), so after k
     iterations the two differ by at most 2 * 10 k 2^-53 max|u|.  The sum of |u -
-    un| then differs by at most twice that per cell, besides its own rounding."""
+    un| then differs by at most twice that per cell, besides its own rounding.
+    The iterates on the chip are the reference's to the bit."""
     k = 37
     for nx, ny in SIZES[1:]:  # 1x1 has converged before the first iteration
         print(f"resident jacobi {nx}x{ny} refl {reflective} rows {rows}", flush=True)
@@ -176,6 +192,7 @@ def test_jacobi_matches_passes(reflective, rows):
                        {"TL_RES_ROWS": rows, "TL_RES_CHUNK": 10}):
                 with env(**kw):
                     _start(d, rx, ry)
+                    exact = [d.download(f) for f in ("u", "u0", "kx", "ky")]
                     st = L.LoopState(n_first=1, n_last=k, eps_abs=0.0)
                     assert L.lib().tl_jacobi_loop(C.byref(st)) == L.TL_OK
                     out.append((st.n_end, st.reason, _errors(k), interior(d.download("u"), 1)))
@@ -189,6 +206,7 @@ def test_jacobi_matches_passes(reflective, rows):
             assert np.max(np.abs(got[3] - ref[3])) <= tol
             assert np.max(np.abs(got[2] ** 2 - ref[2] ** 2)) <= 2 * tol * nx * ny * 1.01
         assert np.array_equal(out[1][3], out[2][3])
+        assert np.array_equal(out[1][3], _jacobi(*exact, rx, ry, k))
 
 
 def test_jacobi_exit():
