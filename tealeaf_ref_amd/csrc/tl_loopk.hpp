@@ -91,6 +91,21 @@ struct ResCheby {
 };
 int resident_cheby(const ResCheby &a, const double *alphas, const double *betas, int count,
                    long pitch, bool want_norm, double *norm);
+// The same for PPCG's outer iterations without a preconditioner and their inner
+// steps; the pointers as in run_ppcg_loop, r_store written only.
+template <typename T>
+struct ResPpcg {
+  T *u, *r, *r_store, *p, *z;
+  const T *pin;
+  const T *Kx, *Ky;
+  T rx, ry, theta_r;
+  int n_first, n_last, n_pause, inner;
+  double eps_abs, rro;
+  Ctl *ctl;
+  double *herr;
+};
+template <typename T>
+int resident_ppcg(ResPpcg<T> a, const double *alphas, const double *betas, long pitch, Ctl *out);
 constexpr int RES_PAUSED = 0;  // reason of a launch that stopped for the host only
 
 bool use_nontemporal();
@@ -1390,6 +1405,24 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   lp.check_switch = 0;
   lp.presteps = 0;
   const T theta_r = (T)(1.0 / theta);
+  Ctl res;
+  if (!b.diag && !b.block && deep_fits()) {
+    const ResPpcg<T> a = {b.u,   b.r,  b.r_store, b.p[c0], b.z,         pin_first ? pin_first : b.p[c0],
+                          b.Kx,  b.Ky, b.rx,      b.ry,    theta_r,     st->n_first,
+                          st->n_last, 0, inner, st->eps_abs, rro_first, m.ctl, m.herr};
+    const int ran = resident_ppcg<T>(a, alphas, betas, G.pitch, &res);
+    if (ran < 0) return -ran;
+    if (ran) {
+      st->n_end = res.n_end;
+      st->reason = res.reason;
+      st->error = res.error;
+      st->rro = res.rro;
+      st->old_error = res.old_error;
+      if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("PPCG", res.n_end);
+      if (inner_iters) *inner_iters += (res.n_end - st->n_first + 1) * inner;
+      return TL_OK;
+    }
+  }
   // Row directions: the w pass walks d, the update -d, the sweep passes
   // alternate from d; with an odd number of sweep passes the next outer
   // iteration flips d, so every pass starts on the rows written last.  The deep
@@ -1462,7 +1495,6 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
     TL_HIP(hipGetLastError());
     return TL_OK;
   };
-  Ctl res;
   if ((rc = drive(st->n_first, st->n_last, launch, tail, &res, m.ctl))) return rc;
   st->n_end = res.n_end;
   st->reason = res.reason;

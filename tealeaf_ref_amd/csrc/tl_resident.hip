@@ -549,6 +549,209 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cheby(ResGeo g, ChebyArgs a
   }
 }
 
+// ---------------------------------------------------------------------------
+// PPCG: outer iterations of run_ppcg_loop with their inner steps in one launch
+// ---------------------------------------------------------------------------
+// The inner steps work on z and z one step before, as k_deep_ppcg's do, and
+// need z's halos alone; two sums end an outer iteration (z.r and (r -
+// r_store).z) and one its first half.
+//
+// What bounds it: with ten inner steps the exchanges, ten of 0.9 us and two of 1.4
+// to 2.1, and from four rows a lane on the arithmetic.  Whole steps against the
+// passes: 256^2 1.48 -> 0.88 ms, 512^2 2.27 -> 1.38, 1024^2 5.4 -> 2.8; FP32 inside the
+// refined solver 256^2 2.4 -> 1.2, 1024^2 6.5 -> 3.1.
+constexpr int RES_PPCG_STEPS = 64;  // inner steps whose coefficients go along as arguments
+template <typename T>
+struct PpcgArgs {
+  ResPpcg<T> f;
+  T a[RES_PPCG_STEPS], b[RES_PPCG_STEPS];
+};
+template <typename T, int R>
+struct PpcgPlan {
+  static constexpr int SIZE = (int)sizeof(T) / 4 * 2 * R;  // registers of one field
+  // u, p and r_store are idle during the inner steps: in LDS, of which the
+  // tallest tiles have no more than u and p fill
+  static constexpr bool LDS = SIZE >= 16, RS_MEMORY = SIZE >= 24;
+  static constexpr size_t BYTES =
+      LDS ? (size_t)(RS_MEMORY ? 2 : 3) * R * RES_THREADS * 2 * sizeof(T) : 0;
+  static_assert(BYTES + sizeof(ResShared<T, R, 2>) <= 160 * 1024, "LDS of a CU");
+};
+
+template <typename T, int R>
+__global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> args) {
+  typedef typename dev::Vec<T, 2>::type VT;
+  constexpr bool LDS = PpcgPlan<T, R>::LDS, RS_MEMORY = PpcgPlan<T, R>::RS_MEMORY;
+  const ResPpcg<T> &a = args.f;
+  extern __shared__ char dyn[];
+  __shared__ ResShared<T, R, 2> sh;
+  if (threadIdx.x < 2) sh.dead[threadIdx.x] = 0;
+  const ResTile<T, R> t(g);
+  ResFaces<T, R, false> k;
+  T *kxr = sh.kxr[t.wave], *side = sh.side[t.wave];
+  Kept<T, R, LDS> u(dyn, 0), p(dyn, 1);
+  Kept<T, RS_MEMORY ? 1 : R, LDS && !RS_MEMORY> rs(dyn, 2);
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    u.set(j, t.load(a.u, g, t.y0 + j));
+    p.set(j, t.load(a.pin, g, t.y0 + j));
+  }
+  if (LDS) __builtin_amdgcn_sched_barrier(0);
+  k.load(t, g, a.Kx, a.Ky, kxr, (VT *)nullptr);
+  VT r[R], z[R], zp[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    r[j] = t.load(a.r, g, t.y0 + j);
+    z[j] = zp[j] = VT(0);
+  }
+  ResGhost<T> pg = load_ghosts<T, R>(t, g, a.pin), gh;
+  const bool lead = t.blk == 0 && threadIdx.x == 0;
+  double rro = a.rro, err = 0.0, sums[2] = {0.0, 0.0};
+  int reason = 0, n_end = 0;
+  bool dead = false, update = false;
+  T be = T(0);
+  unsigned s = 0;
+  __syncthreads();
+  for (int n = a.n_first;; ++n) {
+    // ---- w = A p (in z), p.w
+    double acc = 0.0;
+    {
+      VT v[R];
+#pragma unroll
+      for (int j = 0; j < R; ++j) v[j] = p.get(j);
+      if (t.lane < 2 * R) side[t.lane] = pg.side;
+      __builtin_amdgcn_wave_barrier();
+      dev::res_apply<diff_form<T>()>(t, k, v, pg.dn, pg.up, side, kxr, a.rx, a.ry,
+                                     [&](int j, VT w) {
+        z[j] = w;
+        acc += (double)w.x * (double)v[j].x;
+        acc += (double)w.y * (double)v[j].y;
+      });
+    }
+    double pw;
+    if (!dev::res_exchange<false, 1>(t, g, sh, s++, acc, &pw, (const VT(*)[R]) nullptr,
+                                     (ResGhost<T> *)nullptr)) {
+      dead = true;
+      break;
+    }
+    if (!isfinite(pw) || !isfinite(rro)) {
+      reason = TL_LOOP_NONFINITE;
+      n_end = n;
+      err = isfinite(pw) ? rro : pw;
+      break;
+    }
+    const T al = (T)(rro / pw);
+    const int row = t.row_anew();
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      u.set(j, u.get(j) + al * p.get(j));
+      if constexpr (RS_MEMORY) t.store(a.r_store, g, t.c, row + j, r[j]);
+      else rs.set(j, r[j]);
+      r[j] = r[j] - al * z[j];
+      z[j] = r[j] * a.theta_r;
+      zp[j] = VT(0);
+    }
+    // ---- the inner steps
+    for (int i = 0; i < a.inner; ++i) {
+      if (!dev::res_exchange<true, 0>(t, g, sh, s++, 0.0, (double *)nullptr, &z, &gh)) {
+        dead = true;
+        break;
+      }
+      const T ca = args.a[i], cb = args.b[i];
+      if (t.lane < 2 * R) side[t.lane] = gh.side;
+      __builtin_amdgcn_wave_barrier();
+      VT dn = gh.dn, kd = k.ky(0);
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        if (R * sizeof(T) >= 48) __builtin_amdgcn_sched_barrier(0);
+        const VT c = z[j];
+        T l = dev::lane_below(c.y), rt = dev::lane_above(c.x), kr = dev::lane_above(k.kx[j].x);
+        const T gl = side[j], gr = side[R + j], gk = kxr[j];
+        l = t.lane == 0 ? gl : l;
+        rt = t.lane == WAVE - 1 ? gr : rt;
+        kr = t.lane == WAVE - 1 ? gk : kr;
+        const VT up = j + 1 < R ? z[j + 1 < R ? j + 1 : j] : gh.up, ku = k.ky(j + 1);
+        VT w;
+        w.x = dev::op_cell<diff_form<T>()>(c.x, l, c.y, dn.x, up.x, k.kx[j].x, k.kx[j].y, kd.x,
+                                           ku.x, a.rx, a.ry);
+        w.y = dev::op_cell<diff_form<T>()>(c.y, c.x, rt, dn.y, up.y, k.kx[j].y, kr, kd.y, ku.y,
+                                           a.rx, a.ry);
+        VT zn = c + ca * (c - zp[j]) + cb * (r[j] - w);
+        // a row is finished before the next, or all rows' operands wait together
+        if (R * sizeof(T) >= 48) asm volatile("" : "+v"(zn.x), "+v"(zn.y));
+        zp[j] = c;
+        z[j] = zn;
+        dn = c;
+        kd = ku;
+      }
+    }
+    if (dead) break;
+    double a0 = 0.0, a1 = 0.0;
+    const int back = t.row_anew();
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      VT ro;
+      if constexpr (RS_MEMORY) ro = t.load(a.r_store, g, back + j);
+      else ro = rs.get(j);
+      a0 += ((double)r[j].x - (double)ro.x) * (double)z[j].x;
+      a0 += ((double)r[j].y - (double)ro.y) * (double)z[j].y;
+      a1 += (double)z[j].x * (double)r[j].x;
+      a1 += (double)z[j].y * (double)r[j].y;
+    }
+    if (!dev::res_exchange<true, 2>(t, g, sh, s++, a0, sums, &z, &gh, a1)) {
+      dead = true;
+      break;
+    }
+    // ---- head of iteration n + 1 (loop_head)
+    const double rrn = sums[0], beta = rrn / rro;
+    err = sqrt(fabs(rrn));
+    const bool bad = !isfinite(rrn), conv = !bad && fabs(err) < a.eps_abs;
+    const bool tail = n == a.n_last, pause = n == a.n_pause;
+    if (lead) a.herr[n] = err;
+    be = (T)beta;
+    if (bad || conv || tail || pause) {
+      reason = bad    ? TL_LOOP_NONFINITE
+               : conv ? TL_LOOP_CONVERGED
+               : tail ? TL_LOOP_MAXITERS
+                      : RES_PAUSED;
+      n_end = n;
+      update = true;
+      break;
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) p.set(j, z[j] + be * p.get(j));
+    pg.dn = gh.dn + be * pg.dn;
+    pg.up = gh.up + be * pg.up;
+    pg.side = gh.side + be * pg.side;
+    rro = sums[1];
+  }
+  if (dead) {
+    if (threadIdx.x == 0) *g.abort_flag = 1;
+    return;
+  }
+  const int col = t.col_anew(), row = t.row_anew();
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int y = row + j;
+    t.store(a.u, g, col, y, u.get(j));
+    t.store(a.r, g, col, y, r[j]);
+    VT pj = p.get(j);
+    if (update) {
+      pj = z[j] + be * pj;
+      t.store(a.z, g, col, y, z[j]);
+      if constexpr (!RS_MEMORY) t.store(a.r_store, g, col, y, rs.get(j));
+    }
+    t.store(a.p, g, col, y, pj);
+  }
+  if (lead) {
+    a.ctl->stop = 1;
+    a.ctl->reason = reason;
+    a.ctl->n_end = n_end;
+    a.ctl->error = err;
+    a.ctl->old_error = sums[1];
+    a.ctl->rro = sums[0];
+  }
+}
+
 }  // namespace
 
 namespace tl {
@@ -595,7 +798,8 @@ ResHost res_host() {
 // iterations: 512^2 with 256, 128, 64 and 44 blocks of 1, 2, 4 and 6 rows 3.23,
 // 2.88, 2.94 and 3.43 ms, 1100^2 with 252 and 207 blocks of 5 and 6 rows 3.96 and
 // 4.18.  Chebyshev's blocks wait for their neighbours only: 256^2 with 1, 2, 4 and
-// 8 rows 2.03, 2.20, 2.47 and 3.65 ms.  A single block waits for none.
+// 8 rows 2.03, 2.20, 2.47 and 3.65 ms.  A single block waits for none, and up to 8,
+// one on each XCD, wait 0.2 us less in an exchange (1.2 for 1.4 us).
 struct ResCost {
   double block, row, memory;
   int from;
@@ -617,7 +821,8 @@ int res_rows(int nx, int ny, const int *rows, int nrows, const ResCost &c) {
     const long ty = (ny + (long)RES_WAVES * R - 1) / ((long)RES_WAVES * R), nb = tx * ty;
     if (nb > cap) continue;
     if (forced == R) return R;
-    const double cost = (nb > 1 ? 1.5 + c.block * nb : 0.0) + c.row * R +
+    const double wait = nb == 1 ? 0.0 : (nb <= NUM_XCD ? 1.1 : 1.5);
+    const double cost = wait + c.block * nb + c.row * R +
                         (c.memory > 0.0 && R >= c.from ? c.memory : 0.0);
     if (!best || cost < best_cost) {
       best = R;
@@ -838,5 +1043,55 @@ int resident_cheby(const ResCheby &f, const double *alphas, const double *betas,
   }
   return 1;
 }
+
+template <typename T>
+int resident_ppcg(ResPpcg<T> f, const double *alphas, const double *betas, long pitch, Ctl *out) {
+  State &s = S();
+  if (!resident_on() || f.inner < 1 || f.inner > RES_PPCG_STEPS) return 0;
+  static constexpr int R64[] = {1, 2, 3, 4, 6}, R32[] = {1, 2, 3, 4, 6, 8, 12};
+  const ResCost cost = {0.019, 0.2 * (f.inner + 2), 0.0, 0};
+  const int R = sizeof(T) == 8 ? res_rows(s.nx, s.ny, R64, 5, cost)
+                               : res_rows(s.nx, s.ny, R32, 7, cost);
+  if (!R) return 0;
+  ResGeo g = res_geo(R, pitch);
+  PpcgArgs<T> a;
+  a.f = f;
+  a.f.ctl = res_host().ctl;
+  for (int i = 0; i < RES_PPCG_STEPS; ++i) {
+    a.a[i] = i < f.inner ? (T)alphas[i] : T(0);
+    a.b[i] = i < f.inner ? (T)betas[i] : T(0);
+  }
+  const int chunk = res_chunk();
+  for (;;) {
+    const long left = (long)f.n_last - a.f.n_first + 1;
+    const long run = left < chunk ? left : chunk;
+    a.f.n_pause = (int)(a.f.n_first + run - 1);
+    int rc;
+    if ((rc = res_tags((f.inner + 2L) * run, &g.epoch))) return -rc;
+#define CASE(RR) R == RR ? res_launch(&k_res_ppcg<T, RR>, g, a, PpcgPlan<T, RR>::BYTES)
+    if constexpr (sizeof(T) == 8)
+      rc = CASE(1) : CASE(2) : CASE(3) : CASE(4)
+           : res_launch(&k_res_ppcg<T, 6>, g, a, PpcgPlan<T, 6>::BYTES);
+    else
+      rc = CASE(1) : CASE(2) : CASE(3) : CASE(4) : CASE(6) : CASE(8)
+           : res_launch(&k_res_ppcg<T, 12>, g, a, PpcgPlan<T, 12>::BYTES);
+#undef CASE
+    if (rc == RES_REFUSED)
+      return a.f.n_first == f.n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
+    if (rc || (rc = res_wait())) return -rc;
+    *out = *a.f.ctl;
+    // the sum z.r enters the next iteration; the control block has no other
+    // place for it
+    const double zr = out->old_error;
+    out->old_error = out->error;
+    if (out->reason != RES_PAUSED) return 1;
+    // p has been updated: the next launch starts as a first iteration does
+    a.f.n_first = out->n_end + 1;
+    a.f.rro = zr;
+    a.f.pin = a.f.p;
+  }
+}
+template int resident_ppcg<double>(ResPpcg<double>, const double *, const double *, long, Ctl *);
+template int resident_ppcg<float>(ResPpcg<float>, const double *, const double *, long, Ctl *);
 
 }  // namespace tl

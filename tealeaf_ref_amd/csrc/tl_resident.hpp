@@ -141,7 +141,7 @@ __device__ inline T value_of(const Words<T> &o) {
 template <typename T, int R, int EB>
 struct ResShared {
   typedef typename Vec<T, 2>::type VT;
-  double red[2][RES_WAVES], tot[2][RES_WAVES];
+  double red[2][2][RES_WAVES], tot[2][2][RES_WAVES];  // [parity][sum][wave]
   int dead[2];                       // a wait of this block has run out
   VT bottom[EB][RES_WAVES][WAVE], top[EB][RES_WAVES][WAVE];  // edge rows of every wave
   T side[RES_WAVES][2 * R];          // ghost columns: left rows, then right rows
@@ -293,14 +293,15 @@ struct ResGhost {
 
 // Exchange number s of the loop (tag epoch + s, buffer s & 1).  HALO: the
 // edges of `v` go to the neighbours and their edges come back in `gh`.  SUM:
-// returns the sum of `part` over the lanes of all blocks, added in one fixed
-// order everywhere, so every block has the same bits.  Returns false in
+// returns one or two sums of `part` (and `part2`) over the lanes of all blocks,
+// added in one fixed order everywhere, so every block has the same bits.  Returns false in
 // every wave of a block when a wait of the block has run out (in a wave that
 // waits for halos alone, one exchange later).
-template <bool HALO, bool SUM, typename T, int R, int EB>
+template <bool HALO, int SUM, typename T, int R, int EB>
 __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
                                     ResShared<T, R, EB> &sh, unsigned s, double part, double *total,
-                                    const typename Vec<T, 2>::type (*v)[R], ResGhost<T> *gh) {
+                                    const typename Vec<T, 2>::type (*v)[R], ResGhost<T> *gh,
+                                    double part2 = 0.0) {
   typedef typename Vec<T, 2>::type VT;
   const int eb = EB > 1 ? s & 1 : 0;
   constexpr int SIDE = RES_WAVES * R;        // values of one side
@@ -345,19 +346,24 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
       if (lft ? t.left : t.right) put_value<T>(mine, SIDE, (lft ? RUN_L : RUN_R) + i, e, tag);
     }
   }
-  if constexpr (SUM) {
+  if constexpr (SUM > 0) {
     part = wave_total(part);
-    if (lane == 0) sh.red[buf][t.wave] = part;
+    if (SUM > 1) part2 = wave_total(part2);
+    if (lane == 0) {
+      sh.red[buf][0][t.wave] = part;
+      if (SUM > 1) sh.red[buf][1][t.wave] = part2;
+    }
   }
   __syncthreads();
-  double own = 0.0;
-  if constexpr (SUM) {
+  double own[2] = {0.0, 0.0};
+  if constexpr (SUM > 0) {
 #pragma unroll
-    for (int i = 0; i < RES_WAVES; ++i) own += sh.red[buf][i];
-    if (nb > 1 && t.wave == 0 && lane < 2) {
-      const u64 b = __builtin_bit_cast(u64, own);
-      put(parts, t.blk * RES_PART_WORDS + lane, lane == 0 ? (unsigned)b : (unsigned)(b >> 32),
-          tag);
+    for (int m = 0; m < SUM; ++m)
+#pragma unroll
+      for (int i = 0; i < RES_WAVES; ++i) own[m] += sh.red[buf][m][i];
+    if (nb > 1 && t.wave == 0 && lane < 2 * SUM) {
+      const u64 b = __builtin_bit_cast(u64, SUM > 1 && lane >= 2 ? own[1] : own[0]);
+      put(parts, t.blk * RES_PART_WORDS + lane, lane & 1 ? (unsigned)(b >> 32) : (unsigned)b, tag);
     }
   }
   // ---- wait for the others: lanes of waves 1.. take one block's partial each
@@ -371,12 +377,12 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
     gh->side = T(0);
   }
   const int from = (int)threadIdx.x - WAVE;  // the block this lane takes a partial of
-  const bool want_p = SUM && nb > 1 && from >= 0 && from < nb;
+  const bool want_p = SUM > 0 && nb > 1 && from >= 0 && from < nb;
   const bool want_b = HALO && t.wave == 0 && t.below;
   const bool want_t = HALO && t.wave == RES_WAVES - 1 && t.above;
   const bool lft = lane < R;
   const bool want_s = HALO && lane < 2 * R && (lft ? t.left : t.right);
-  double q = 0.0;
+  double q[2] = {0.0, 0.0};
   if (want_p || want_b || want_t || want_s) {
     const unsigned pp = (want_p ? from : 0) * RES_PART_WORDS;
     unsigned pr = 0, ps = 0;
@@ -387,15 +393,17 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
         ps = (lft ? t.blk - 1 : t.blk + 1) * RES_HALO_WORDS + (lft ? RUN_R : RUN_L) + t.wave * R +
              (lft ? lane : lane - R);
     }
-    Words<double> a = {};
+    Words<double> a[2] = {};
     Words<T> r0 = {}, r1 = {}, sw = {};
     int spins = 0;
     long long t_start = 0;
     for (;;) {
-      if (want_p) {
-        a.w[0] = get(parts, pp);
-        a.w[1] = get(parts, pp + 1);
-      }
+      if (want_p)
+#pragma unroll
+        for (int m = 0; m < SUM; ++m) {
+          a[m].w[0] = get(parts, pp + 2 * m);
+          a[m].w[1] = get(parts, pp + 2 * m + 1);
+        }
       if constexpr (HALO) {
         if (want_b || want_t) {
           r0 = get_words<T>(halos, RES_COLS, pr);
@@ -403,7 +411,7 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
         }
         if (want_s) sw = get_words<T>(halos, SIDE, ps);
       }
-      bool ok = !want_p || tagged<double>(a, tag);
+      bool ok = !want_p || (tagged<double>(a[0], tag) && (SUM < 2 || tagged<double>(a[1], tag)));
       if constexpr (HALO) {
         if (want_b || want_t) ok = ok && tagged<T>(r0, tag) && tagged<T>(r1, tag);
         if (want_s) ok = ok && tagged<T>(sw, tag);
@@ -418,7 +426,9 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
         }
       }
     }
-    if (want_p) q = value_of<double>(a);
+    if (want_p)
+#pragma unroll
+      for (int m = 0; m < SUM; ++m) q[m] = value_of<double>(a[m]);
     if constexpr (HALO) {
       VT row;
       row.x = value_of<T>(r0);
@@ -428,19 +438,25 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
       if (want_s) gh->side = value_of<T>(sw);
     }
   }
-  if constexpr (SUM) {
+  if constexpr (SUM > 0) {
     if (nb > 1) {
       const int waves = (nb + WAVE - 1) / WAVE;  // waves 1..waves hold partials
-      if (t.wave >= 1 && t.wave <= waves) {
-        q = wave_total(q);
-        if (lane == 0) sh.tot[buf][t.wave - 1] = q;
-      }
+      if (t.wave >= 1 && t.wave <= waves)
+#pragma unroll
+        for (int m = 0; m < SUM; ++m) {
+          q[m] = wave_total(q[m]);
+          if (lane == 0) sh.tot[buf][m][t.wave - 1] = q[m];
+        }
       __syncthreads();
-      own = 0.0;
-      for (int i = 0; i < waves; ++i) own += sh.tot[buf][i];
-      if (sh.dead[buf]) return false;
+#pragma unroll
+      for (int m = 0; m < SUM; ++m) {
+        own[m] = 0.0;
+        for (int i = 0; i < waves; ++i) own[m] += sh.tot[buf][m][i];
+      }
+      if (sh.dead[0] || sh.dead[1]) return false;  // this one, or one for halos alone before
     }
-    *total = own;
+#pragma unroll
+    for (int m = 0; m < SUM; ++m) total[m] = own[m];
     return true;
   }
   // no second barrier: what the exchange before found is settled

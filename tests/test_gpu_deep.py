@@ -19,24 +19,24 @@ pytestmark = pytest.mark.gpu
 SIZES = [(3, 2), (7, 31), (107, 9), (109, 64), (217, 45), (250, 37), (501, 133), (130, 400)]
 
 
-@pytest.mark.parametrize("inner", [4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 16, 21, 30])
-@pytest.mark.parametrize("reflective", [False, True])
-def test_ppcg_sweeps(inner, reflective):
+def _ppcg_sweeps(sizes, inner, reflective, envs):
     """z after one outer iteration, i.e. the Chebyshev polynomial of r.
 
     Tolerance: with bounds that hold the spectrum the recurrence is stable, so
     a sweep's rounding (row sums of about 10 operations on terms of up to
     |A| |sd|, which is about 2 |r|) reaches z divided by theta = |A|/2 and is
     not amplified by more than the condition of the bounds used here, at most
-    100.  That is 10 * 100 roundings per sweep relative to the largest z."""
+    100.  That is 10 * 100 roundings per sweep relative to the largest z; and to
+    the largest that enters, since alpha, whose sums are added in another order,
+    is rounded there (many sweeps leave a z that is smaller by orders)."""
     pd = C.POINTER(C.c_double)
-    for nx, ny in SIZES:
-        print(f"deep ppcg {nx}x{ny} inner {inner} reflective {reflective}", flush=True)
+    for nx, ny in sizes:
+        print(f"ppcg {nx}x{ny} inner {inner} reflective {reflective} {envs[1]}", flush=True)
         d, rx, ry = _chunk(nx, ny, 1, reflective)
         try:
             out = []
-            for deep in (0, 1):
-                with env(TL_DEEP=deep):
+            for kw in envs:
+                with env(**kw):
                     r0 = _start(d, rx, ry)
                     hi = 1.05 * _norm_a(d, rx, ry)
                     ca, cb, theta = chebyshev_coefs(hi / 100.0, hi, inner)
@@ -48,6 +48,7 @@ def test_ppcg_sweeps(inner, reflective):
                     d.update_halo([0, 0, 0, 0, 0, 1, 1] + [0] * 4, 1)
                     L.call("tl_ppcg_inner", ca.ctypes.data_as(pd), cb.ctypes.data_as(pd), 1, inner)
                     L.call("tl_ppcg_update_z")
+                    z0 = float(np.max(np.abs(interior(d.download("z"), 1))))
                     rro = d.scalar("tl_ppcg_init", 3)
                     st = L.LoopState(n_first=2, n_last=2, eps_abs=0.0, rro=rro, old_error=r0)
                     n = C.c_int(0)
@@ -62,15 +63,32 @@ def test_ppcg_sweeps(inner, reflective):
         assert got[:3] == ref[:3] == (L.TL_OK, 2, inner)
         tol = 1000.0 * inner * 2.0 ** -53
         for i in (4, 5):
-            scale = float(np.max(np.abs(ref[i])))
+            scale = max(z0, float(np.max(np.abs(ref[i]))))
             assert np.max(np.abs(got[i] - ref[i])) <= tol * scale, (nx, ny, i)
+
+
+@pytest.mark.parametrize("inner", [4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 16, 21, 30])
+@pytest.mark.parametrize("reflective", [False, True])
+def test_ppcg_sweeps(inner, reflective):
+    """Passes of many sweeps against passes of one and two."""
+    _ppcg_sweeps(SIZES, inner, reflective, ({"TL_DEEP": 0}, {"TL_RESIDENT": 0}))
+
+
+@pytest.mark.parametrize("rows,inner", [(1, 10), (2, 1), (3, 2), (4, 10), (6, 7), (0, 64)])
+@pytest.mark.parametrize("reflective", [False, True])
+def test_ppcg_on_chip(rows, inner, reflective):
+    """The outer iterations on the chip against the passes of one and two sweeps."""
+    _ppcg_sweeps(TILE_SIZES[1:], inner, reflective, ({"TL_DEEP": 0}, {"TL_RES_ROWS": rows}))
 
 
 @pytest.mark.parametrize("inner", [7, 10, 14])
 @pytest.mark.parametrize("outers", [1, 2, 3, 4, 5, 8])
-def test_ppcg_outer_iterations(inner, outers):
+@pytest.mark.parametrize("way", [{"TL_RESIDENT": 0}, {"TL_RESIDENT": 1},
+                                 {"TL_RES_ROWS": 2, "TL_RES_CHUNK": 2}])
+def test_ppcg_outer_iterations(inner, outers, way):
     """Fields after 1 to 8 outer iterations, in which r and r_store change
-    places every time, and the directions and u's updates go round 3 or 4.
+    places every time, and the directions and u's updates go round 3 or 4; and
+    on the chip, in one launch and in several.
 
     Tolerance: an outer iteration's rounding (test_ppcg_sweeps, through z) is
     carried on by CG's recurrences; 100 times the sum over the iterations, the
@@ -82,8 +100,8 @@ def test_ppcg_outer_iterations(inner, outers):
         d, rx, ry = _chunk(nx, ny, 1, False)
         try:
             out = []
-            for deep in (0, 1):
-                with env(TL_DEEP=deep):
+            for kw in ({"TL_DEEP": 0}, way):
+                with env(**kw):
                     r0 = _start(d, rx, ry)
                     scale = {"r": float(np.max(np.abs(interior(d.download("r"), 1)))),
                              "u": float(np.max(np.abs(interior(d.download("u"), 1))))}
@@ -117,8 +135,9 @@ def test_ppcg_outer_iterations(inner, outers):
 
 
 @pytest.mark.parametrize("inner", [4, 7, 10, 13, 20])
-def test_mixed_sweeps(inner):
-    """The FP32 passes inside the refined solver: both ways reach the true
+@pytest.mark.parametrize("rows", [None, 1, 4, 8, 12])
+def test_mixed_sweeps(inner, rows):
+    """The FP32 passes (rows None) and the on-chip loop inside the refined solver: all reach the true
     residual asked for, and |u - x| <= |u0 - A u| (the smallest eigenvalue of A
     is 1) bounds how far apart the two solutions may be."""
     for nx, ny in ((7, 31), (231, 40), (233, 64), (500, 133)):
@@ -126,8 +145,9 @@ def test_mixed_sweeps(inner):
         d, rx, ry = _chunk(nx, ny, 1, False)
         try:
             us = []
-            for deep in (0, 1):
-                with env(TL_DEEP=deep):
+            for kw in ({"TL_DEEP": 0},
+                       {"TL_RESIDENT": 0} if rows is None else {"TL_RES_ROWS": rows}):
+                with env(**kw):
                     r0 = math.sqrt(_start(d, rx, ry))
                     st = d.mixed_solve(solver=L.MIXED_PPCG, rel_tol=1e-10, inner_steps=inner,
                                        presteps=20)
