@@ -56,8 +56,9 @@ dev::Geo geo_resident(int cols_per_tile, int blocks_per_cu) {
   g.rows_per_tile = (int)r;
   g.tiles_y = (s.ny + g.rows_per_tile - 1) / g.rows_per_tile;
   g.tiles = (long)g.tiles_x * g.tiles_y;
-  long b = g.tiles < MAX_GRID ? g.tiles : MAX_GRID;
-  if (b >= NUM_XCD) b -= b % NUM_XCD;
+  long b = (g.tiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
+  if (g.tiles < NUM_XCD) b = g.tiles;
+  if (b > MAX_GRID) b = MAX_GRID;
   dev::Geo G;
   G.nx = s.nx;
   G.ny = s.ny;
