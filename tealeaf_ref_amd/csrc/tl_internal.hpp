@@ -22,6 +22,7 @@ namespace tl {
 constexpr int PADL = 32;          // doubles before interior column 1 (256 B)
 constexpr int BLOCK = 256;        // threads per block for streaming kernels
 constexpr int WAVE = 64;          // CDNA wavefront width
+constexpr int HSCAL = 64, HHIST = 1024;
 constexpr int MAX_GRID = 2048;    // max blocks of a reduction kernel (= partials)
 constexpr int NUM_XCD = 8;        // MI355X: 8 XCDs, blocks dealt round robin
 
@@ -66,8 +67,9 @@ struct State {
 
   // reductions: partial sums per block, and small device scalars
   double *partials = nullptr;  // NPART arrays of MAX_GRID doubles
-  double *dscal = nullptr;     // scratch scalars (results of finish kernels)
-  double *hscal = nullptr;     // pinned host mirror of dscal
+  // pinned host memory that kernels write: HSCAL scalars (results of finish
+  // kernels), then alpha and beta of a CG loop's first HHIST iterations
+  double *hscal = nullptr;
   void *ctl = nullptr;         // loop control block (device)
   void *hctl = nullptr;        // pinned host copies of the control block
   hipEvent_t loop_ev[2] = {nullptr, nullptr};  // batch markers of the loop driver
@@ -171,7 +173,7 @@ inline void klaunch(void (*k)(F...), dim3 grid, dim3 block, A... args) {
 }
 
 // finish a reduction: sum `n` partials of `slot` (deterministically) into
-// dscal[idx]; returns after copying it to the host (synchronises)
+// hscal[idx] (synchronises)
 int finish_sums(const int *slots, int nslots, int n, double *out);
 
 // field of a TL_FIELD_* id (the current buffer of ping-ponged fields)

@@ -65,6 +65,10 @@ struct ResCg {
   double rro;
   Ctl *ctl;
   double *hrro, *halpha, *hbeta, *herr;
+  // where the host wants alpha and beta of the first HHIST iterations from
+  // n_base on (pinned memory), or null
+  double *hist;
+  int n_base;
 };
 // 1: the loop has run and *out holds its result; 0: the mesh does not fit;
 // < 0: -(error code)
@@ -1340,7 +1344,8 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   ResCg<T> a = {b.u,  b.r,  b.p[c0], b.w,         b.z,        pin_first ? pin_first : b.p[c0],
                 b.Mi, b.Di, b.cp,    b.bfp,       b.Kx,       b.Ky,
                 b.rx, b.ry, st->n_first, st->n_last, 0,       lp,
-                st->rro, m.ctl, m.hrro, m.halpha, m.hbeta, m.herr};
+                st->rro, m.ctl, m.hrro, m.halpha, m.hbeta, m.herr,
+                cg_alphas || cg_betas ? s.hscal + HSCAL : nullptr, st->n_first};
   const int ran = resident_cg<T>(
       a, b.block ? TL_PREC_JAC_BLOCK : (b.diag ? TL_PREC_JAC_DIAG : TL_PREC_NONE), G.pitch, &res);
   if (ran < 0) return -ran;
@@ -1375,6 +1380,13 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   }
   if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("CG", res.n_end);
   const int last_done = res.reason == TL_LOOP_SWITCH ? res.n_end - 1 : res.n_end;
+  if (ran && last_done - st->n_first < HHIST) {  // the kernel has handed them over
+    for (int n = st->n_first; n <= last_done; ++n) {
+      if (cg_alphas) cg_alphas[n] = s.hscal[HSCAL + n - st->n_first];
+      if (cg_betas) cg_betas[n] = s.hscal[HSCAL + HHIST + n - st->n_first];
+    }
+    return TL_OK;
+  }
   if ((rc = copy_hist(cg_alphas, m.halpha, st->n_first, last_done))) return rc;
   if ((rc = copy_hist(cg_betas, m.hbeta, st->n_first, last_done))) return rc;
   return TL_OK;

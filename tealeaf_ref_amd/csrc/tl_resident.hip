@@ -268,6 +268,14 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
     a.ctl->old_error = err;
     a.ctl->rro = rrn;
   }
+  if (a.hist && t.blk == 0) {
+    __syncthreads();  // the leading lane has written them
+    const int last = a.n_base + HHIST - 1 < n_end ? a.n_base + HHIST - 1 : n_end;
+    for (int i = a.n_first + threadIdx.x; i <= last; i += RES_THREADS) {
+      a.hist[i - a.n_base] = a.halpha[i];
+      a.hist[HHIST + i - a.n_base] = a.hbeta[i];
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -184,11 +184,11 @@ int finish_sums(const int *slots, int nslots, int n, double *out) {
   State &s = S();
   int4 sl = make_int4(slots[0], nslots > 1 ? slots[1] : 0, nslots > 2 ? slots[2] : 0,
                       nslots > 3 ? slots[3] : 0);
+  // the kernel writes the sums to pinned host memory itself: a copy after it
+  // would cost as much again (4.5 copies a time step of a small deck)
   hipLaunchKernelGGL(k_finish, dim3(1), dim3(BLOCK), 0, s.stream, s.partials, n, sl, nslots,
-                     s.dscal);
+                     s.hscal);
   TL_HIP(hipGetLastError());
-  TL_HIP(hipMemcpyAsync(s.hscal, s.dscal, sizeof(double) * nslots, hipMemcpyDeviceToHost,
-                        s.stream));
   TL_HIP(hipStreamSynchronize(s.stream));
   for (int i = 0; i < nslots; ++i) out[i] = s.hscal[i];
   return TL_OK;
@@ -229,7 +229,6 @@ extern "C" int tl_finalize(void) {
   if (s.stream) (void)hipStreamSynchronize(s.stream);
   for (int i = 0; Field *f = all_fields(i); ++i) free_field(*f);
   if (s.partials) (void)hipFree(s.partials);
-  if (s.dscal) (void)hipFree(s.dscal);
   if (s.hscal) (void)hipHostFree(s.hscal);
   if (s.ctl) (void)hipFree(s.ctl);
   if (s.hctl) (void)hipHostFree(s.hctl);
@@ -279,8 +278,8 @@ extern "C" int tl_init(int nx, int ny, int halo, int device) {
     }
   TL_HIP(hipMalloc((void **)&s.partials, sizeof(double) * MAX_GRID * NPART));
   TL_HIP(hipMemsetAsync(s.partials, 0, sizeof(double) * MAX_GRID * NPART, s.stream));
-  TL_HIP(hipMalloc((void **)&s.dscal, sizeof(double) * 64));
-  TL_HIP(hipHostMalloc((void **)&s.hscal, sizeof(double) * 64, hipHostMallocDefault));
+  TL_HIP(hipHostMalloc((void **)&s.hscal, sizeof(double) * (HSCAL + 2 * HHIST),
+                       hipHostMallocDefault));
   // the fused loops' control block, its host copies and the loop driver's batch events
   // (set up here so that a loop call allocates nothing but its history)
   TL_HIP(hipMalloc(&s.ctl, 64));
