@@ -109,6 +109,7 @@ extern "C" int tl_snapshot_load(int slot, int field_id) {
   State &s = S();
   Field *f = field_by_id(field_id);
   if (!f) return fail(TL_ERR_ARG, "unknown field id " + std::to_string(field_id));
+  field_written(f);
   TL_HIP(hipMemcpyAsync(f->base, s.snaps[slot], s.field_bytes, hipMemcpyDeviceToDevice,
                         s.stream));
   return TL_OK;

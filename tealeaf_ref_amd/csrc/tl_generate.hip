@@ -95,6 +95,7 @@ extern "C" int tl_generate(double xmin, double ymin, double dx, double dy, int n
   if (e == hipSuccess) {
     const long n = ((long)s.nx + 2L * s.h) * ((long)s.ny + 2L * s.h);
     const int nb = (int)((n + BLOCK - 1) / BLOCK < 8192 ? (n + BLOCK - 1) / BLOCK : 8192);
+    field_written(&s.density);
     hipLaunchKernelGGL(k_generate, dim3(nb), dim3(BLOCK), 0, s.stream, s.nx, s.ny, s.h, s.pitch,
                        xmin, ymin, dx, dy, nstates, dst, s.density.p11, s.energy0.p11,
                        s.u[s.ucur].p11);

@@ -63,6 +63,10 @@ struct State {
       Kx, Ky, volume, cp, bfp;
   Field u[2], p[2], sd[2];
   int ucur = 0, pcur = 0, sdcur = 0;
+  // Kx and Ky are what tl_common_init formed from the density as it is now (its
+  // reciprocal with k_recip): no call has written either since
+  bool k_fresh = false;
+  int k_recip = 0;
   int walk_dir = 1;        // row direction of the next Chebyshev walk
 
   // reductions: partial sums per block, and small device scalars
@@ -178,6 +182,11 @@ int finish_sums(const int *slots, int nslots, int n, double *out);
 
 // field of a TL_FIELD_* id (the current buffer of ping-ponged fields)
 Field *field_by_id(int id);
+// a call writes the field (null: none) for its caller
+inline void field_written(const Field *f) {
+  State &s = S();
+  if (f == &s.density || f == &s.Kx || f == &s.Ky) s.k_fresh = false;
+}
 
 // synchronous copy of the cells inside both halos between a caller's host
 // array (halo host_halo) and the pitched device array whose cell (1,1) is

@@ -682,6 +682,7 @@ extern "C" int tl_common_init(double rx, double ry, const int zero_boundary[4]) 
   if (!zero_boundary) return fail(TL_ERR_ARG, "null zero_boundary");
   s.rx = rx;
   s.ry = ry;
+  s.k_fresh = false;
   s.zb_all = zero_boundary[0] && zero_boundary[1] && zero_boundary[2] && zero_boundary[3];
   G_LAUNCH(k_init_u, s.energy1.p11, s.density.p11, s.u[s.ucur].p11, s.u0.p11);
   const long nk = (long)(s.nx + 2 * s.h - 1) * (s.ny + 2 * s.h - 1);
@@ -691,6 +692,8 @@ extern "C" int tl_common_init(double rx, double ry, const int zero_boundary[4]) 
                      make_int4(zero_boundary[0], zero_boundary[1], zero_boundary[2],
                                zero_boundary[3]));
   TL_HIP(hipGetLastError());
+  s.k_fresh = s.zb_all;
+  s.k_recip = s.coefficient == TL_RECIP_CONDUCTIVITY ? 1 : 0;
   const long nd = (long)(s.nx + 2 * s.h - 2) * (s.ny + 2 * s.h - 2);
   hipLaunchKernelGGL(k_init_di, dim3(flat_blocks(nd)), dim3(BLOCK), 0, s.stream, s.nx, s.ny, s.h,
                      s.pitch, s.Kx.p11, s.Ky.p11, s.Di.p11, s.Mi.p11, rx, ry,

@@ -320,7 +320,9 @@ __device__ inline bool nonfinite_stop(int n, double v, double v2, Ctl *ctl) {
 // r for CG, z for PPCG and preconditioned CG), w = A p, partials of p.w.
 // On the launch that stops the loop only the p update is done, so p ends as
 // the reference leaves it.
-template <bool NT, typename T, int V>
+// DENS: the faces come from the density `Kx` points to (see walkv): 40 bytes a
+// cell instead of 48.
+template <bool NT, typename T, int V, bool DENS = false>
 __global__ __launch_bounds__(BLOCK, TL_W_WAVES) void k_loop_w(Geo G, int n, int first, int tail,
                                                    LoopParams lp, double rro_in,
                                                    const T *__restrict__ src,
@@ -333,7 +335,8 @@ __global__ __launch_bounds__(BLOCK, TL_W_WAVES) void k_loop_w(Geo G, int n, int 
                                                    int nprev, double *__restrict__ out_part,
                                                    Ctl *ctl, double *__restrict__ hrro,
                                                    double *__restrict__ hbeta,
-                                                   double *__restrict__ herr, int dir) {
+                                                   double *__restrict__ herr, int dir,
+                                                   int recip) {
   typedef typename dev::Vec<T, V>::type VT;
   __shared__ double lds[BLOCK / WAVE];
   // launches queued past the stop return at once; a block of the launch
@@ -370,7 +373,7 @@ __global__ __launch_bounds__(BLOCK, TL_W_WAVES) void k_loop_w(Geo G, int n, int 
       return upd ? src[i] + beta * pin[i] : pin[i];
     };
     auto none = [](int) { return dev::NoExtra(); };
-    dev::walkv<NT, T, V, diff_form<T>(), TL_PF_W, TL_LDSX_W>(
+    dev::walkv<NT, T, V, diff_form<T>(), TL_PF_W, TL_LDSX_W, 0, DENS>(
         G, tt, Kx, Ky, rx, ry, ldop, ld1, none, [&](int y, VT v, VT wv, dev::NoExtra) {
       if (tt.c < G.nx) {
         dev::stv<(NT && TL_ST_NT_LOOP), T, V>(w + (long)y * P, tt.c, G.nx, wv);
@@ -379,7 +382,7 @@ __global__ __launch_bounds__(BLOCK, TL_W_WAVES) void k_loop_w(Geo G, int n, int 
         for (int e = 0; e < V; ++e)
           if (tt.c + e < G.nx) acc += (double)wv[e] * (double)v[e];
       }
-    }, dir);
+    }, dir, dev::ApplyA(), recip);
   }
   if (h.stop) return;
   acc = dev::block_sum(acc, lds);
@@ -1094,6 +1097,9 @@ struct LoopBufs {
   const T *Di = nullptr, *cp = nullptr, *bfp = nullptr;
   // two more buffers for directions, which nothing else uses during CG
   T *spare[2] = {nullptr, nullptr};
+  // density that Kx and Ky were formed from and have not changed since, or null
+  const T *dens = nullptr;
+  int recip = 0;  // the conductivity is its reciprocal
 };
 
 // The u updates of CG_DEFER iterations in one pass unless TL_CG_DEFER=0 (read
@@ -1104,6 +1110,14 @@ inline bool cg_defer() {
 }
 
 inline int abs_blocks(const Geo &G) { return G.blocks < 0 ? -G.blocks : G.blocks; }
+
+// The first pass's kernel: the faces from the density where b has it.
+template <typename T, int V>
+auto w_kernel(const LoopBufs<T> &b, bool nt) {
+  if constexpr (sizeof(T) == 8)
+    if (b.dens) return nt ? k_loop_w<true, T, V, true> : k_loop_w<false, T, V, true>;
+  return nt ? k_loop_w<true, T, V> : k_loop_w<false, T, V>;
+}
 
 // Two inner sweeps per pass unless TL_SWEEP_PAIRS=0 (read on every call).
 inline bool sweep_pairs() {
@@ -1284,7 +1298,8 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   const Geo G = b.G;
   const int nb = abs_blocks(G);
   const bool nt = use_nontemporal();
-  auto kw = nt ? k_loop_w<true, T, V> : k_loop_w<false, T, V>;
+  auto kw = w_kernel<T, V>(b, nt);
+  const T *kx_or_dens = b.dens ? b.dens : b.Kx;
   // u is updated once for CG_DEFER iterations, whose directions go round as
   // many buffers; with the block preconditioner in every iteration
   const bool defer = !b.block && cg_defer();
@@ -1309,8 +1324,8 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
     hipEvent_t ev;
     prof_arm(0, &ev);
     klaunch(kw, dim3(nb), dim3(BLOCK), G, n, first ? 1 : 0, 0, lp,
-            st->rro, b.cg_src, pin, p_out(i), b.Kx, b.Ky, b.w, b.rx, b.ry,
-            m.part(P2), nb, m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1);
+            st->rro, b.cg_src, pin, p_out(i), kx_or_dens, b.Ky, b.w, b.rx, b.ry,
+            m.part(P2), nb, m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1, b.recip);
     prof_end(0, ev);
     prof_arm(1, &ev);
     if (b.block)
@@ -1335,8 +1350,8 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   auto tail = [&](int n) -> int {
     const int i = n - st->n_first;
     hipLaunchKernelGGL(kw, dim3(nb), dim3(BLOCK), 0, s.stream, G, n, 0, 1, lp, st->rro, b.cg_src,
-                       (const T *)p_in(i), p_out(i), b.Kx, b.Ky, b.w, b.rx, b.ry, m.part(P2), nb,
-                       m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1);
+                       (const T *)p_in(i), p_out(i), kx_or_dens, b.Ky, b.w, b.rx, b.ry, m.part(P2), nb,
+                       m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1, b.recip);
     TL_HIP(hipGetLastError());
     return TL_OK;
   };
@@ -1407,7 +1422,8 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   const int nb = abs_blocks(G);
   const int nzr = sweep_parts<T, V>(b, inner);  // partials of the sweeps
   const bool nt = use_nontemporal();
-  auto kw = nt ? k_loop_w<true, T, V> : k_loop_w<false, T, V>;
+  auto kw = w_kernel<T, V>(b, nt);
+  const T *kx_or_dens = b.dens ? b.dens : b.Kx;
   auto kur = nt ? k_pp_ur<true, T, V> : k_pp_ur<false, T, V>;
   const int c0 = *b.pcur;
   int sd = *b.sdcur;
@@ -1470,8 +1486,8 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
     hipEvent_t ev;
     prof_arm(5, &ev);
     klaunch(kw, dim3(nb), dim3(BLOCK), G, n, first ? 1 : 0, 0, lp,
-            rro_first, b.z, pin, p_out(i), b.Kx, b.Ky, b.w, b.rx, b.ry,
-            m.part(P3), nzr, m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, d);
+            rro_first, b.z, pin, p_out(i), kx_or_dens, b.Ky, b.w, b.rx, b.ry,
+            m.part(P3), nzr, m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, d, b.recip);
     prof_end(5, ev);
     if (deep) {
       const DeepUpdate up = {n, first ? 1 : 0, nb, nzr, i & 1, rro_first};
@@ -1502,8 +1518,8 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   auto tail = [&](int n) -> int {
     const int i = n - st->n_first;
     hipLaunchKernelGGL(kw, dim3(nb), dim3(BLOCK), 0, s.stream, G, n, 0, 1, lp, rro_first, b.z,
-                       (const T *)p_in(i), p_out(i), b.Kx, b.Ky, b.w, b.rx, b.ry, m.part(P3), nzr,
-                       m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1);
+                       (const T *)p_in(i), p_out(i), kx_or_dens, b.Ky, b.w, b.rx, b.ry, m.part(P3), nzr,
+                       m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1, b.recip);
     TL_HIP(hipGetLastError());
     return TL_OK;
   };

@@ -711,6 +711,19 @@ int cheby_run_fused(const double *ch_alphas, const double *ch_betas, int step_fi
 
 namespace {
 
+// Whether the w pass forms the faces from the density (40 bytes a cell for 48,
+// but four divisions for two cells): on meshes of at least 12 million cells, of
+// which the caches hold little.  200 CG iterations reading the faces and forming
+// them: 1500^2 7.81 and 8.03 ms, 2600^2 22.0 and 22.4, 3500^2 35.6 and 34.7, 4096^2
+// 46.5 and 45.0, 5000^2 78.5 and 73.5, 8192^2 229 and 214; PPCG at 3000^2 49.5 and
+// 49.9, 4096^2 118 and 115.  TL_DENS_FACES (read on every call) forces either.
+bool dens_faces() {
+  const char *e = getenv("TL_DENS_FACES");
+  if (e) return atoi(e) != 0;
+  const State &s = S();
+  return (double)s.nx * (double)s.ny >= 12e6;
+}
+
 // The FP64 fields as one buffer set of the shared loop kernels.
 LoopBufs<double> fp64_bufs() {
   State &s = S();
@@ -743,6 +756,10 @@ LoopBufs<double> fp64_bufs() {
   // the buffers that u's and sd's current ones alternate with
   b.spare[0] = s.u[1 - s.ucur].p11;
   b.spare[1] = s.sd[1 - s.sdcur].p11;
+  if (s.k_fresh && dens_faces()) {
+    b.dens = s.density.p11;
+    b.recip = s.k_recip;
+  }
   if (b.block) {
     // tiles start on the 4-row blocks of the preconditioner
     Geo &G = b.G;

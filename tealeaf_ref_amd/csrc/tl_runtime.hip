@@ -421,6 +421,7 @@ static int copy_field(int id, double *host, int host_halo, bool up) {
 }
 
 extern "C" int tl_upload(int field_id, const double *host, int host_halo) {
+  if (S().init) field_written(field_by_id(field_id));
   return copy_field(field_id, const_cast<double *>(host), host_halo, true);
 }
 
@@ -470,6 +471,7 @@ extern "C" int tl_upload_device(int field_id, const double *dev, long ld) {
   TL_REQUIRE_INIT();
   Field *f = field_by_id(field_id);
   if (!f) return fail(TL_ERR_ARG, "unknown field id " + std::to_string(field_id));
+  field_written(f);
   return copy_interior_device(f->p11, const_cast<double *>(dev), ld, true, "tl_upload_device");
 }
 

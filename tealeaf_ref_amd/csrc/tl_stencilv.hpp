@@ -116,11 +116,15 @@ struct ApplyA {};
 // block must walk the same rows.
 // Outside the mesh the operand is mirrored (EDGE = 0), zero (EDGE = 1) or
 // read from the halo cells as they are in memory (EDGE = 2).
+// With DENS (EDGE = 0) the faces are formed from the density `Kx` points to (Ky
+// unused), in the operations of k_init_k, so that they are its values to the
+// bit: one field is read instead of two.  Faces on the mesh's edge are zero.
 template <bool NT, typename T, int V, bool DIFF, int PF, bool LDSX = false, int EDGE = 0,
-          typename LDV, typename LD1, typename EXTRA, typename BODY, typename CELL = ApplyA>
+          bool DENS = false, typename LDV, typename LD1, typename EXTRA, typename BODY, typename CELL = ApplyA>
 __device__ inline void walkv(const Geo &g, const TileV<V> &tt, const T *__restrict__ Kx,
                              const T *__restrict__ Ky, T rx, T ry, LDV ldv_op, LD1 ld1_op,
-                             EXTRA extra, BODY body, int dir = 1, CELL cell = CELL()) {
+                             EXTRA extra, BODY body, int dir = 1, CELL cell = CELL(),
+                             int recip = 0) {
   typedef typename Vec<T, V>::type VT;
   typedef decltype(extra(0)) E;
   constexpr int NW = BLOCK / WAVE;
@@ -148,12 +152,43 @@ __device__ inline void walkv(const Geo &g, const TileV<V> &tt, const T *__restri
   const int yb = ys - dir, ya = ys + dir;
   VT vb = (EDGE == 2 || (yb >= 0 && yb < ny)) ? ldv_op(cl, yb) : (EDGE == 1 ? VT(0) : vc);
   VT va = (EDGE == 2 || (ya >= 0 && ya < ny)) ? ldv_op(cl, ya) : (EDGE == 1 ? VT(0) : vc);
-  VT kb = ldv<NT, T, V>(Ky + (long)(fwd ? ys : ys + 1) * P + cl);
-  VT ka = ldv<NT, T, V>(Ky + face_ahead(ys));
-  VT kx = ldv<NT, T, V>(Kx + (long)ys * P + cl);
+  // DENS: conductivity of a cell, the face of two, and rows of conductivities at
+  // y (dc) and ahead (da)
+  auto cond = [&](VT d) {
+    if (recip) d = T(1) / d;
+    return d;
+  };
+  auto face = [](T a, T b) { return (a + b) / (T(2) * a * b); };
+  auto faces = [&](VT a, VT b, bool in) {
+    VT f;
+#pragma unroll
+    for (int e = 0; e < V; ++e) f[e] = in ? face(a[e], b[e]) : T(0);
+    return f;
+  };
+  auto ld_dens = [&](int y) { return ldv<NT, T, V>(Kx + (long)y * P + cl); };
+  // beside: left of the wave in lane 0, right of the block in its last lane
+  const bool need_dl = lane == 0 && tt.x0 > 0;
+  const bool last_lane = lane == WAVE - 1 && edge_r, need_dr = last_lane && xr < nx;
+  auto ld_dens1 = [&](int y) {
+    return need_dl ? Kx[(long)y * P + tt.x0 - 1] : need_dr ? Kx[(long)y * P + xr] : T(1);
+  };
+  VT dc = VT(0), da = VT(0), kb, ka, kx = VT(0);
+  T ek = T(0);
+  if constexpr (DENS) {
+    const bool inb = yb >= 0 && yb < ny, ina = ya >= 0 && ya < ny;
+    dc = cond(ld_dens(ys));
+    kb = faces(dc, inb ? cond(ld_dens(yb)) : dc, inb);
+    da = ina ? cond(ld_dens(ya)) : dc;
+    ka = faces(dc, da, ina);
+    ek = ld_dens1(ys);
+  } else {
+    kb = ldv<NT, T, V>(Ky + (long)(fwd ? ys : ys + 1) * P + cl);
+    ka = ldv<NT, T, V>(Ky + face_ahead(ys));
+    kx = ldv<NT, T, V>(Kx + (long)ys * P + cl);
+    ek = need_kxr ? Kx[(long)ys * P + xr] : T(0);
+  }
   T el = need_left ? ld1_op(tt.x0 - 1, ys) : T(0);
   T er = need_right ? ld1_op(xr, ys) : T(0);
-  T ek = need_kxr ? Kx[(long)ys * P + xr] : T(0);
   E ex = extra(ys);
   // the loads that iteration j takes over when it becomes current: the
   // operand row beyond y_j (`in` false where it lies outside the mesh and
@@ -169,11 +204,16 @@ __device__ inline void walkv(const Geo &g, const TileV<V> &tt, const T *__restri
     const int yj = ys + j * dir, yo = yj + dir;
     o.in = EDGE == 2 || (yo >= 0 && yo < ny);
     o.v = o.in ? ldv_op(cl, yo) : VT(0);
-    o.ka = ldv<NT, T, V>(Ky + face_ahead(yj));
-    o.kx = ldv<NT, T, V>(Kx + (long)yj * P + cl);
+    if constexpr (DENS) {
+      o.ka = o.in ? ld_dens(yo) : VT(1);  // the row of densities beyond y_j
+      o.ek = ld_dens1(yj);
+    } else {
+      o.ka = ldv<NT, T, V>(Ky + face_ahead(yj));
+      o.kx = ldv<NT, T, V>(Kx + (long)yj * P + cl);
+      o.ek = need_kxr ? Kx[(long)yj * P + xr] : T(0);
+    }
     o.el = need_left ? ld1_op(tt.x0 - 1, yj) : T(0);
     o.er = need_right ? ld1_op(xr, yj) : T(0);
-    o.ek = need_kxr ? Kx[(long)yj * P + xr] : T(0);
     o.ex = extra(yj);
   };
   // q[i]: iteration k + 1 + i, the last one loaded during iteration k
@@ -188,6 +228,14 @@ __device__ inline void walkv(const Geo &g, const TileV<V> &tt, const T *__restri
     if (PF > 0 && k + PF < count) load_stage(k + PF, q[D - 1]);
     T left = from_lower_lane(vc[V - 1]);
     T right = from_upper_lane(vc[0]);
+    const T beside = DENS && recip ? T(1) / ek : ek;
+    if constexpr (DENS) {
+      T dl = from_lower_lane(dc[V - 1]);
+      if (need_dl) dl = beside;
+#pragma unroll
+      for (int e = 0; e < V; ++e)
+        kx[e] = c + e > 0 && c + e < nx ? face(e == 0 ? dl : dc[e > 0 ? e - 1 : 0], dc[e]) : T(0);
+    }
     T kxr = from_upper_lane(kx[0]);
     if (LDSX) {
       const int par = k & 1;
@@ -205,7 +253,11 @@ __device__ inline void walkv(const Geo &g, const TileV<V> &tt, const T *__restri
     }
     if (need_left) left = el;
     if (need_right) right = er;
-    if (need_kxr) kxr = ek;
+    if constexpr (DENS) {
+      if (last_lane) kxr = need_dr ? face(dc[V - 1], beside) : T(0);
+    } else if (need_kxr) {
+      kxr = ek;
+    }
     if (c == 0 && EDGE != 2) left = EDGE == 1 ? T(0) : vc[0];  // the left edge
     const VT &vd = fwd ? vb : va, &vu = fwd ? va : vb;
     const VT &kyd = fwd ? kb : ka, &kyu = fwd ? ka : kb;
@@ -235,8 +287,14 @@ __device__ inline void walkv(const Geo &g, const TileV<V> &tt, const T *__restri
     vc = va;
     va = nv;
     kb = ka;
-    ka = q[0].ka;
-    kx = q[0].kx;
+    if constexpr (DENS) {
+      dc = da;
+      da = cond(q[0].ka);
+      ka = faces(dc, da, q[0].in);
+    } else {
+      ka = q[0].ka;
+      kx = q[0].kx;
+    }
     el = q[0].el;
     er = q[0].er;
     ek = q[0].ek;
