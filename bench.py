@@ -11,8 +11,8 @@ Prints one JSON line.  `value` is seconds per timestep (lower is better);
 `precision_comparison` times FP64 CG / PPCG against the FP32-inner,
 FP64-refined forms at a relative residual of 1e-10 on the inverse-density
 deck;
-`roofline` uses the algorithmic bytes of the CG calc_w kernel (48 B per cell:
-read r, p, Kx, Ky; write p, w) over its HIP-event-timed launches (every 16th
+`roofline` uses the algorithmic bytes of the CG calc_w kernel (40 B per cell:
+read r, p, density; write p, w) over its HIP-event-timed launches (every 17th
 launch; launches queued past a loop's exit, which return at once, are left
 out) and takes `traffic` from the committed rocprofv3 FETCH_SIZE /
 WRITE_SIZE summary; `solvers` times Chebyshev, PPCG and Jacobi steps with
@@ -35,8 +35,9 @@ sys.path.insert(0, ROOT)
 PEAK_HBM_GBS = 8000.0
 # every EVENT_PERIOD-th launch of each kernel class in the timed steps records
 # its own start and end in HIP events (timing every launch slows a CG step
-# by a few per cent)
-EVENT_PERIOD = 16
+# by a few per cent); odd, since every fourth update pass differs from the rest
+EVENT_PERIOD = 17
+# one iteration a pass, as the reference's dataflow has it
 CG_W_BYTES_PER_CELL = 48.0      # fused calc_w: r, p, Kx, Ky in; p, w out
 CG_UR_BYTES_PER_CELL = 48.0     # calc_ur: u, p, r, w in; u, r out
 CG_ITER_BYTES_PER_CELL = 96.0
@@ -140,8 +141,44 @@ def gpu_run(cells, solver, steps, warmup, workdir, **deck_kw):
     return elapsed, iters, prof
 
 
-# algorithmic bytes per cell of one launch of the kernel classes of
-# tl_profile_get; a PPCG sweep pass, Chebyshev pass or Jacobi pass does two
+def pass_bytes(n):
+    """Algorithmic bytes per cell of one launch of the kernel classes of
+    tl_profile_get on an n x n mesh, as the loops run them: the w pass reads
+    the density for Kx and Ky from 12 million cells on; three update passes of
+    24 B (r, w in; r out) and one of 72 with u of four iterations; ten PPCG
+    sweeps with the update of r (Kx, Ky, r, w in; z, r out) or ten Chebyshev
+    iterations (u, p, u0, Kx, Ky in; u, p out) a pass; u of four PPCG
+    iterations (u, four p in; u out)."""
+    w = 40.0 if n * n >= 12e6 else 48.0
+    return {0: ("cg calc_w", w), 1: ("cg calc_ur", 36.0), 2: ("ppcg pass of ten sweeps", 48.0),
+            3: ("chebyshev pass of ten", 56.0), 4: ("jacobi pass", 48.0), 5: ("ppcg calc_w", w),
+            6: ("ppcg u of four iterations", 48.0)}
+
+
+PASS_TRAFFIC = {0: ("k_loop_w<true, double, 2, true>", "passes_{n}.md"),
+                1: ("k_cg_ur (mean)", "passes_{n}.md"),
+                2: ("k_deep_ppcg<double, 2, 10, 2, 1>", "passes_{n}.md"),
+                3: ("k_deep_cheby<10, 0>", "passes_{n}.md"),
+                4: ("k_jl_pair", "jacobi_fp64_{n}_hbm_traffic.md"),
+                5: ("k_loop_w<true, double, 2, true>", "passes_{n}.md"),
+                6: ("k_cg_u<double, 2>", "passes_{n}.md")}
+
+
+def pass_launches(solver, rows, inner=0):
+    """Launches that did work per kernel class of pass_bytes: the counts of
+    work_launches, with ten sweeps or Chebyshev iterations a pass and u of four
+    PPCG iterations in one."""
+    n = work_launches(solver, rows, inner)
+    if solver == "ppcg":
+        n[2] = n[5] * ((inner + 9) // 10)
+        n[6] = n[5] // 4
+    if solver == "chebyshev":
+        n[3] = n[3] // 5
+    return n
+
+
+# the same for passes of one or two sweeps or iterations (TL_DEEP=0,
+# TL_CG_DEFER=0, TL_DENS_FACES=0); a PPCG sweep pass, Chebyshev pass or Jacobi pass does two
 # sweeps or iterations for the bytes of one (plus, for Jacobi, the store of
 # the first iteration's u)
 # the PPCG sweep class: one first pass (48 B: r, Kx, Ky in; sd, rtemp, utemp
@@ -232,14 +269,15 @@ def solver_runs(cells, steps, warmup):
         rec["model_bytes_per_cell_step"] = model / steps
         rec["model_gbs"] = model * cells * cells / elapsed / 1e9
         rec["model_frac"] = rec["model_gbs"] / PEAK_HBM_GBS
-        kern = class_rates(prof, cells)
+        classes = pass_bytes(cells)
+        kern = class_rates(prof, cells, classes, PASS_TRAFFIC)
         rec["kernels"] = kern
         # the step's rate in counter-measured bytes: launches that did work x
         # the measured bytes per launch of their class, over the step time;
         # `covered` is the share of the step those launches take
-        counts = work_launches(solver, prof["rows"], kw.get("inner_steps", 0))
+        counts = pass_launches(solver, prof["rows"], kw.get("inner_steps", 0))
         mbytes = covered_ms = 0.0
-        for cls, (name, _) in CLASS_BYTES.items():
+        for cls, (name, _) in classes.items():
             k = kern.get(name)
             if counts[cls] and k and "measured_bytes_per_launch" in k:
                 mbytes += counts[cls] * k["measured_bytes_per_launch"]
@@ -248,7 +286,7 @@ def solver_runs(cells, steps, warmup):
             rec["step_measured_gbs"] = mbytes / elapsed / 1e9
             rec["step_measured_frac"] = rec["step_measured_gbs"] / PEAK_HBM_GBS
             rec["step_time_covered"] = covered_ms * 1e-3 / elapsed
-            rec["work_launches"] = {CLASS_BYTES[c][0]: v for c, v in counts.items() if v}
+            rec["work_launches"] = {classes[c][0]: v for c, v in counts.items() if v}
         log(f"[bench] {cells}^2 {solver}: {rec}")
         out[solver] = rec
     return out
@@ -357,9 +395,20 @@ MIXED_CG_TRAFFIC = {0: ("k_loop_w<float>", "ppcg_mixed_{n}_hbm_traffic.md"),
                     1: ("k_cg_ur<float>", "ppcg_mixed_{n}_hbm_traffic.md")}
 
 
+# as the loops run them (see pass_bytes); the FP32 w pass reads Kx and Ky
+MIXED_PASS_BYTES = {0: ("fp32 cg calc_w", 24.0), 1: ("fp32 cg calc_ur", 18.0),
+                    2: ("fp32 ppcg pass of ten sweeps", 24.0), 5: ("fp32 ppcg calc_w", 24.0),
+                    6: ("fp32 ppcg u of four iterations", 24.0)}
+MIXED_PASS_TRAFFIC = {0: ("k_loop_w<true, float, 4, false>", "passes_{n}.md"),
+                      1: ("k_cg_ur<float> (mean)", "passes_{n}.md"),
+                      2: ("k_deep_ppcg<float, 4, 10, 2, 1>", "passes_{n}.md"),
+                      5: ("k_loop_w<true, float, 4, false>", "passes_{n}.md"),
+                      6: ("k_cg_u<float, 4>", "passes_{n}.md")}
+
+
 def mixed_kernel_rates(prof, cells):
-    """Per-class launch time and HBM rates of a mixed-precision PPCG run."""
-    return class_rates(prof, cells, MIXED_PPCG_BYTES, MIXED_PPCG_TRAFFIC)
+    """Per-class launch time and HBM rates of a mixed-precision run."""
+    return class_rates(prof, cells, MIXED_PASS_BYTES, MIXED_PASS_TRAFFIC)
 
 
 def host_true_residual(cells, rx, ry):
@@ -464,9 +513,9 @@ def precision_comparison(cells, inner_steps=10, target=1e-10, later_step=False):
         if name == "mixed_ppcg":
             rec["kernels"] = mixed_kernel_rates(prof, cells)
         elif name == "mixed_cg":
-            rec["kernels"] = class_rates(prof, cells, MIXED_CG_BYTES, MIXED_CG_TRAFFIC)
+            rec["kernels"] = mixed_kernel_rates(prof, cells)
         elif not extra:
-            rec["kernels"] = class_rates(prof, cells)
+            rec["kernels"] = class_rates(prof, cells, pass_bytes(cells), PASS_TRAFFIC)
         summ = [last["volume"], last["mass"], last["energy"], last["temperature"]]
         if ref_u is None:
             ref_u, ref_sum = u, summ
@@ -752,7 +801,7 @@ def profile_run(cells, iters, solver="cg", copies=4):
     deck capped at `iters` iterations, then `copies` launches of the plain
     copy kernel (tl_ppcg_store_r: r_store = r over the interior, 8 B read +
     8 B written per cell), whose counters calibrate FETCH_SIZE / WRITE_SIZE.
-    Solvers: "cg"; "ppcg" (10 inner steps; the switch to PPCG at the 100th
+    Solvers: "cg"; "chebyshev" (20 presteps); "ppcg" (10 inner steps; the switch to PPCG at the 100th
     CG iteration: tl_ch_cg_presteps 100 with an epslim no error exceeds);
     "mixed_ppcg" (FP32 PPCG under FP64 refinement, inverse-density
     coefficient, at most 2 refinements of at most `iters` iterations)."""
@@ -762,6 +811,8 @@ def profile_run(cells, iters, solver="cg", copies=4):
     kw = {}
     if solver == "ppcg":
         kw = {"inner_steps": 10, "presteps": 100, "epslim": 1e30}
+    elif solver == "chebyshev":
+        kw = {"presteps": 20, "epslim": 1e30}
     elif solver == "mixed_ppcg":
         kw = {"inner_steps": 10, "coefficient": "inverse_density",
               "extra": ("tl_mixed_precision", "tl_mixed_max_refinements=2")}
@@ -797,7 +848,7 @@ def main():
     ap.add_argument("--mixed-sizes", default="4096,8192",
                     help="comma-separated mesh sizes of the FP64 vs FP32-refined comparison "
                          "('' to skip)")
-    ap.add_argument("--profile-solver", default="cg", choices=["cg", "ppcg", "mixed_ppcg"],
+    ap.add_argument("--profile-solver", default="cg", choices=["cg", "chebyshev", "ppcg", "mixed_ppcg"],
                     help="solver of the counter-profiling mode")
     ap.add_argument("--profile-iters", type=int, default=0,
                     help="counter-profiling mode: one CG step capped at this many iterations "
@@ -848,9 +899,10 @@ def main():
     # (every EVENT_PERIOD-th launch; the few launches queued past the exit,
     # which return at once, are left out: rocprof's average over all launches
     # includes them and reads ~0.5 % lower)
-    w_gbs = CG_W_BYTES_PER_CELL * cells / (ms_w / n_w * 1e-3) / 1e9 if ms_w else None
-    ur_gbs = CG_UR_BYTES_PER_CELL * cells / (ms_ur / n_ur * 1e-3) / 1e9 if ms_ur else None
-    step_gbs = CG_ITER_BYTES_PER_CELL * cells * exec_iters / elapsed / 1e9
+    w_bytes, ur_bytes = (pass_bytes(args.cells)[c][1] for c in (0, 1))
+    w_gbs = w_bytes * cells / (ms_w / n_w * 1e-3) / 1e9 if ms_w else None
+    ur_gbs = ur_bytes * cells / (ms_ur / n_ur * 1e-3) / 1e9 if ms_ur else None
+    step_gbs = (w_bytes + ur_bytes) * cells * exec_iters / elapsed / 1e9
     out = {
         "metric": "s/timestep + HBM GB/s at 4096^2: FP64 CG vs FP32-refined PPCG @1e-10 residual",
         "value": s_per_step,
@@ -874,9 +926,10 @@ def main():
         "roofline": {"bound": "hbm", "kernel": "cg calc_w (w = A p, p = r + beta p, p.w)",
                      "achieved": w_gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": (w_gbs / PEAK_HBM_GBS) if w_gbs else None,
-                     "traffic": measured_traffic("k_loop_w", args.cells),
-                     "traffic_source": "profiles/cg_fp64_4096_hbm_traffic.md",
-                     "bytes_per_cell": CG_W_BYTES_PER_CELL,
+                     "traffic": measured_traffic(PASS_TRAFFIC[0][0], args.cells,
+                                                 PASS_TRAFFIC[0][1]),
+                     "traffic_source": "profiles/" + PASS_TRAFFIC[0][1].format(n=args.cells),
+                     "bytes_per_cell": w_bytes,
                      "avg_launch_ms": ms_w / n_w if n_w else None, "timed_launches": n_w,
                      "idle_launches": idle_w,
                      "event_sample_period": EVENT_PERIOD,
