@@ -95,13 +95,13 @@ struct ResCheby {
 };
 int resident_cheby(const ResCheby &a, const double *alphas, const double *betas, int count,
                    long pitch, bool want_norm, double *norm);
-// The same for PPCG's outer iterations without a preconditioner and their inner
-// steps; the pointers as in run_ppcg_loop, r_store written only.
+// The same for PPCG's outer iterations and their inner steps; the pointers as in
+// run_ppcg_loop, r_store written only.
 template <typename T>
 struct ResPpcg {
   T *u, *r, *r_store, *p, *z;
   const T *pin;
-  const T *Kx, *Ky;
+  const T *Mi, *Di, *cp, *bfp, *Kx, *Ky;
   T rx, ry, theta_r;
   int n_first, n_last, n_pause, inner;
   double eps_abs, rro;
@@ -109,7 +109,8 @@ struct ResPpcg {
   double *herr;
 };
 template <typename T>
-int resident_ppcg(ResPpcg<T> a, const double *alphas, const double *betas, long pitch, Ctl *out);
+int resident_ppcg(ResPpcg<T> a, int prec, const double *alphas, const double *betas, long pitch,
+                  Ctl *out);
 constexpr int RES_PAUSED = 0;  // reason of a launch that stopped for the host only
 
 bool use_nontemporal();
@@ -1434,11 +1435,13 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   lp.presteps = 0;
   const T theta_r = (T)(1.0 / theta);
   Ctl res;
-  if (!b.diag && !b.block && deep_fits()) {
-    const ResPpcg<T> a = {b.u,   b.r,  b.r_store, b.p[c0], b.z,         pin_first ? pin_first : b.p[c0],
-                          b.Kx,  b.Ky, b.rx,      b.ry,    theta_r,     st->n_first,
-                          st->n_last, 0, inner, st->eps_abs, rro_first, m.ctl, m.herr};
-    const int ran = resident_ppcg<T>(a, alphas, betas, G.pitch, &res);
+  if (deep_fits()) {
+    const ResPpcg<T> a = {b.u,  b.r,   b.r_store, b.p[c0], b.z, pin_first ? pin_first : b.p[c0],
+                          b.Mi, b.Di,  b.cp,      b.bfp,   b.Kx, b.Ky,
+                          b.rx, b.ry,  theta_r,   st->n_first, st->n_last, 0,
+                          inner, st->eps_abs, rro_first, m.ctl, m.herr};
+    const int prec = b.block ? TL_PREC_JAC_BLOCK : b.diag ? TL_PREC_JAC_DIAG : TL_PREC_NONE;
+    const int ran = resident_ppcg<T>(a, prec, alphas, betas, G.pitch, &res);
     if (ran < 0) return -ran;
     if (ran) {
       st->n_end = res.n_end;

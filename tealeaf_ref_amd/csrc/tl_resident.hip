@@ -562,7 +562,8 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cheby(ResGeo g, ChebyArgs a
 // ---------------------------------------------------------------------------
 // The inner steps work on z and z one step before, as k_deep_ppcg's do, and
 // need z's halos alone; two sums end an outer iteration (z.r and (r -
-// r_store).z) and one its first half.
+// r_store).z) and one its first half.  With a preconditioner M the steps start
+// from M^-1 r / theta and add beta M^-1 (r - A z).
 //
 // What bounds it: with ten inner steps the exchanges, ten of 0.9 us and two of 1.4
 // to 2.1, and from four rows a lane on the arithmetic.  Whole steps against the
@@ -585,9 +586,11 @@ struct PpcgPlan {
   static_assert(BYTES + sizeof(ResShared<T, R, 2>) <= 160 * 1024, "LDS of a CU");
 };
 
-template <typename T, int R>
+template <typename T, int R, int PREC>
 __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> args) {
   typedef typename dev::Vec<T, 2>::type VT;
+  constexpr bool DIAG = PREC == TL_PREC_JAC_DIAG, BLK = PREC == TL_PREC_JAC_BLOCK;
+  constexpr bool M_REGS = DIAG && R * sizeof(T) < 48;  // else read again in every step
   constexpr bool LDS = PpcgPlan<T, R>::LDS, RS_MEMORY = PpcgPlan<T, R>::RS_MEMORY;
   const ResPpcg<T> &a = args.f;
   extern __shared__ char dyn[];
@@ -611,6 +614,42 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> 
     r[j] = t.load(a.r, g, t.y0 + j);
     z[j] = zp[j] = VT(0);
   }
+  // Mi; and of the block preconditioner's groups of four rows Di and cp of the
+  // first and bfp of the others (cells outside the mesh have bfp = cp = 0, Di = 1)
+  VT m[M_REGS ? R : 1], di[BLK ? R / 4 : 1], c0[BLK ? R / 4 : 1], bf[BLK ? R : 1];
+  if constexpr (M_REGS)
+#pragma unroll
+    for (int j = 0; j < R; ++j) m[j] = t.load(a.Mi, g, t.y0 + j);
+  if constexpr (BLK)
+#pragma unroll
+    for (int b = 0; b < R; b += 4) {
+      di[b / 4] = t.load(a.Di, g, t.y0 + b);
+      c0[b / 4] = t.load(a.cp, g, t.y0 + b);
+      if (!t.okx || b >= t.rows) di[b / 4].x = T(1);
+      if (!t.oky || b >= t.rows) di[b / 4].y = T(1);
+#pragma unroll
+      for (int q = 1; q < 4; ++q) bf[b + q] = t.load(a.bfp, g, t.y0 + b + q);
+    }
+  // M^-1 of a row, or of all rows (tea_block_solve, as in k_res_cg)
+  auto mul = [&](int j, VT x, int row) {
+    if constexpr (M_REGS) return m[j] * x;
+    else if constexpr (DIAG) return t.load(a.Mi, g, row + j) * x;
+    else return x;
+  };
+  auto solve = [&](VT (&x)[R]) {
+#pragma unroll
+    for (int b = 0; b < R; b += 4) {
+      x[b] = x[b] / di[b / 4];
+#pragma unroll
+      for (int q = 1; q < 4; ++q)
+        x[b + q] = (x[b + q] - (-k.ky(b + q) * a.ry) * x[b + q - 1]) * bf[b + q];
+#pragma unroll
+      for (int q = 2; q >= 0; --q) {
+        const VT c = q > 0 ? (-k.ky(b + q + 1) * a.ry) * bf[b + (q > 0 ? q : 1)] : c0[b / 4];
+        x[b + q] = b + q + 1 < t.rows ? x[b + q] - c * x[b + q + 1] : x[b + q];
+      }
+    }
+  };
   ResGhost<T> pg = load_ghosts<T, R>(t, g, a.pin), gh;
   const bool lead = t.blk == 0 && threadIdx.x == 0;
   double rro = a.rro, err = 0.0, sums[2] = {0.0, 0.0};
@@ -655,8 +694,13 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> 
       if constexpr (RS_MEMORY) t.store(a.r_store, g, t.c, row + j, r[j]);
       else rs.set(j, r[j]);
       r[j] = r[j] - al * z[j];
-      z[j] = r[j] * a.theta_r;
+      z[j] = BLK ? r[j] : mul(j, r[j], row) * a.theta_r;
       zp[j] = VT(0);
+    }
+    if constexpr (BLK) {
+      solve(z);
+#pragma unroll
+      for (int j = 0; j < R; ++j) z[j] = z[j] * a.theta_r;
     }
     // ---- the inner steps
     for (int i = 0; i < a.inner; ++i) {
@@ -668,6 +712,8 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> 
       if (t.lane < 2 * R) side[t.lane] = gh.side;
       __builtin_amdgcn_wave_barrier();
       VT dn = gh.dn, kd = k.ky(0);
+      VT d[BLK ? R : 1];
+      const int at = t.row_anew();
 #pragma unroll
       for (int j = 0; j < R; ++j) {
         if (R * sizeof(T) >= 48) __builtin_amdgcn_sched_barrier(0);
@@ -683,13 +729,28 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> 
                                            ku.x, a.rx, a.ry);
         w.y = dev::op_cell<diff_form<T>()>(c.y, c.x, rt, dn.y, up.y, k.kx[j].y, kr, kd.y, ku.y,
                                            a.rx, a.ry);
-        VT zn = c + ca * (c - zp[j]) + cb * (r[j] - w);
+        if constexpr (BLK) {
+          d[j] = r[j] - w;
+          dn = c;
+          kd = ku;
+          continue;
+        }
+        VT zn = c + ca * (c - zp[j]) + cb * mul(j, r[j] - w, at);
         // a row is finished before the next, or all rows' operands wait together
         if (R * sizeof(T) >= 48) asm volatile("" : "+v"(zn.x), "+v"(zn.y));
         zp[j] = c;
         z[j] = zn;
         dn = c;
         kd = ku;
+      }
+      if constexpr (BLK) {
+        solve(d);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          const VT c = z[j];
+          z[j] = c + ca * (c - zp[j]) + cb * d[j];
+          zp[j] = c;
+        }
       }
     }
     if (dead) break;
@@ -1053,13 +1114,15 @@ int resident_cheby(const ResCheby &f, const double *alphas, const double *betas,
 }
 
 template <typename T>
-int resident_ppcg(ResPpcg<T> f, const double *alphas, const double *betas, long pitch, Ctl *out) {
+int resident_ppcg(ResPpcg<T> f, int prec, const double *alphas, const double *betas, long pitch,
+                  Ctl *out) {
   State &s = S();
   if (!resident_on() || f.inner < 1 || f.inner > RES_PPCG_STEPS) return 0;
-  static constexpr int R64[] = {1, 2, 3, 4, 6}, R32[] = {1, 2, 3, 4, 6, 8, 12};
+  static constexpr int R64[] = {1, 2, 3, 4, 6}, R32[] = {1, 2, 3, 4, 6, 8, 12}, RBLK[] = {4};
   const ResCost cost = {0.019, 0.2 * (f.inner + 2), 0.0, 0};
-  const int R = sizeof(T) == 8 ? res_rows(s.nx, s.ny, R64, 5, cost)
-                               : res_rows(s.nx, s.ny, R32, 7, cost);
+  const int R = sizeof(T) == 4                 ? res_rows(s.nx, s.ny, R32, 7, cost)
+                : prec == TL_PREC_JAC_BLOCK ? res_rows(s.nx, s.ny, RBLK, 1, cost)
+                                            : res_rows(s.nx, s.ny, R64, 5, cost);
   if (!R) return 0;
   ResGeo g = res_geo(R, pitch);
   PpcgArgs<T> a;
@@ -1076,14 +1139,20 @@ int resident_ppcg(ResPpcg<T> f, const double *alphas, const double *betas, long 
     a.f.n_pause = (int)(a.f.n_first + run - 1);
     int rc;
     if ((rc = res_tags((f.inner + 2L) * run, &g.epoch))) return -rc;
-#define CASE(RR) R == RR ? res_launch(&k_res_ppcg<T, RR>, g, a, PpcgPlan<T, RR>::BYTES)
-    if constexpr (sizeof(T) == 8)
-      rc = CASE(1) : CASE(2) : CASE(3) : CASE(4)
-           : res_launch(&k_res_ppcg<T, 6>, g, a, PpcgPlan<T, 6>::BYTES);
+#define RUN(RR, PP) res_launch(&k_res_ppcg<T, RR, PP>, g, a, PpcgPlan<T, RR>::BYTES)
+#define CASE(RR, PP) R == RR ? RUN(RR, PP)
+    constexpr int NONE = TL_PREC_NONE, DIAG = TL_PREC_JAC_DIAG, BLK = TL_PREC_JAC_BLOCK;
+    if constexpr (sizeof(T) == 4)
+      rc = CASE(1, NONE) : CASE(2, NONE) : CASE(3, NONE) : CASE(4, NONE) : CASE(6, NONE)
+           : CASE(8, NONE) : RUN(12, NONE);
+    else if (prec == BLK)
+      rc = RUN(4, BLK);
+    else if (prec == DIAG)
+      rc = CASE(1, DIAG) : CASE(2, DIAG) : CASE(3, DIAG) : CASE(4, DIAG) : RUN(6, DIAG);
     else
-      rc = CASE(1) : CASE(2) : CASE(3) : CASE(4) : CASE(6) : CASE(8)
-           : res_launch(&k_res_ppcg<T, 12>, g, a, PpcgPlan<T, 12>::BYTES);
+      rc = CASE(1, NONE) : CASE(2, NONE) : CASE(3, NONE) : CASE(4, NONE) : RUN(6, NONE);
 #undef CASE
+#undef RUN
     if (rc == RES_REFUSED)
       return a.f.n_first == f.n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
     if (rc || (rc = res_wait())) return -rc;
@@ -1099,7 +1168,9 @@ int resident_ppcg(ResPpcg<T> f, const double *alphas, const double *betas, long 
     a.f.pin = a.f.p;
   }
 }
-template int resident_ppcg<double>(ResPpcg<double>, const double *, const double *, long, Ctl *);
-template int resident_ppcg<float>(ResPpcg<float>, const double *, const double *, long, Ctl *);
+template int resident_ppcg<double>(ResPpcg<double>, int, const double *, const double *, long,
+                                   Ctl *);
+template int resident_ppcg<float>(ResPpcg<float>, int, const double *, const double *, long,
+                                  Ctl *);
 
 }  // namespace tl

@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
 SIZES = [(3, 2), (7, 31), (107, 9), (109, 64), (217, 45), (250, 37), (501, 133), (130, 400)]
 
 
-def _ppcg_sweeps(sizes, inner, reflective, envs):
+def _ppcg_sweeps(sizes, inner, reflective, envs, precond=1):
     """z after one outer iteration, i.e. the Chebyshev polynomial of r.
 
     Tolerance: with bounds that hold the spectrum the recurrence is stable, so
@@ -32,7 +32,7 @@ def _ppcg_sweeps(sizes, inner, reflective, envs):
     pd = C.POINTER(C.c_double)
     for nx, ny in sizes:
         print(f"ppcg {nx}x{ny} inner {inner} reflective {reflective} {envs[1]}", flush=True)
-        d, rx, ry = _chunk(nx, ny, 1, reflective)
+        d, rx, ry = _chunk(nx, ny, precond, reflective)
         try:
             out = []
             for kw in envs:
@@ -79,6 +79,16 @@ def test_ppcg_sweeps(inner, reflective):
 def test_ppcg_on_chip(rows, inner, reflective):
     """The outer iterations on the chip against the passes of one and two sweeps."""
     _ppcg_sweeps(TILE_SIZES[1:], inner, reflective, ({"TL_DEEP": 0}, {"TL_RES_ROWS": rows}))
+
+
+@pytest.mark.parametrize("precond,rows,inner", [(2, 1, 10), (2, 2, 3), (2, 3, 7), (2, 4, 10),
+                                                (2, 6, 5), (3, 4, 10), (3, 4, 3)])
+@pytest.mark.parametrize("reflective", [False, True])
+def test_preconditioned_ppcg_on_chip(precond, rows, inner, reflective):
+    """With jac_diag and jac_block against the passes of one and two sweeps; M^-1
+    is at most 1, since A's diagonal and its blocks' eigenvalues are at least 1."""
+    _ppcg_sweeps(TILE_SIZES[1:], inner, reflective, ({"TL_RESIDENT": 0}, {"TL_RES_ROWS": rows}),
+                 precond)
 
 
 @pytest.mark.parametrize("inner", [7, 10, 14])
