@@ -207,7 +207,7 @@ def class_rates(prof, cells, classes=CLASS_BYTES, traffic=CLASS_TRAFFIC):
     out = {}
     for cls, (name, bpc) in classes.items():
         n, ms, idle = prof.get(cls, (0, 0.0, 0))
-        if not n:
+        if n < 4:  # one CG update in four carries u: fewer samples are no mean
             continue
         k = {"timed_launches": n, "idle_launches": idle, "avg_launch_ms": ms / n,
              "achieved_gbs": bpc * cells * cells / (ms / n * 1e-3) / 1e9, "bytes_per_cell": bpc}

@@ -361,11 +361,15 @@ int tl_hbm_stream(long n, int reps, double *copy_gbs, double *triad_gbs);
 /* ---- timing of the dominant kernels (HIP events on the library stream) --- */
 /* on = 1 times every launch of the solver kernels with HIP events, on = N > 1
  * every N-th launch of each class (events between launches slow a loop by a
- * few per cent; sampling keeps that out of a timed run), on = 0 stops. */
+ * few per cent; sampling keeps that out of a timed run), on = 0 stops.  While
+ * it is on, the loops run the pass kernels also on meshes that they would
+ * otherwise solve in one launch with the mesh on the chip. */
 int tl_profile_enable(int on);
 /* Returns timed launch count and their total milliseconds for a kernel class:
- * 0 = CG calc_w, 1 = CG calc_ur, 2 = PPCG inner sweep, 3 = Chebyshev iterate,
- * 4 = Jacobi, 5 = PPCG calc_w, 6 = PPCG calc_ur, 7 = mixed-precision FP64
+ * 0 = CG calc_w, 1 = CG calc_ur (u of four iterations in every fourth), 2 =
+ * PPCG inner sweeps (up to ten a pass, with the update of r), 3 = Chebyshev
+ * iterations (up to ten a pass), 4 = Jacobi, 5 = PPCG calc_w, 6 = PPCG's u of
+ * four iterations, or calc_ur with a preconditioner, 7 = mixed-precision FP64
  * refinement (u += d, true residual).  Launches that returned at once (queued
  * past a loop's exit: shorter than a quarter of the median timed launch of
  * the class) are left out and counted by tl_profile_idle. */
