@@ -112,7 +112,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
   bool dead = false, update = false;
   T be = T(0);
   ResGhost<T> gh;
-  unsigned s = 0;
+  ResOrder<true> o;
   if (lead) a.hrro[a.n_first] = rro;
   __syncthreads();
   // body(j, w) of row j of w = A p
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
       acc += (double)wv.y * (double)p[j].y;
     });
     double pw;
-    if (!dev::res_exchange<false, true>(t, g, sh, s++, acc, &pw, (const VT(*)[R]) nullptr,
+    if (!dev::res_exchange<false, true>(t, g, sh, o, acc, &pw, (const VT(*)[R]) nullptr,
                                         (ResGhost<T> *)nullptr)) {
       dead = true;
       break;
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
         acc += (double)r[j].x * (double)r[j].x;
         acc += (double)r[j].y * (double)r[j].y;
       }
-      ok = dev::res_exchange<true, true>(t, g, sh, s++, acc, &rrn, &r, &gh);
+      ok = dev::res_exchange<true, true>(t, g, sh, o, acc, &rrn, &r, &gh);
     } else {
       if constexpr (PREC == TL_PREC_JAC_DIAG) {
 #pragma unroll
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
         acc += (double)r[j].x * (double)z[j].x;
         acc += (double)r[j].y * (double)z[j].y;
       }
-      ok = dev::res_exchange<true, true>(t, g, sh, s++, acc, &rrn, &z, &gh);
+      ok = dev::res_exchange<true, true>(t, g, sh, o, acc, &rrn, &z, &gh);
     }
     if (!ok) {
       dead = true;
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
   double err = 0.0;
   int reason = 0, n = a.n_first;
   bool dead = false;
-  unsigned s = 0;
+  ResOrder<true> o;
   __syncthreads();
   for (;; ++n) {
     if (t.lane < 2 * R) side[t.lane] = gh.side;
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_jacobi(ResGeo g, ResJacobi 
       u[j] = v;
     }
     double sum;
-    if (!dev::res_exchange<true, true>(t, g, sh, s++, acc, &sum, &u, &gh)) {
+    if (!dev::res_exchange<true, true>(t, g, sh, o, acc, &sum, &u, &gh)) {
       dead = true;
       break;
     }
@@ -498,6 +498,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cheby(ResGeo g, ChebyArgs a
   __syncthreads();
   double acc = 0.0;
   const int col = t.col_anew();
+  ResOrder<false> o;
   for (int n = 0;; ++n) {
     const bool end = n + 1 == a.count, out = end && a.last;
     const T al = a.a[n], be = a.b[n];
@@ -531,7 +532,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cheby(ResGeo g, ChebyArgs a
       kd = ku;
     }
     if (end) break;
-    if (!dev::res_exchange<true, false>(t, g, sh, (unsigned)n, 0.0, (double *)nullptr, &u, &gh)) {
+    if (!dev::res_exchange<true, false>(t, g, sh, o, 0.0, (double *)nullptr, &u, &gh)) {
       if (threadIdx.x == 0) *g.abort_flag = 1;
       return;
     }
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cheby(ResGeo g, ChebyArgs a
     if (threadIdx.x == 0 && (sh.dead[0] || sh.dead[1])) *g.abort_flag = 1;
   } else {
     double rr;
-    if (!dev::res_exchange<false, true>(t, g, sh, (unsigned)a.count, acc, &rr,
+    if (!dev::res_exchange<false, true>(t, g, sh, o, acc, &rr,
                                         (const VT(*)[R]) nullptr, (ResGhost<T> *)nullptr)) {
       if (threadIdx.x == 0) *g.abort_flag = 1;
       return;
@@ -656,7 +657,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> 
   int reason = 0, n_end = 0;
   bool dead = false, update = false;
   T be = T(0);
-  unsigned s = 0;
+  ResOrder<false> o;
   __syncthreads();
   for (int n = a.n_first;; ++n) {
     // ---- w = A p (in z), p.w
@@ -675,7 +676,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> 
       });
     }
     double pw;
-    if (!dev::res_exchange<false, 1>(t, g, sh, s++, acc, &pw, (const VT(*)[R]) nullptr,
+    if (!dev::res_exchange<false, 1>(t, g, sh, o, acc, &pw, (const VT(*)[R]) nullptr,
                                      (ResGhost<T> *)nullptr)) {
       dead = true;
       break;
@@ -704,7 +705,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> 
     }
     // ---- the inner steps
     for (int i = 0; i < a.inner; ++i) {
-      if (!dev::res_exchange<true, 0>(t, g, sh, s++, 0.0, (double *)nullptr, &z, &gh)) {
+      if (!dev::res_exchange<true, 0>(t, g, sh, o, 0.0, (double *)nullptr, &z, &gh)) {
         dead = true;
         break;
       }
@@ -766,7 +767,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_ppcg(ResGeo g, PpcgArgs<T> 
       a1 += (double)z[j].x * (double)r[j].x;
       a1 += (double)z[j].y * (double)r[j].y;
     }
-    if (!dev::res_exchange<true, 2>(t, g, sh, s++, a0, sums, &z, &gh, a1)) {
+    if (!dev::res_exchange<true, 2>(t, g, sh, o, a0, sums, &z, &gh, a1)) {
       dead = true;
       break;
     }

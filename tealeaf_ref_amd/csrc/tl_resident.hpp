@@ -15,9 +15,9 @@
 // 32-bit tag, written and read with relaxed atomics of agent scope: a reader
 // that finds the tag of the current exchange has the payload, so neither
 // fences nor flags are needed, and a word is never read half written.  Tags
-// count up over the life of the chunk; the buffers start as zeros, and
-// exchange s uses buffer s & 1, which its readers have left when exchange
-// s + 2 writes it, because exchange s + 1 waits for them.
+// count up over the life of the chunk, and the buffers start as zeros.  There
+// are two copies of them, so that no word is written again before its readers
+// have it (tl_res_order.hpp).
 //
 // The grid never exceeds one block per CU and is launched cooperatively, so
 // that all blocks are resident; a wait that lasts longer than `limit` ticks of
@@ -25,6 +25,7 @@
 #pragma once
 
 #include "tl_loopk.hpp"
+#include "tl_res_order.hpp"
 
 namespace tl {
 
@@ -135,8 +136,8 @@ __device__ inline T value_of(const Words<T> &o) {
 }
 
 // One block's LDS besides the fields it keeps there.  What one wave writes for
-// others is indexed by the exchange's parity (EB = 1 for the edge rows where
-// every second exchange has none): a wave that is an exchange ahead never
+// others is indexed by the exchange's or the sum's parity (EB = 1 for the edge
+// rows where every second exchange has none): a wave that is an exchange ahead never
 // writes what another still reads.
 template <typename T, int R, int EB>
 struct ResShared {
@@ -291,28 +292,30 @@ struct ResGhost {
   T side;
 };
 
-// Exchange number s of the loop (tag epoch + s, buffer s & 1).  HALO: the
+// The loop's next exchange, number o.s.  HALO: the
 // edges of `v` go to the neighbours and their edges come back in `gh`.  SUM:
 // returns one or two sums of `part` (and `part2`) over the lanes of all blocks,
 // added in one fixed order everywhere, so every block has the same bits.  Returns false in
 // every wave of a block when a wait of the block has run out (in a wave that
 // waits for halos alone, one exchange later).
-template <bool HALO, int SUM, typename T, int R, int EB>
+template <bool HALO, int SUM, typename T, int R, int EB, typename ORDER>
 __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
-                                    ResShared<T, R, EB> &sh, unsigned s, double part, double *total,
+                                    ResShared<T, R, EB> &sh, ORDER &o, double part, double *total,
                                     const typename Vec<T, 2>::type (*v)[R], ResGhost<T> *gh,
                                     double part2 = 0.0) {
   typedef typename Vec<T, 2>::type VT;
-  const int eb = EB > 1 ? s & 1 : 0;
+  static_assert(SUM > 0 || !ORDER::every_sums, "the loop's order");
+  const int buf = o.halos(), sb = o.sums();  // the exchange's parity, and the sum's
+  const int eb = EB > 1 ? buf : 0;
   constexpr int SIDE = RES_WAVES * R;        // values of one side
-  const unsigned tag = g.epoch + s;
-  const int buf = s & 1;
+  const unsigned tag = o.tag(g.epoch);
+  o.next(SUM > 0);
   const int nb = g.tx * g.ty;
   // the tallest tiles form their addresses anew in every exchange: no registers
   // to hold them through the loop
   int lane = t.lane;
   if (R * sizeof(T) >= 64) asm volatile("" : "+v"(lane));
-  u64 *parts = g.part + buf * (RES_MAX_BLOCKS * RES_PART_WORDS);
+  u64 *parts = g.part + sb * (RES_MAX_BLOCKS * RES_PART_WORDS);
   u64 *halos = g.halo + buf * (RES_MAX_BLOCKS * RES_HALO_WORDS);
   constexpr int W = res_words<T>();
   // runs of a block's halo: bottom row, top row, left side, right side
@@ -350,8 +353,8 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
     part = wave_total(part);
     if (SUM > 1) part2 = wave_total(part2);
     if (lane == 0) {
-      sh.red[buf][0][t.wave] = part;
-      if (SUM > 1) sh.red[buf][1][t.wave] = part2;
+      sh.red[sb][0][t.wave] = part;
+      if (SUM > 1) sh.red[sb][1][t.wave] = part2;
     }
   }
   __syncthreads();
@@ -360,7 +363,7 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
 #pragma unroll
     for (int m = 0; m < SUM; ++m)
 #pragma unroll
-      for (int i = 0; i < RES_WAVES; ++i) own[m] += sh.red[buf][m][i];
+      for (int i = 0; i < RES_WAVES; ++i) own[m] += sh.red[sb][m][i];
     if (nb > 1 && t.wave == 0 && lane < 2 * SUM) {
       const u64 b = __builtin_bit_cast(u64, SUM > 1 && lane >= 2 ? own[1] : own[0]);
       put(parts, t.blk * RES_PART_WORDS + lane, lane & 1 ? (unsigned)(b >> 32) : (unsigned)b, tag);
@@ -445,13 +448,13 @@ __device__ inline bool res_exchange(const ResTile<T, R> &t, const ResGeo &g,
 #pragma unroll
         for (int m = 0; m < SUM; ++m) {
           q[m] = wave_total(q[m]);
-          if (lane == 0) sh.tot[buf][m][t.wave - 1] = q[m];
+          if (lane == 0) sh.tot[sb][m][t.wave - 1] = q[m];
         }
       __syncthreads();
 #pragma unroll
       for (int m = 0; m < SUM; ++m) {
         own[m] = 0.0;
-        for (int i = 0; i < waves; ++i) own[m] += sh.tot[buf][m][i];
+        for (int i = 0; i < waves; ++i) own[m] += sh.tot[sb][m][i];
       }
       if (sh.dead[0] || sh.dead[1]) return false;  // this one, or one for halos alone before
     }
