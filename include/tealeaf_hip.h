@@ -6,8 +6,8 @@
  * library owns every device buffer from tl_init() to tl_finalize(); no device
  * pointer crosses this boundary.  Every entry point returns 0 on success or a
  * TL_ERR_* code (message in tl_last_error()).  Entry points that return a
- * scalar through a pointer synchronise the library's stream; all others are
- * asynchronous and ordered on that stream.  Not thread safe.
+ * scalar through a pointer synchronise the library's stream, as do the solver
+ * loops; all others are asynchronous and ordered on that stream.  Not thread safe.
  *
  * Host arrays use the reference layout: x fastest, bounds
  * (x_min-halo : x_max+halo, y_min-halo : y_max+halo) with x_min = y_min = 1
@@ -261,8 +261,10 @@ int tl_jacobi_loop(tl_loop_state *st);
 int tl_loop_errors(int lo, int hi, double *err);
 
 /* Chebyshev iterations n_first..n_last with coefficient index
- * step_first.. (tea_solve.f90:265-279), queued without synchronisation;
- * the residual norm is computed only on the last one when want_norm != 0. */
+ * step_first.. (tea_solve.f90:265-279); the residual norm is computed only on
+ * the last one when want_norm != 0.  Without it the iterations are queued, except
+ * where they run with the mesh on the chip: the call then waits for them, since
+ * it reports a launch whose blocks waited in vain for one another. */
 int tl_cheby_run(const double *ch_alphas, const double *ch_betas, int step_first,
                  int count, int want_norm, double *norm);
 

@@ -1107,10 +1107,10 @@ int resident_cheby(const ResCheby &f, const double *alphas, const double *betas,
     if (rc == RES_REFUSED) return done == 0 ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
     if (rc) return -rc;
   }
-  if (want_norm) {
-    if ((rc = res_wait())) return -rc;
-    *norm = *a.norm;
-  }
+  // waited for without the norm too: a wait of a block that ran out is this
+  // call's error, and u must not pass on as its result
+  if ((rc = res_wait())) return -rc;
+  if (want_norm) *norm = *a.norm;
   return 1;
 }
 
