@@ -1362,8 +1362,12 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
                 b.rx, b.ry, st->n_first, st->n_last, 0,       lp,
                 st->rro, m.ctl, m.hrro, m.halpha, m.hbeta, m.herr,
                 cg_alphas || cg_betas ? s.hscal + HSCAL : nullptr, st->n_first};
-  const int ran = resident_cg<T>(
-      a, b.block ? TL_PREC_JAC_BLOCK : (b.diag ? TL_PREC_JAC_DIAG : TL_PREC_NONE), G.pitch, &res);
+  // On the chip p is formed from M^-1 r, or r without a preconditioner; where it
+  // is to come from a z that the loop does not form (PPCG active, no
+  // preconditioner) the passes run.
+  const bool own = b.cg_src == (b.diag || b.block ? b.z : b.r);
+  const int prec = b.block ? TL_PREC_JAC_BLOCK : b.diag ? TL_PREC_JAC_DIAG : TL_PREC_NONE;
+  const int ran = own ? resident_cg<T>(a, prec, G.pitch, &res) : 0;
   if (ran < 0) return -ran;
   if (!ran && (rc = drive(st->n_first, st->n_last, launch, tail, &res, m.ctl))) return rc;
   st->n_end = res.n_end;
