@@ -55,7 +55,8 @@ __device__ inline ResGhost<T> load_ghosts(const ResTile<T, R> &t, const ResGeo &
 // per CU); the preconditioner's fields are then read again in every
 // iteration, from the L2.  The splits are those at which the kernel spills no
 // vector register, and it must not: the compiler may place a spill inside a
-// region that only some lanes run, where it misses the others.
+// region that only some lanes run, where it misses the others.  The build
+// fails where one does (spills.awk).
 //
 // What bounds it: the two exchanges of an iteration, about 1.4 us each of 4.6
 // (512^2), and with 16 cells per lane the arithmetic (3 of 6 us).  Against
