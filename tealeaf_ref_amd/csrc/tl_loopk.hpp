@@ -1302,8 +1302,12 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   auto kw = w_kernel<T, V>(b, nt);
   const T *kx_or_dens = b.dens ? b.dens : b.Kx;
   // u is updated once for CG_DEFER iterations, whose directions go round as
-  // many buffers; with the block preconditioner in every iteration
-  const bool defer = !b.block && cg_defer();
+  // many buffers; with the block preconditioner in every iteration, and in a
+  // loop of one or two, where the pass that updates u at the end and the copy of
+  // p out of the spare buffer cost more than they save (one iteration at 4096^2
+  // 307 us for 373 put off, 2000^2 94 for 117, 8192^2 1410 for 1647, two at 4096^2
+  // 552 for 587; of three, put off 747 and 828 not)
+  const bool defer = !b.block && cg_defer() && st->n_last - st->n_first >= 2;
   auto kur0 = nt ? k_cg_ur<true, T, V, 0> : k_cg_ur<false, T, V, 0>;
   auto kur1 = nt ? k_cg_ur<true, T, V, 1> : k_cg_ur<false, T, V, 1>;
   auto kurN = nt ? k_cg_ur<true, T, V, CG_DEFER> : k_cg_ur<false, T, V, CG_DEFER>;
