@@ -589,9 +589,22 @@ int cheby_run_block(const double *ch_alphas, const double *ch_betas, int step_fi
   return 1;
 }
 
+// Two or three Chebyshev iterations are left to the two-iteration passes on
+// meshes under 40 million cells: a many-step pass of two reads its ghosts for no
+// more steps (us, many-step and two-iteration passes: 2 its at 1200^2 41 and 37,
+// 3000^2 166 and 129, 4096^2 291 and 236, 8192^2 1086 and 1128; 3 its at 4096^2 472
+// and 432, 8192^2 1883 and 1924; 4 its at 250^2 23 and 25, 4096^2 300 and 439).
+// TL_DEEP=2 (read on every call) takes the many-step passes for them too.
+bool cheby_pairs(int count) {
+  const State &s = S();
+  const char *e = getenv("TL_DEEP");
+  return count < 4 && (double)s.nx * (double)s.ny < 4e7 && !(e && atoi(e) > 1);
+}
+
 // Chebyshev iterations without a preconditioner: on the chip where the mesh
 // fits, else an even count of at most DEEP_MAX per pass after a single one where
-// `count` is odd (cheby_run_fused's contract).
+// `count` is odd (cheby_run_fused's contract; also 0 where the two-iteration
+// passes are the faster).
 int cheby_run_deep(const double *ch_alphas, const double *ch_betas, int step_first, int count,
                    int want_norm, double *norm) {
   State &s = S();
@@ -600,6 +613,7 @@ int cheby_run_deep(const double *ch_alphas, const double *ch_betas, int step_fir
   const int ran = resident_cheby(f, ch_alphas + step_first - 1, ch_betas + step_first - 1, count,
                                  s.pitch, want_norm, norm);
   if (ran) return ran;
+  if (cheby_pairs(count)) return 0;
   int done = 0, nparts = 0;
   if (count & 1) {
     const Geo G = geo(2 * BLOCK);
@@ -655,8 +669,10 @@ int cheby_run_fused(const double *ch_alphas, const double *ch_betas, int step_fi
   if (s.precond == TL_PREC_JAC_BLOCK)
     return s.reflective ? 0 : cheby_run_block(ch_alphas, ch_betas, step_first, count, want_norm,
                                               norm);
-  if (!s.reflective && s.precond == TL_PREC_NONE && count >= 2 && deep_fits())
-    return cheby_run_deep(ch_alphas, ch_betas, step_first, count, want_norm, norm);
+  if (!s.reflective && s.precond == TL_PREC_NONE && count >= 2 && deep_fits()) {
+    const int ran = cheby_run_deep(ch_alphas, ch_betas, step_first, count, want_norm, norm);
+    if (ran) return ran;
+  }
   const Geo G = geo_resident(2 * BLOCK, TL_CHEBY_PAIR_WAVES);
   const int nb = G.blocks < 0 ? -G.blocks : G.blocks;
   const int diag = s.precond == TL_PREC_JAC_DIAG;

@@ -1084,6 +1084,20 @@ int resident_jacobi(ResJacobi a, long pitch, Ctl *out) {
   }
 }
 
+// Runs too short for a launch of more than one block, cooperative and 8 us
+// dearer for it: under nine iterations, which the passes do sooner (us without the
+// norm, on the chip and by passes: 130^2 2 its 30 and 20, 6 its 36 and 28, 8 its 38
+// and 34; 512^2 31 and 22, 38 and 29, 41 and 35; 1400^2 4 its 58 and 45, 8 its 70
+// and 49), but for three and five on meshes of a million cells and more, where the
+// odd iteration takes a pass of its own (1024^2 42 and 42, 45 and 45; 1400^2 55
+// and 59, 62 and 64).  A row count asked for by TL_RES_ROWS is taken for any run.
+static bool cheby_short(int count, int blocks) {
+  const State &s = S();
+  if (blocks == 1 || count >= 9 || env_int("TL_RES_ROWS", 0) > 0) return false;
+  const bool large = (double)s.nx * (double)s.ny >= 1e6;
+  return !(large && (count == 3 || count == 5));
+}
+
 int resident_cheby(const ResCheby &f, const double *alphas, const double *betas, int count,
                    long pitch, bool want_norm, double *norm) {
   State &s = S();
@@ -1091,6 +1105,7 @@ int resident_cheby(const ResCheby &f, const double *alphas, const double *betas,
   const int R = res_rows(s.nx, s.ny, ROWS64, 6, CHEBY_COST);
   if (!R) return 0;
   ResGeo g = res_geo(R, pitch);
+  if (cheby_short(count, g.tx * g.ty)) return 0;
   ChebyArgs a;
   a.f = f;
   a.norm = res_host().norm;
