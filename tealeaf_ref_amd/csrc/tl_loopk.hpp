@@ -70,10 +70,11 @@ struct ResCg {
   double *hist;
   int n_base;
 };
-// 1: the loop has run and *out holds its result; 0: the mesh does not fit;
-// < 0: -(error code)
+// 1: the loop has run and *out holds its result; 0: the mesh does not fit, or a
+// later launch was refused, and `a` says where the passes go on (n_first, rro,
+// pin); < 0: -(error code)
 template <typename T>
-int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out);
+int resident_cg(ResCg<T> &a, int prec, long pitch, Ctl *out);
 // The same for the Jacobi iterations of tl_jacobi_loop, u read and written in
 // place.
 struct ResJacobi {
@@ -85,16 +86,17 @@ struct ResJacobi {
   Ctl *ctl;
   double *herr;
 };
-int resident_jacobi(ResJacobi a, long pitch, Ctl *out);
+int resident_jacobi(ResJacobi &a, long pitch, Ctl *out);
 // The same for `count` Chebyshev iterations without a preconditioner
-// (cheby_run_deep's contract); u and p read and written in place.
+// (cheby_run_deep's contract); u and p read and written in place.  Where it returns
+// 0, *ran iterations have run.
 struct ResCheby {
   double *u, *p, *w, *r;
   const double *u0, *Kx, *Ky;
   double rx, ry;
 };
 int resident_cheby(const ResCheby &a, const double *alphas, const double *betas, int count,
-                   long pitch, bool want_norm, double *norm);
+                   long pitch, bool want_norm, double *norm, int *ran);
 // The same for PPCG's outer iterations and their inner steps; the pointers as in
 // run_ppcg_loop, r_store written only.
 template <typename T>
@@ -109,7 +111,7 @@ struct ResPpcg {
   double *herr;
 };
 template <typename T>
-int resident_ppcg(ResPpcg<T> a, int prec, const double *alphas, const double *betas, long pitch,
+int resident_ppcg(ResPpcg<T> &a, int prec, const double *alphas, const double *betas, long pitch,
                   Ctl *out);
 constexpr int RES_PAUSED = 0;  // reason of a launch that stopped for the host only
 
@@ -1313,9 +1315,13 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   auto kurN = nt ? k_cg_ur<true, T, V, CG_DEFER> : k_cg_ur<false, T, V, CG_DEFER>;
   auto kub = nt ? k_cg_ur_blk<true, T, V> : k_cg_ur_blk<false, T, V>;
   const int c0 = *b.pcur;
+  // where the passes begin: after the iterations that have run on the chip
+  int n0 = st->n_first;
+  double rro0 = st->rro;
+  const T *pin0 = pin_first ? pin_first : b.p[c0];
   T *ring[CG_DEFER] = {b.p[c0], b.p[1 - c0], b.spare[0], b.spare[1]};
   const int turn = defer ? CG_DEFER : 2;
-  // the direction entering iteration i of this call (from 0), and the one it makes
+  // the direction entering iteration i of the passes (from 0), and the one it makes
   auto p_in = [&](int i) { return ring[i % turn]; };
   auto p_out = [&](int i) { return ring[(i + 1) % turn]; };
   LoopParams lp;
@@ -1324,12 +1330,12 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   lp.check_switch = st->check_switch;
   lp.presteps = st->presteps;
   auto launch = [&](int n, bool first) -> int {
-    const int i = n - st->n_first;
-    const T *pin = (first && pin_first) ? pin_first : p_in(i);
+    const int i = n - n0;
+    const T *pin = first ? pin0 : p_in(i);
     hipEvent_t ev;
     prof_arm(0, &ev);
     klaunch(kw, dim3(nb), dim3(BLOCK), G, n, first ? 1 : 0, 0, lp,
-            st->rro, b.cg_src, pin, p_out(i), kx_or_dens, b.Ky, b.w, b.rx, b.ry,
+            rro0, b.cg_src, pin, p_out(i), kx_or_dens, b.Ky, b.w, b.rx, b.ry,
             m.part(P2), nb, m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1, b.recip);
     prof_end(0, ev);
     prof_arm(1, &ev);
@@ -1353,15 +1359,15 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
     return TL_OK;
   };
   auto tail = [&](int n) -> int {
-    const int i = n - st->n_first;
-    hipLaunchKernelGGL(kw, dim3(nb), dim3(BLOCK), 0, s.stream, G, n, 0, 1, lp, st->rro, b.cg_src,
+    const int i = n - n0;
+    hipLaunchKernelGGL(kw, dim3(nb), dim3(BLOCK), 0, s.stream, G, n, 0, 1, lp, rro0, b.cg_src,
                        (const T *)p_in(i), p_out(i), kx_or_dens, b.Ky, b.w, b.rx, b.ry, m.part(P2), nb,
                        m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1, b.recip);
     TL_HIP(hipGetLastError());
     return TL_OK;
   };
   Ctl res;
-  ResCg<T> a = {b.u,  b.r,  b.p[c0], b.w,         b.z,        pin_first ? pin_first : b.p[c0],
+  ResCg<T> a = {b.u,  b.r,  b.p[c0], b.w,         b.z,        pin0,
                 b.Mi, b.Di, b.cp,    b.bfp,       b.Kx,       b.Ky,
                 b.rx, b.ry, st->n_first, st->n_last, 0,       lp,
                 st->rro, m.ctl, m.hrro, m.halpha, m.hbeta, m.herr,
@@ -1373,7 +1379,12 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
   const int prec = b.block ? TL_PREC_JAC_BLOCK : b.diag ? TL_PREC_JAC_DIAG : TL_PREC_NONE;
   const int ran = own ? resident_cg<T>(a, prec, G.pitch, &res) : 0;
   if (ran < 0) return -ran;
-  if (!ran && (rc = drive(st->n_first, st->n_last, launch, tail, &res, m.ctl))) return rc;
+  if (!ran) {
+    n0 = a.n_first;
+    rro0 = a.rro;
+    pin0 = a.pin;
+    if ((rc = drive(n0, st->n_last, launch, tail, &res, m.ctl))) return rc;
+  }
   st->n_end = res.n_end;
   st->reason = res.reason;
   st->error = res.error;
@@ -1384,13 +1395,13 @@ int run_cg_loop(const LoopBufs<T> &b, tl_loop_state *st, double *cg_alphas, doub
     // non-finite p.w was found
     const bool at_end = res.reason == TL_LOOP_SWITCH ||
                         (res.reason == TL_LOOP_NONFINITE && res.stop == STOP_UPDATE);
-    const int done = res.n_end - st->n_first + (at_end ? 0 : 1);
+    const int done = res.n_end - n0 + (at_end ? 0 : 1);
     const int left = defer ? done % CG_DEFER : 0;
     if (left > 0) {
       CgDefer<T> d = {};
       for (int q = 0; q < left; ++q) d.p[q] = p_out(done - left + q);
       hipLaunchKernelGGL((k_cg_u<T, V>), dim3(nb), dim3(BLOCK), 0, s.stream, G,
-                         st->n_first + done - 1, left, b.u, d, m.halpha, (const Ctl *)nullptr);
+                         n0 + done - 1, left, b.u, d, m.halpha, (const Ctl *)nullptr);
       TL_HIP(hipGetLastError());
     }
     // the launch that stopped the loop applied the last p update
@@ -1435,6 +1446,9 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   const T *kx_or_dens = b.dens ? b.dens : b.Kx;
   auto kur = nt ? k_pp_ur<true, T, V> : k_pp_ur<false, T, V>;
   const int c0 = *b.pcur;
+  // where the passes begin: after the iterations that have run on the chip
+  int n0 = st->n_first;
+  const T *pin0 = pin_first ? pin_first : b.p[c0];
   int sd = *b.sdcur;
   LoopParams lp;
   lp.eps_abs = st->eps_abs;
@@ -1444,7 +1458,7 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   const T theta_r = (T)(1.0 / theta);
   Ctl res;
   if (deep_fits()) {
-    const ResPpcg<T> a = {b.u,  b.r,   b.r_store, b.p[c0], b.z, pin_first ? pin_first : b.p[c0],
+    ResPpcg<T> a = {b.u,  b.r,   b.r_store, b.p[c0], b.z, pin0,
                           b.Mi, b.Di,  b.cp,      b.bfp,   b.Kx, b.Ky,
                           b.rx, b.ry,  theta_r,   st->n_first, st->n_last, 0,
                           inner, st->eps_abs, rro_first, m.ctl, m.herr};
@@ -1461,6 +1475,9 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
       if (inner_iters) *inner_iters += (res.n_end - st->n_first + 1) * inner;
       return TL_OK;
     }
+    n0 = a.n_first;
+    rro_first = a.rro;
+    pin0 = a.pin;
   }
   // Row directions: the w pass walks d, the update -d, the sweep passes
   // alternate from d; with an odd number of sweep passes the next outer
@@ -1475,24 +1492,24 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
   // those.
   T *ring[CG_DEFER] = {b.p[c0], b.p[1 - c0], b.utemp, b.spare[1]};
   const int turn = !deep ? 2 : deep_passes(inner) == 1 && b.spare[1] ? 4 : 3;
-  // the direction entering iteration i of this call (from 0), and the one it makes
+  // the direction entering iteration i of the passes (from 0), and the one it makes
   auto p_in = [&](int i) { return ring[i % turn]; };
   auto p_out = [&](int i) { return ring[(i + 1) % turn]; };
-  // u += alpha p of the `count` iterations of this call before iteration i
+  // u += alpha p of the `count` iterations of the passes before iteration i
   auto flush_u = [&](int i, int count, const Ctl *ctl) -> int {
     CgDefer<T> d = {};
     for (int q = 0; q < count; ++q) d.p[q] = p_out(i - count + q);
     hipEvent_t ev;
     prof_arm(6, &ev);
-    klaunch(&k_cg_u<T, V>, dim3(nb), dim3(BLOCK), G, st->n_first + i - 1, count, b.u, d, m.halpha,
+    klaunch(&k_cg_u<T, V>, dim3(nb), dim3(BLOCK), G, n0 + i - 1, count, b.u, d, m.halpha,
             ctl);
     prof_end(6, ev);
     TL_HIP(hipGetLastError());
     return TL_OK;
   };
   auto launch = [&](int n, bool first) -> int {
-    const int i = n - st->n_first;
-    const T *pin = (first && pin_first) ? pin_first : p_in(i);
+    const int i = n - n0;
+    const T *pin = first ? pin0 : p_in(i);
     const int d = (!deep && (passes & 1) && (i & 1)) ? -1 : 1;
     hipEvent_t ev;
     prof_arm(5, &ev);
@@ -1527,20 +1544,20 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
     return queue_sweeps<T, V>(b, alphas, betas, inner, theta_r, 1, m.ctl, m, sd, rt_cur, d);
   };
   auto tail = [&](int n) -> int {
-    const int i = n - st->n_first;
+    const int i = n - n0;
     hipLaunchKernelGGL(kw, dim3(nb), dim3(BLOCK), 0, s.stream, G, n, 0, 1, lp, rro_first, b.z,
                        (const T *)p_in(i), p_out(i), kx_or_dens, b.Ky, b.w, b.rx, b.ry, m.part(P3), nzr,
                        m.part(P1), m.ctl, m.hrro, m.hbeta, m.herr, 1, b.recip);
     TL_HIP(hipGetLastError());
     return TL_OK;
   };
-  if ((rc = drive(st->n_first, st->n_last, launch, tail, &res, m.ctl))) return rc;
+  if ((rc = drive(n0, st->n_last, launch, tail, &res, m.ctl))) return rc;
   st->n_end = res.n_end;
   st->reason = res.reason;
   st->error = res.error;
   st->rro = res.rro;
   st->old_error = res.old_error;
-  const int executed = res.n_end - st->n_first + 1;  // outer iterations that ran
+  const int executed = res.n_end - n0 + 1;  // outer iterations of the passes
   if (deep) {
     // updates that ran: not that of an iteration with a non-finite p.w
     const int done =
@@ -1563,7 +1580,7 @@ int run_ppcg_loop(const LoopBufs<T> &b, tl_loop_state *st, const double *alphas,
     *b.sdcur = *b.sdcur ^ ((executed * swaps) & 1);
   }
   if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("PPCG", res.n_end);
-  if (inner_iters) *inner_iters += executed * inner;
+  if (inner_iters) *inner_iters += (res.n_end - st->n_first + 1) * inner;
   return TL_OK;
 }
 

@@ -610,9 +610,12 @@ int cheby_run_deep(const double *ch_alphas, const double *ch_betas, int step_fir
   State &s = S();
   const ResCheby f = {s.u[s.ucur].p11, s.p[s.pcur].p11, s.w.p11, s.r.p11, s.u0.p11,
                       s.Kx.p11,        s.Ky.p11,        s.rx,    s.ry};
+  int chip;
   const int ran = resident_cheby(f, ch_alphas + step_first - 1, ch_betas + step_first - 1, count,
-                                 s.pitch, want_norm, norm);
+                                 s.pitch, want_norm, norm, &chip);
   if (ran) return ran;
+  if (chip)  // a launch was refused: the rest by passes
+    return cheby_run_fused(ch_alphas, ch_betas, step_first + chip, count - chip, want_norm, norm);
   if (cheby_pairs(count)) return 0;
   int done = 0, nparts = 0;
   if (count & 1) {
@@ -1176,31 +1179,15 @@ extern "C" int tl_loop_errors(int lo, int hi, double *err) {
   return copy_hist(err, loop_mem().herr, lo, hi);
 }
 
-extern "C" int tl_jacobi_loop(tl_loop_state *st) {
-  TL_REQUIRE_INIT();
-  int rc = check_state(st);
-  if (rc) return rc;
-  if ((rc = ensure_loop_buffers(st->n_last))) return rc;
+// Jacobi iterations by passes: the vector walk where every face is external
+// (reflective faces read zero outside the mesh, as the reference reads the
+// never-written halo of un), two iterations a pass unless that is off; the
+// per-cell walk otherwise.
+static int jacobi_loop_passes(tl_loop_state *st) {
   State &s = S();
-  // the vector walk where every face is external (reflective faces read zero
-  // outside the mesh, as the reference reads the never-written halo of un);
-  // the per-cell walk otherwise
+  int rc;
   const bool vec = s.zb_all;
-  if (vec) {
-    const ResJacobi a = {s.u[s.ucur].p11, s.u0.p11,  s.Kx.p11, s.Ky.p11,    s.rx,
-                         s.ry,            st->n_first, st->n_last, 0, st->eps_abs,
-                         (Ctl *)s.ctl,    loop_mem().herr};
-    Ctl res;
-    const int ran = resident_jacobi(a, s.pitch, &res);
-    if (ran < 0) return -ran;
-    if (ran) {
-      st->n_end = res.n_end;
-      st->reason = res.reason;
-      st->error = res.error;
-      return res.reason == TL_LOOP_NONFINITE ? nonfinite_fail("Jacobi", res.n_end) : TL_OK;
-    }
-    if (sweep_pairs()) return jacobi_loop_pairs(st);
-  }
+  if (vec && sweep_pairs()) return jacobi_loop_pairs(st);
   const Geo G = vec ? geo(2 * BLOCK) : geo(BLOCK);
   const int nb = G.blocks < 0 ? -G.blocks : G.blocks;
   const int u0c = s.ucur;
@@ -1244,4 +1231,30 @@ extern "C" int tl_jacobi_loop(tl_loop_state *st) {
   if (res.reason == TL_LOOP_NONFINITE) return nonfinite_fail("Jacobi", res.n_end);
   s.ucur = u0c ^ ((res.n_end - st->n_first + 1) & 1);
   return TL_OK;
+}
+
+extern "C" int tl_jacobi_loop(tl_loop_state *st) {
+  TL_REQUIRE_INIT();
+  int rc = check_state(st);
+  if (rc) return rc;
+  if ((rc = ensure_loop_buffers(st->n_last))) return rc;
+  State &s = S();
+  const int n_first = st->n_first;
+  if (s.zb_all) {
+    ResJacobi a = {s.u[s.ucur].p11, s.u0.p11,  s.Kx.p11,   s.Ky.p11, s.rx, s.ry, n_first,
+                   st->n_last,      0,         st->eps_abs, (Ctl *)s.ctl, loop_mem().herr};
+    Ctl res;
+    const int ran = resident_jacobi(a, s.pitch, &res);
+    if (ran < 0) return -ran;
+    if (ran) {
+      st->n_end = res.n_end;
+      st->reason = res.reason;
+      st->error = res.error;
+      return res.reason == TL_LOOP_NONFINITE ? nonfinite_fail("Jacobi", res.n_end) : TL_OK;
+    }
+    st->n_first = a.n_first;  // the passes begin where the chip left off
+  }
+  rc = jacobi_loop_passes(st);
+  st->n_first = n_first;
+  return rc;
 }

@@ -919,9 +919,11 @@ constexpr int RES_REFUSED = -1;
 // One launch of a kernel over a's mesh: cooperatively, so that every block is
 // resident when the first one waits (a single block waits for none).  The
 // runtime refuses cooperative launches while another process holds the
-// device's; the chunk's loops then run the pass kernels from there on.
+// device's; the chunk's loops then run the pass kernels from there on, also in the
+// middle of a loop, whose launches leave the fields as the passes do.
+// `launch`: its number in the loop (TL_RES_REFUSE takes that one as refused).
 template <typename A>
-int res_launch(void (*k)(ResGeo, A), ResGeo g, A a, size_t lds) {
+int res_launch(int launch, void (*k)(ResGeo, A), ResGeo g, A a, size_t lds) {
   State &s = S();
   const int nb = g.tx * g.ty;
   if (nb == 1) {
@@ -930,7 +932,8 @@ int res_launch(void (*k)(ResGeo, A), ResGeo g, A a, size_t lds) {
     return TL_OK;
   }
   void *args[] = {&g, &a};
-  if (hipLaunchCooperativeKernel((const void *)k, dim3(nb), dim3(RES_THREADS), args,
+  if (launch != env_int("TL_RES_REFUSE", -1) &&
+      hipLaunchCooperativeKernel((const void *)k, dim3(nb), dim3(RES_THREADS), args,
                                  (unsigned)lds, s.stream) == hipSuccess)
     return TL_OK;
   (void)hipGetLastError();
@@ -983,13 +986,13 @@ int res_chunk() {
 }
 
 template <typename T, int R, int PREC>
-int cg_launch(const ResGeo &g, const ResCg<T> &a) {
-  return res_launch(&k_res_cg<T, R, PREC>, g, a, CgPlan<T, R, PREC>::BYTES);
+int cg_launch(int launch, const ResGeo &g, const ResCg<T> &a) {
+  return res_launch(launch, &k_res_cg<T, R, PREC>, g, a, CgPlan<T, R, PREC>::BYTES);
 }
 
 template <typename T>
-int cg_dispatch(int R, int prec, const ResGeo &g, const ResCg<T> &a) {
-#define CASE(RR, PP)   if (R == RR && prec == PP) return cg_launch<T, RR, PP>(g, a)
+int cg_dispatch(int launch, int R, int prec, const ResGeo &g, const ResCg<T> &a) {
+#define CASE(RR, PP)   if (R == RR && prec == PP) return cg_launch<T, RR, PP>(launch, g, a)
   CASE(1, TL_PREC_NONE);
   CASE(2, TL_PREC_NONE);
   CASE(3, TL_PREC_NONE);
@@ -1029,22 +1032,22 @@ long resident_words(int nx, int ny) {
 }
 
 template <typename T>
-int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out) {
+int resident_cg(ResCg<T> &a, int prec, long pitch, Ctl *out) {
   State &s = S();
   if (!resident_on()) return 0;
   const int R = rows_for<T>(s.nx, s.ny, prec);
   if (!R) return 0;
   ResGeo g = res_geo(R, pitch);
   a.ctl = res_host().ctl;
-  const int n_first = a.n_first, chunk = res_chunk();
-  for (;;) {
+  const int chunk = res_chunk();
+  for (int k = 0;; ++k) {
     const long left = (long)a.n_last - a.n_first + 1;
     const long run = left < chunk ? left : chunk;
     a.n_pause = (int)(a.n_first + run - 1);
     int rc;
     if ((rc = res_tags(2 * run, &g.epoch))) return -rc;
-    rc = cg_dispatch<T>(R, prec, g, a);
-    if (rc == RES_REFUSED) return a.n_first == n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
+    rc = cg_dispatch<T>(k, R, prec, g, a);
+    if (rc == RES_REFUSED) return 0;
     if (rc || (rc = res_wait())) return -rc;
     *out = *a.ctl;
     if (out->reason != RES_PAUSED) return 1;
@@ -1054,10 +1057,10 @@ int resident_cg(ResCg<T> a, int prec, long pitch, Ctl *out) {
     a.pin = a.p;
   }
 }
-template int resident_cg<double>(ResCg<double>, int, long, Ctl *);
-template int resident_cg<float>(ResCg<float>, int, long, Ctl *);
+template int resident_cg<double>(ResCg<double> &, int, long, Ctl *);
+template int resident_cg<float>(ResCg<float> &, int, long, Ctl *);
 
-int resident_jacobi(ResJacobi a, long pitch, Ctl *out) {
+int resident_jacobi(ResJacobi &a, long pitch, Ctl *out) {
   State &s = S();
   if (!resident_on()) return 0;
   static constexpr int ROWS[] = {1, 2, 3, 4, 5, 6, 8};
@@ -1065,18 +1068,18 @@ int resident_jacobi(ResJacobi a, long pitch, Ctl *out) {
   if (!R) return 0;
   ResGeo g = res_geo(R, pitch);
   a.ctl = res_host().ctl;
-  const int n_first = a.n_first, chunk = res_chunk();
-  for (;;) {
+  const int chunk = res_chunk();
+  for (int k = 0;; ++k) {
     const long left = (long)a.n_last - a.n_first + 1;
     const long run = left < chunk ? left : chunk;
     a.n_pause = (int)(a.n_first + run - 1);
     int rc;
     if ((rc = res_tags(run, &g.epoch))) return -rc;
-#define CASE(RR) R == RR ? res_launch(&k_res_jacobi<RR>, g, a, JacobiPlan<RR>::BYTES)
+#define CASE(RR) R == RR ? res_launch(k, &k_res_jacobi<RR>, g, a, JacobiPlan<RR>::BYTES)
     rc = CASE(1) : CASE(2) : CASE(3) : CASE(4) : CASE(5) : CASE(6)
-         : res_launch(&k_res_jacobi<8>, g, a, JacobiPlan<8>::BYTES);
+         : res_launch(k, &k_res_jacobi<8>, g, a, JacobiPlan<8>::BYTES);
 #undef CASE
-    if (rc == RES_REFUSED) return a.n_first == n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
+    if (rc == RES_REFUSED) return 0;
     if (rc || (rc = res_wait())) return -rc;
     *out = *a.ctl;
     if (out->reason != RES_PAUSED) return 1;
@@ -1099,8 +1102,9 @@ static bool cheby_short(int count, int blocks) {
 }
 
 int resident_cheby(const ResCheby &f, const double *alphas, const double *betas, int count,
-                   long pitch, bool want_norm, double *norm) {
+                   long pitch, bool want_norm, double *norm, int *ran) {
   State &s = S();
+  *ran = 0;
   if (!resident_on()) return 0;
   const int R = res_rows(s.nx, s.ny, ROWS64, 6, CHEBY_COST);
   if (!R) return 0;
@@ -1110,17 +1114,21 @@ int resident_cheby(const ResCheby &f, const double *alphas, const double *betas,
   a.f = f;
   a.norm = res_host().norm;
   int rc;
-  for (int done = 0; done < count; done += a.count) {
+  for (int done = 0, k = 0; done < count; done += a.count, ++k) {
     a.count = count - done < RES_CHEBY_STEPS ? count - done : RES_CHEBY_STEPS;
     a.last = done + a.count == count;
     memcpy(a.a, alphas + done, sizeof(double) * a.count);
     memcpy(a.b, betas + done, sizeof(double) * a.count);
     if ((rc = res_tags(a.count + 1, &g.epoch))) return -rc;
-#define CASE(RR) R == RR ? res_launch(&k_res_cheby<RR>, g, a, ChebyPlan<RR>::BYTES)
+#define CASE(RR) R == RR ? res_launch(k, &k_res_cheby<RR>, g, a, ChebyPlan<RR>::BYTES)
     rc = CASE(1) : CASE(2) : CASE(3) : CASE(4) : CASE(6)
-         : res_launch(&k_res_cheby<8>, g, a, ChebyPlan<8>::BYTES);
+         : res_launch(k, &k_res_cheby<8>, g, a, ChebyPlan<8>::BYTES);
 #undef CASE
-    if (rc == RES_REFUSED) return done == 0 ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
+    if (rc == RES_REFUSED) {
+      *ran = done;
+      if (done && (rc = res_wait())) return -rc;
+      return 0;
+    }
     if (rc) return -rc;
   }
   // waited for without the norm too: a wait of a block that ran out is this
@@ -1131,7 +1139,7 @@ int resident_cheby(const ResCheby &f, const double *alphas, const double *betas,
 }
 
 template <typename T>
-int resident_ppcg(ResPpcg<T> f, int prec, const double *alphas, const double *betas, long pitch,
+int resident_ppcg(ResPpcg<T> &f, int prec, const double *alphas, const double *betas, long pitch,
                   Ctl *out) {
   State &s = S();
   if (!resident_on() || f.inner < 1 || f.inner > RES_PPCG_STEPS) return 0;
@@ -1150,13 +1158,13 @@ int resident_ppcg(ResPpcg<T> f, int prec, const double *alphas, const double *be
     a.b[i] = i < f.inner ? (T)betas[i] : T(0);
   }
   const int chunk = res_chunk();
-  for (;;) {
+  for (int k = 0;; ++k) {
     const long left = (long)f.n_last - a.f.n_first + 1;
     const long run = left < chunk ? left : chunk;
     a.f.n_pause = (int)(a.f.n_first + run - 1);
     int rc;
     if ((rc = res_tags((f.inner + 2L) * run, &g.epoch))) return -rc;
-#define RUN(RR, PP) res_launch(&k_res_ppcg<T, RR, PP>, g, a, PpcgPlan<T, RR>::BYTES)
+#define RUN(RR, PP) res_launch(k, &k_res_ppcg<T, RR, PP>, g, a, PpcgPlan<T, RR>::BYTES)
 #define CASE(RR, PP) R == RR ? RUN(RR, PP)
     constexpr int NONE = TL_PREC_NONE, DIAG = TL_PREC_JAC_DIAG, BLK = TL_PREC_JAC_BLOCK;
     if constexpr (sizeof(T) == 4)
@@ -1170,8 +1178,10 @@ int resident_ppcg(ResPpcg<T> f, int prec, const double *alphas, const double *be
       rc = CASE(1, NONE) : CASE(2, NONE) : CASE(3, NONE) : CASE(4, NONE) : RUN(6, NONE);
 #undef CASE
 #undef RUN
-    if (rc == RES_REFUSED)
-      return a.f.n_first == f.n_first ? 0 : -fail(TL_ERR_HIP, "cooperative launch");
+    if (rc == RES_REFUSED) {
+      f = a.f;
+      return 0;
+    }
     if (rc || (rc = res_wait())) return -rc;
     *out = *a.f.ctl;
     // the sum z.r enters the next iteration; the control block has no other
@@ -1185,9 +1195,9 @@ int resident_ppcg(ResPpcg<T> f, int prec, const double *alphas, const double *be
     a.f.pin = a.f.p;
   }
 }
-template int resident_ppcg<double>(ResPpcg<double>, int, const double *, const double *, long,
+template int resident_ppcg<double>(ResPpcg<double> &, int, const double *, const double *, long,
                                    Ctl *);
-template int resident_ppcg<float>(ResPpcg<float>, int, const double *, const double *, long,
+template int resident_ppcg<float>(ResPpcg<float> &, int, const double *, const double *, long,
                                   Ctl *);
 
 }  // namespace tl
