@@ -11,11 +11,8 @@
 
 namespace tl {
 
-// The ring of up to eight stages holds the diagonal too (8 rows x 4 fields x
-// 1 KB per wave, 128 KB of the CU's 160 KB for four waves); with ten stages it
-// does not fit, and every stage forms it from the faces again.
-constexpr bool deep_cheby_di(int stages) { return stages <= 10; }
-constexpr int deep_cheby_fields(int stages) { return deep_cheby_di(stages) ? 4 : 3; }
+// Fields of the ring: kx, ky (times rx, ry), u0 and the diagonal.
+constexpr int DEEP_CHEBY_FIELDS = 4;
 
 struct DeepCheby {
   const double *u, *p, *u0, *Kx, *Ky;
@@ -28,15 +25,15 @@ struct DeepCheby {
 namespace {
 
 // LAST: the last pass of a run also stores w and r and the partials of r.r.
-// At 4096^2 ten iterations take 217 us in one pass (270 with w and r), eight
-// 200, against 166 us for every two before: 21.7 us an iteration instead of 83.
-// Bound, as k_deep_ppcg, by the instructions of its one wave per SIMD, with
-// memory close behind (1.0 GB at 4.7 TB/s).
+// At 4096^2 ten iterations take 207 us in one pass (268 with w and r), against 166
+// us for every two before: 20.7 us an iteration instead of 83.  Bound, as
+// k_deep_ppcg, by the instructions of its one wave per SIMD, with memory close
+// behind (1.05 GB at 5.1 TB/s).  The ring of ten stages takes the CU's 160 KB: 10
+// rows x 4 fields x 1 KB for each of four waves.
 template <int STAGES, int LAST>
 __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double> co,
                                                       DeepCheby a) {
-  constexpr int V = 2, NF = deep_cheby_fields(STAGES);
-  constexpr bool DI = deep_cheby_di(STAGES);
+  constexpr int V = 2, NF = DEEP_CHEBY_FIELDS;
   typedef double T;
   typedef typename dev::Vec<T, V>::type VT;
   extern __shared__ char dyn[];
@@ -94,18 +91,13 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
       VT kyu = in.ky;
       Faces f = {kx1, ky1, VT(0), u01};
       T kxr = dev::from_above(f.kx[0]);
-      auto diagonal = [&](const Faces &k, VT up, T right) {
-        VT d;
 #pragma unroll
-        for (int e = 0; e < V; ++e)
-          d[e] = T(1) + (up[e] + k.ky[e]) + (dev::vec_right<T, V>(k.kx, e, right) + k.kx[e]);
-        return d;
-      };
-      f.di = diagonal(f, kyu, kxr);
+      for (int e = 0; e < V; ++e)
+        f.di[e] = T(1) + (kyu[e] + f.ky[e]) + (dev::vec_right<T, V>(f.kx, e, kxr) + f.kx[e]);
       at(slot, 0) = f.kx;
       at(slot, 1) = f.ky;
       at(slot, 2) = f.u0;
-      if (DI) at(slot, 3) = f.di;
+      at(slot, 3) = f.di;
       VT ahead = in.u, p = ps[0], w = VT(0), r = VT(0);
       ps[0] = in.p;
 #pragma unroll
@@ -114,13 +106,12 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
         Faces nf = f;
         if (s + 1 < STAGES) {
           const int o = (slot - s - 1 + STAGES) % STAGES;
-          nf = {at(o, 0), at(o, 1), DI ? at(o, DI ? 3 : 0) : VT(0), at(o, 2)};
+          nf = {at(o, 0), at(o, 1), at(o, 3), at(o, 2)};
         }
         __builtin_amdgcn_sched_barrier(0);
         const VT c = centre[s];
         const T lo = dev::from_below(c[V - 1]), hi = dev::from_above(c[0]);
         if (s > 0) kxr = dev::from_above(f.kx[0]);
-        if (!DI && s > 0) f.di = diagonal(f, kyu, kxr);
 #pragma unroll
         for (int e = 0; e < V; ++e) {
           const T l = dev::vec_left<T, V>(c, e, lo), rr = dev::vec_right<T, V>(c, e, hi);
@@ -194,7 +185,7 @@ __global__ __launch_bounds__(BLOCK) void k_deep_cheby(DeepGeo g, DeepCoef<double
 }
 
 constexpr size_t deep_cheby_lds(int stages) {
-  return (size_t)(BLOCK / WAVE) * stages * deep_cheby_fields(stages) * WAVE * 16;
+  return (size_t)(BLOCK / WAVE) * stages * DEEP_CHEBY_FIELDS * WAVE * 16;
 }
 
 template <int STAGES>
