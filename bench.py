@@ -7,7 +7,9 @@ dt 0.004, a field summary every step.  A "step" is one pass of the reference's
 diffuse() loop body: timestep + tea_leaf() solve + field_summary, run by the
 native host with every field resident in HBM.
 
-Prints one JSON line.  `value` is seconds per timestep (lower is better);
+Prints one JSON line of under 4 kB, short enough to be read from the end of a log;
+--record writes the whole record, of which it is the headline.  `value` is
+seconds per timestep (lower is better);
 `precision_comparison` times FP64 CG / PPCG against the FP32-inner,
 FP64-refined forms at a relative residual of 1e-10 on the inverse-density
 deck;
@@ -21,6 +23,7 @@ the same per-kernel rates, on algorithmic and on counter-measured bytes;
 host cores on a bounded sample of the same deck.
 """
 import argparse
+import contextlib
 import json
 import os
 import re
@@ -93,8 +96,75 @@ def measured_traffic(kernel, cells, profile="cg_fp64_{n}_hbm_traffic.md"):
     return float(m.group(1)) if m else None
 
 
+_stderr = None  # where log() writes while the host's lines are set aside
+
+
 def log(*a):
-    print(*a, file=sys.stderr, flush=True)
+    print(*a, file=_stderr or sys.stderr, flush=True)
+
+
+@contextlib.contextmanager
+def host_lines_aside():
+    """The native host prints a step's lines to file descriptor 2, as the reference
+    does; they go to a temporary file, so that what is logged here stays short.
+    After a failure the file's end is shown."""
+    global _stderr
+    sys.stderr.flush()
+    saved = os.dup(2)
+    with tempfile.TemporaryFile() as aside, os.fdopen(saved, "w") as err:
+        os.dup2(aside.fileno(), 2)
+        _stderr = err
+        try:
+            yield
+        except BaseException:
+            aside.seek(max(0, aside.seek(0, os.SEEK_END) - 2000))
+            log(aside.read().decode(errors="replace"))
+            raise
+        finally:
+            _stderr = None
+            sys.stderr.flush()
+            os.dup2(err.fileno(), 2)
+
+
+def brief(rec, digits=6):
+    """The plain values of a record, its numbers to `digits` digits."""
+    def one(v):
+        return float(f"{v:.{digits}g}") if isinstance(v, float) else v
+    return {k: one(v) for k, v in rec.items() if isinstance(v, (int, float, bool)) or v is None}
+
+
+def headline(out):
+    """The line that is printed: every key of the record up to `roofline` as it is,
+    and of the longer sections the times and errors alone.  The whole record
+    (per-kernel rates, iteration counts, hosts: some 20 kB) goes to --record."""
+    line = {k: v for k, v in out.items() if not isinstance(v, (dict, list)) or k == "config"}
+    line["roofline"] = out["roofline"]
+    if "solvers" in out:
+        line["solvers"] = {
+            k: {q: v for q, v in brief(r).items()
+                if q in ("s_per_step", "iterations_per_step", "step_measured_frac")}
+            for k, r in out["solvers"].items()}
+    for k in ("small", "achievable_hbm"):
+        if k in out:
+            line[k] = brief(out[k])
+    if "precision_comparison" in out:
+        line["precision_comparison"] = [
+            {"workload": c["workload"].split(",")[0],
+             **{k: [q["s_per_step"], q["true_rel_residual"]]
+                for k, q in ((k, brief(r)) for k, r in c["runs"].items())},
+             **{k: v for k, v in brief(c).items()}} for c in out["precision_comparison"]]
+    for k in ("adjoint", "adjoint_large"):
+        if k in out:
+            line[k] = {
+                "workload": ",".join(out[k]["workload"].split(",")[:2]), **brief(out[k]),
+                **{prec: {q: v for q, v in brief(out[k][prec]).items()
+                          if q in ("J", "forward_s_per_step", "forward_backward_s_per_step",
+                                   "fd_max_rel_err", "vs_saved_gradient_rel_l2_window")}
+                   for prec in ("fp64", "mixed") if prec in out[k]}}
+    if "cpu_baseline" in out:
+        line["cpu_baseline"] = {k: v for k, v in out["cpu_baseline"].items()
+                                if not isinstance(v, dict)}
+    return line
 
 
 def gpu_run(cells, solver, steps, warmup, workdir, **deck_kw):
@@ -287,7 +357,7 @@ def solver_runs(cells, steps, warmup):
             rec["step_measured_frac"] = rec["step_measured_gbs"] / PEAK_HBM_GBS
             rec["step_time_covered"] = covered_ms * 1e-3 / elapsed
             rec["work_launches"] = {classes[c][0]: v for c, v in counts.items() if v}
-        log(f"[bench] {cells}^2 {solver}: {rec}")
+        log(f"[bench] {cells}^2 {solver}: {brief(rec)}")
         out[solver] = rec
     return out
 
@@ -309,7 +379,7 @@ def stream_bandwidth(n=1 << 28, reps=10):
     out = {"elements": n, "dtype": "f64", "kernels": "hand-written HIP (tl_hbm_stream)",
            "copy_gbs": cp.value, "triad_gbs": tr.value,
            "copy_frac": cp.value / PEAK_HBM_GBS, "triad_frac": tr.value / PEAK_HBM_GBS}
-    log(f"[bench] stream bandwidth: {out}")
+    log(f"[bench] stream bandwidth: {brief(out)}")
     return out
 
 
@@ -324,7 +394,7 @@ def small_run(steps=10):
     rec = {"workload": "512x512 FP64 CG, seeded deck (3 rectangles, seed 1), tl_eps 1e-15",
            "s_per_step": elapsed / steps, "iterations_per_step": its / steps,
            "us_per_iteration": elapsed / its * 1e6}
-    log(f"[bench] small: {rec}")
+    log(f"[bench] small: {brief(rec)}")
     return rec
 
 
@@ -523,7 +593,7 @@ def precision_comparison(cells, inner_steps=10, target=1e-10, later_step=False):
             rec["u_rel_err_vs_fp64_cg"] = float(np.max(np.abs(u - ref_u)) / np.max(np.abs(ref_u)))
             rec["summary_rel_err_vs_fp64_cg"] = max(
                 abs(a - b) / abs(b) for a, b in zip(summ, ref_sum) if b != 0.0)
-        log(f"[bench] {cells}^2 {name}: {rec}")
+        log(f"[bench] {cells}^2 {name}: {brief(rec)}")
         runs[name] = rec
     out = {"workload": f"{cells}x{cells}, seeded deck (3 rectangles + 2 circles, seed 2), "
                        f"tl_coefficient_inverse_density, true relative residual {target:g}, "
@@ -544,7 +614,7 @@ def precision_comparison(cells, inner_steps=10, target=1e-10, later_step=False):
             if extra:
                 rec["refinements"] = r["refinements"]
                 rec["sweeps"] = r["ppcg_inner"]
-            log(f"[bench] {cells}^2 {name} second step: {rec}")
+            log(f"[bench] {cells}^2 {name} second step: {brief(rec)}")
             out["second_step"][name] = rec
     t = {k: v["s_per_step"] for k, v in runs.items()}
     out["speedup_mixed_ppcg_vs_fp64_cg"] = t["fp64_cg"] / t["mixed_ppcg"]
@@ -669,7 +739,7 @@ def adjoint_bench(cells, steps, every, n_fd, h, precision, mixed_eps=1e-12, seed
                 np.linalg.norm(g[::8, ::8] - gs) / np.linalg.norm(gs))
             rec["vs_saved_gradient_norm_rel"] = float(
                 abs(np.linalg.norm(g) - saved["g_norm"]) / saved["g_norm"])
-        log(f"[bench] adjoint {cells}^2 {prec}: {rec}")
+        log(f"[bench] adjoint {cells}^2 {prec}: {brief(rec)}")
         out[prec] = rec
         grads[prec] = g
         p.close()
@@ -693,14 +763,16 @@ def adjoint_bench(cells, steps, every, n_fd, h, precision, mixed_eps=1e-12, seed
                   - float(((um[win] - target[win]) ** 2).sum())) / (2 * h)
             cells_fd.append(c)
             fds.append(fd)
-            log(f"[bench] adjoint FD cell {c}: fd {fd:.10e} " + " ".join(
-                f"{k} {grads[k][c]:.10e}" for k in grads))
+            if len(fds) % 8 == 0 or len(fds) == n_fd:
+                log(f"[bench] adjoint FD: {len(fds)} of {n_fd} cells")
         fd_s = time.perf_counter() - t0
         p.close()
         out["finite_differences"] = {
             "cells": n_fd, "h": h, "forward_solver": f"mixed precision CG, true relative "
                                                     f"residual {fd_eps:g}",
-            "seconds": fd_s}
+            "seconds": fd_s,
+            "quotients": [{"cell": c, "fd": fd, **{k: float(grads[k][c]) for k in grads}}
+                          for c, fd in zip(cells_fd, fds)]}
         for k, g in grads.items():
             errs = [abs(fd - g[c]) / abs(g[c]) for c, fd in zip(cells_fd, fds)]
             out[k].update({"fd_cells": n_fd, "fd_h": h, "fd_max_rel_err": max(errs),
@@ -834,59 +906,8 @@ def profile_run(cells, iters, solver="cg", copies=4):
                       "copy_bytes_each": 16 * cells * cells}))
 
 
-def main():
-    ap = argparse.ArgumentParser(description=__doc__)
-    ap.add_argument("--gpus", type=int, default=1)
-    ap.add_argument("--steps", type=int, default=5)
-    ap.add_argument("--warmup", type=int, default=1)
-    ap.add_argument("--cells", type=int, default=4096)
-    ap.add_argument("--solver", default="cg", choices=["cg"])
-    ap.add_argument("--cpu-cap", type=int, default=1500, help="iterations of the CPU sample")
-    ap.add_argument("--cpu-cap-one-thread", type=int, default=100,
-                    help="iterations of the one-thread CPU sample")
-    ap.add_argument("--no-cpu-baseline", action="store_true")
-    ap.add_argument("--mixed-sizes", default="4096,8192",
-                    help="comma-separated mesh sizes of the FP64 vs FP32-refined comparison "
-                         "('' to skip)")
-    ap.add_argument("--profile-solver", default="cg", choices=["cg", "chebyshev", "ppcg", "mixed_ppcg"],
-                    help="solver of the counter-profiling mode")
-    ap.add_argument("--profile-iters", type=int, default=0,
-                    help="counter-profiling mode: one CG step capped at this many iterations "
-                         "plus copy-kernel calibration launches; prints a short JSON line")
-    ap.add_argument("--adjoint-cells", type=int, default=2048,
-                    help="mesh of the adjoint case (0 to skip)")
-    ap.add_argument("--adjoint-steps", type=int, default=20)
-    ap.add_argument("--adjoint-every", type=int, default=5, help="checkpoint interval")
-    ap.add_argument("--adjoint-fd", type=int, default=32, help="finite-difference cells")
-    ap.add_argument("--adjoint-h", type=float, default=1e-6)
-    ap.add_argument("--adjoint-precision", default="both", choices=["fp64", "mixed", "both"])
-    ap.add_argument("--adjoint-solver", default="cg", choices=["cg", "ppcg"])
-    ap.add_argument("--adjoint-save", default=None,
-                    help="write target, gradient window/subsample and norm to this .npz")
-    ap.add_argument("--adjoint-compare", default=None,
-                    help="take the target from this .npz (--adjoint-save of an earlier run) "
-                         "and compare the gradient with the one saved there")
-    ap.add_argument("--adjoint-mixed-eps", type=float, default=1e-12,
-                    help="true relative residual of the mixed-precision solves")
-    ap.add_argument("--adjoint-large-cells", type=int, default=8192,
-                    help="mesh of the bounded mixed + adjoint ride-along (0 to skip)")
-    ap.add_argument("--adjoint-large-steps", type=int, default=2,
-                    help="timesteps of the bounded mixed + adjoint ride-along")
-    ap.add_argument("--no-small", action="store_true", help="skip the 512^2 CG case")
-    ap.add_argument("--no-stream", action="store_true",
-                    help="skip the STREAM-style copy/triad bandwidth measurement")
-    ap.add_argument("--solver-steps", type=int, default=1,
-                    help="timed steps of the Chebyshev and PPCG runs (0 to skip)")
-    args = ap.parse_args()
-    if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
-        print("bench.py runs on one GPU only: the solver keeps the whole mesh as one chunk "
-              "on a single MI355X (multi-GPU decomposition is not built).", file=sys.stderr)
-        sys.exit(2)
-
-    if args.profile_iters:
-        profile_run(args.cells, args.profile_iters, args.profile_solver)
-        return
-
+def measure(args):
+    """The whole record of a run."""
     with tempfile.TemporaryDirectory() as wd:
         elapsed, iters, prof = gpu_run(args.cells, args.solver, args.steps, args.warmup, wd)
     cells = args.cells * args.cells
@@ -967,7 +988,71 @@ def main():
                                                args.cpu_cap_one_thread)
         except Exception as e:  # report, do not fail the GPU measurement
             out["cpu_baseline"] = {"value": None, "error": str(e)}
-    print(json.dumps(out))
+    return out
+
+
+def main():
+    ap = argparse.ArgumentParser(description=__doc__)
+    ap.add_argument("--gpus", type=int, default=1)
+    ap.add_argument("--steps", type=int, default=5)
+    ap.add_argument("--warmup", type=int, default=1)
+    ap.add_argument("--cells", type=int, default=4096)
+    ap.add_argument("--solver", default="cg", choices=["cg"])
+    ap.add_argument("--cpu-cap", type=int, default=1500, help="iterations of the CPU sample")
+    ap.add_argument("--cpu-cap-one-thread", type=int, default=100,
+                    help="iterations of the one-thread CPU sample")
+    ap.add_argument("--no-cpu-baseline", action="store_true")
+    ap.add_argument("--mixed-sizes", default="4096,8192",
+                    help="comma-separated mesh sizes of the FP64 vs FP32-refined comparison "
+                         "('' to skip)")
+    ap.add_argument("--profile-solver", default="cg", choices=["cg", "chebyshev", "ppcg", "mixed_ppcg"],
+                    help="solver of the counter-profiling mode")
+    ap.add_argument("--profile-iters", type=int, default=0,
+                    help="counter-profiling mode: one CG step capped at this many iterations "
+                         "plus copy-kernel calibration launches; prints a short JSON line")
+    ap.add_argument("--adjoint-cells", type=int, default=2048,
+                    help="mesh of the adjoint case (0 to skip)")
+    ap.add_argument("--adjoint-steps", type=int, default=20)
+    ap.add_argument("--adjoint-every", type=int, default=5, help="checkpoint interval")
+    ap.add_argument("--adjoint-fd", type=int, default=32, help="finite-difference cells")
+    ap.add_argument("--adjoint-h", type=float, default=1e-6)
+    ap.add_argument("--adjoint-precision", default="both", choices=["fp64", "mixed", "both"])
+    ap.add_argument("--adjoint-solver", default="cg", choices=["cg", "ppcg"])
+    ap.add_argument("--adjoint-save", default=None,
+                    help="write target, gradient window/subsample and norm to this .npz")
+    ap.add_argument("--adjoint-compare", default=None,
+                    help="take the target from this .npz (--adjoint-save of an earlier run) "
+                         "and compare the gradient with the one saved there")
+    ap.add_argument("--adjoint-mixed-eps", type=float, default=1e-12,
+                    help="true relative residual of the mixed-precision solves")
+    ap.add_argument("--adjoint-large-cells", type=int, default=8192,
+                    help="mesh of the bounded mixed + adjoint ride-along (0 to skip)")
+    ap.add_argument("--adjoint-large-steps", type=int, default=2,
+                    help="timesteps of the bounded mixed + adjoint ride-along")
+    ap.add_argument("--record", default=None,
+                    help="write the whole record (per-kernel rates, finite differences, hosts) "
+                         "to this file")
+    ap.add_argument("--no-small", action="store_true", help="skip the 512^2 CG case")
+    ap.add_argument("--no-stream", action="store_true",
+                    help="skip the STREAM-style copy/triad bandwidth measurement")
+    ap.add_argument("--solver-steps", type=int, default=1,
+                    help="timed steps of the Chebyshev and PPCG runs (0 to skip)")
+    args = ap.parse_args()
+    if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
+        print("bench.py runs on one GPU only: the solver keeps the whole mesh as one chunk "
+              "on a single MI355X (multi-GPU decomposition is not built).", file=sys.stderr)
+        sys.exit(2)
+
+    if args.profile_iters:
+        profile_run(args.cells, args.profile_iters, args.profile_solver)
+        return
+
+    with host_lines_aside():
+        out = measure(args)
+    if args.record:
+        with open(args.record, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(headline(out)), flush=True)
 
 
 if __name__ == "__main__":
