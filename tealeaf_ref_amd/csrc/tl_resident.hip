@@ -58,11 +58,13 @@ __device__ inline ResGhost<T> load_ghosts(const ResTile<T, R> &t, const ResGeo &
 // region that only some lanes run, where it misses the others.  The build
 // fails where one does (spills.awk).
 //
-// What bounds it: the two exchanges of an iteration, about 1.4 us each of 4.6
-// (512^2), and with 16 cells per lane the arithmetic (3 of 6 us).  Against
-// the pass kernels: 512^2 step 5.7 -> 2.5 ms, 777x1031 with jac_diag 23.0 ->
-// 4.8 ms, 1500x997 with jac_block (eight rows) 87.5 -> 19 ms, the 1024^2 adjoint's
-// CG solves 155 -> 41 ms.
+// What bounds it: the two exchanges of an iteration.  Of a wave's time they take
+// 0.81 at 512^2 (64 blocks of four rows, 5.0 us an iteration), 0.86 at 777x1031
+// with jac_diag (231 blocks of four rows, 6.8 us), and with eight rows a lane,
+// where the arithmetic counts, 0.71 at 1024^2 (7.0 us) and 0.68 at 1500x997 with
+// jac_block (8.9 us).  Against the pass kernels: 512^2 step 5.7 -> 2.4 ms, 777x1031
+// with jac_diag 23.0 -> 4.8 ms, 1500x997 with jac_block 87.5 -> 20.3 ms, the 1024^2
+// adjoint's CG solves 155 -> 41 ms.
 enum Where { REGS, MEMORY };
 template <typename T, int R, int PREC>
 struct CgPlan {
@@ -293,9 +295,10 @@ __global__ __launch_bounds__(RES_THREADS) void k_res_cg(ResGeo g, ResCg<T> a) {
 // by Di is the product with the rounded 1 / Di, corrected by its remainder
 // (Markstein 1990), the division's own result in three operations for about ten.
 //
-// What bounds it: the exchange, 2.1 us of 3.7 with 225 blocks of five rows
-// (1100x1000: a step of 1000 iterations 14.6 -> 3.9 ms against the pass kernels;
-// 1400^2 18.3 -> 4.8, 512^2 5.6 -> 2.9, 100^2 3.0 -> 1.2).
+// What bounds it: the exchange, 0.81 of a wave's time with 225 blocks of five rows
+// (1100x1000: 3.9 us an iteration).  Steps of 1000 iterations by passes and on the
+// chip: 1100x1000 11.1 and 4.0 ms, 1400^2 14.2 and 5.0, 512^2 5.5 and 2.9, 100^2 4.4
+// and 2.3.
 // tea_leaf_jacobi_kernel.f90:60-66
 __device__ inline double jacobi_num(double s0, double l, double r, double d, double u, double kxl,
                                     double kxr, double kyd, double kyu, double rx, double ry) {
@@ -863,14 +866,15 @@ ResHost res_host() {
 // others wait for, `row` for every row a lane holds, `memory` more where
 // preconditioner fields are read again (from `from` rows on).  Fitted to steps
 // of 400 CG iterations: 512^2 with 128, 88, 64, 44 and 32 blocks of 2, 3, 4, 6
-// and 8 rows 2.24, 2.15, 2.12, 2.39 and 2.61 ms; 640^2 with 200, 100 and 50
-// blocks of 2, 4 and 8 rows 2.66, 2.25 and 2.66; 777^2 with jac_diag and 231,
-// 154 and 119 blocks of 4, 6 and 8 rows 2.68, 2.86 and 2.92; and of 1000 Jacobi
-// iterations: 512^2 with 256, 128, 64 and 44 blocks of 1, 2, 4 and 6 rows 3.23,
-// 2.88, 2.94 and 3.43 ms, 1100^2 with 252 and 207 blocks of 5 and 6 rows 3.96 and
-// 4.18.  Chebyshev's blocks wait for their neighbours only: 256^2 with 1, 2, 4 and
-// 8 rows 2.03, 2.20, 2.47 and 3.65 ms.  A single block waits for none, and up to 8,
-// one on each XCD, wait 0.2 us less in an exchange (1.2 for 1.4 us).
+// and 8 rows 2.16, 2.05, 2.04, 2.29 and 2.54 ms; 640^2 with 200, 100 and 50
+// blocks of 2, 4 and 8 rows 2.62, 2.12 and 2.59; 777^2 with jac_diag and 175,
+// 119 and 91 blocks of 4, 6 and 8 rows 2.61, 2.86 and 3.00; and of 1000 Jacobi
+// iterations: 512^2 with 256, 128, 64 and 44 blocks of 1, 2, 4 and 6 rows 3.21,
+// 2.92, 3.11 and 3.63 ms, 1100^2 with 252 and 207 blocks of 5 and 6 rows 4.02 and
+// 4.30.  Chebyshev's blocks wait for their neighbours only: 1000 iterations at
+// 256^2 with 1, 2, 4 and 8 rows 1.54, 1.70, 1.96 and 3.12.  A single block waits
+// for none, and up to 8, one on each XCD, wait 0.2 us less in an exchange (1.2 for
+// 1.4 us).
 struct ResCost {
   double block, row, memory;
   int from;

@@ -1,8 +1,9 @@
 """Loops of a few iterations: they take the kernels that are the faster there, not
 those that pay off over many.  Both routes are timed in turn on the same chunk;
 where the rule picks the older one the two are the same launches, so that their
-medians differ by noise only (a few per cent at 20 us and more), against 1.19
-to 1.45 where the rule is missing."""
+times differ by noise only (a few per cent at 20 us and more), against 1.19
+to 1.45 where the rule is missing; lower quartiles are compared, which a busy host
+moves least."""
 import ctypes as C
 import time
 
@@ -16,11 +17,11 @@ from test_gpu_deep import SIZES, _cheby
 from test_gpu_resident import _chunk, _norm_a, _start, env
 
 pytestmark = pytest.mark.gpu
-MARGIN = 1.12
+MARGIN = 1.15
 
 
-def _medians(call, routes, repeats=31):
-    """Median seconds of `call` under each environment, in turn."""
+def _times(call, routes, repeats=41):
+    """Lower quartile of the seconds of `call` under each environment, in turn."""
     times = [[] for _ in routes]
     for k in range(repeats + 3):
         for t, kw in zip(times, routes):
@@ -31,7 +32,7 @@ def _medians(call, routes, repeats=31):
                 L.call("tl_synchronize")
                 if k >= 3:
                     t.append(time.perf_counter() - a)
-    return [float(np.median(t)) for t in times]
+    return [float(np.percentile(t, 25)) for t in times]
 
 
 def test_one_cg_iteration():
@@ -46,7 +47,7 @@ def test_one_cg_iteration():
             st.n_first = st.n_last = 1
             assert L.lib().tl_cg_loop(C.byref(st), None, None) == L.TL_OK
 
-        new, old = _medians(call, ({}, {"TL_CG_DEFER": 0}))
+        new, old = _times(call, ({}, {"TL_CG_DEFER": 0}))
         print(f"one cg iteration {new * 1e6:.1f} us, u in each update {old * 1e6:.1f}", flush=True)
         assert new <= MARGIN * old
     finally:
@@ -77,7 +78,7 @@ def test_few_chebyshev_iterations(n, count):
                 call()
             out.append([interior(d.download(f), 1) for f in ("u", "p", "r")])
         assert all(np.array_equal(a, b) for a, b in zip(*out))
-        new, old = _medians(call, ({}, {"TL_DEEP": 0}))
+        new, old = _times(call, ({}, {"TL_DEEP": 0}))
         print(f"chebyshev {n}^2 {count} its {new * 1e6:.1f} us, pairs {old * 1e6:.1f}", flush=True)
         assert new <= MARGIN * old
     finally:
